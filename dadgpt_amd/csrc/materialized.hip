@@ -3,10 +3,13 @@
 // between its batched GEMMs (src/model.cpp:395-420 forward, :575-616 backward, :765-790
 // decode).
 //
-// Every kernel walks rows with one wave per row (four rows per 256-lane workgroup); a lane
-// holds columns lane, lane + 64, ... (16-byte pieces 4 floats wide when the row allows), so
-// each load instruction of a wave covers 256 or 1024 contiguous bytes. Row maxima and sums
-// are wave reductions through lane shuffles. The matrices are fp32, as the reference's.
+// Every kernel works on whole rows, one wave per row at a time; a lane holds 4 consecutive
+// columns of every 256 (one 16-byte piece), so each load instruction of a wave covers 1024
+// contiguous bytes. Row maxima and sums are wave reductions on DPP. The matrices are fp32, as
+// the reference's. Bound: HBM. Rows of 4 to 1,024 columns are read once into registers
+// (kMaxPieces pieces a lane), several rows per wave so that enough bytes are in flight, and the
+// causal kernels never read what lies past the diagonal; other rows take the loop kernels,
+// which pass over the row again for each reduction.
 //
 // Arithmetic order per element follows the reference's operators: scores are multiplied by
 // the scale, then masked to -1e9 (src/model.cpp:407-408; cuda/gpu_ops.cu:476-525), the
@@ -28,94 +31,273 @@ namespace {
 constexpr int kRowsPerBlock = 4;
 constexpr float kMaskValue = -1e9f;  // cuda/gpu_ops.cu:482
 
+// The wave's first row (a scalar; the host keeps row counts below 2^26), RPW rows per wave.
+template <int RPW = 1>
+__device__ __forceinline__ unsigned wave_row0() {
+  return (blockIdx.x * kRowsPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * RPW;
+}
+
 __device__ __forceinline__ float wave_max(float x) { return lanes::group_max<64>(x); }
 __device__ __forceinline__ float wave_sum(float x) { return lanes::group_sum<64>(x); }
 
-template <int V, typename F>
-__device__ __forceinline__ void read_row(const float* row, int cols, int lane, F f) {
-  if constexpr (V == 4) {
-    for (int c = lane * 4; c < cols; c += 256) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(row + c);
-      f(c, v.x), f(c + 1, v.y), f(c + 2, v.z), f(c + 3, v.w);
+// Four floats at any 4-byte address: gfx950 loads and stores 16 bytes at dword alignment in one
+// instruction, so rows of any length and offset move in the same pieces as aligned ones.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Columns c .. c+3 of a row of `cols` >= 4 columns (0 past the end), in two steps so that a
+// kernel issues all its loads before it waits for one. load_raw never branches: the piece that
+// crosses the row's end loads its last four columns instead (whole_piece moves those into
+// place), and pieces past the one that holds column `last` load that one again.
+__device__ __forceinline__ f32x4 load_raw(const float* row, int c, int last, int cols) {
+  return *reinterpret_cast<const f32x4u*>(row + min(c, min(last & ~3, cols - 4)));
+}
+__device__ __forceinline__ f32x4 whole_piece(f32x4 v, int c, int cols) {
+  if (cols % 4 != 0) {  // wave-uniform
+    const int shift = c + 4 - cols;  // 1 to 3 for the piece that crosses the end
+    if (shift > 0) {
+      if (shift & 2) v = f32x4{v[2], v[3], 0.f, 0.f};
+      if (shift & 1) v = f32x4{v[1], v[2], v[3], 0.f};
     }
-  } else {
-    for (int c = lane; c < cols; c += 64) f(c, row[c]);
   }
+  return c < cols ? v : f32x4{0.f, 0.f, 0.f, 0.f};
+}
+// The same in one step, for any number of columns.
+__device__ __forceinline__ f32x4 load_piece(const float* row, int c, int cols) {
+  if (cols >= 4) return whole_piece(load_raw(row, c, cols - 1, cols), c, cols);
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  for (int e = 0; e < 3; ++e)
+    if (c + e < cols) v[e] = row[c + e];
+  return v;
+}
+__device__ __forceinline__ void store_piece(float* row, int c, int cols, const f32x4& v) {
+  if (c + 4 <= cols) {
+    *reinterpret_cast<f32x4u*>(row + c) = v;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+    if (c + e < cols) row[c + e] = v[e];
 }
 
 // What a softmax row sees of its input: the raw value (kPlain), scale then causal mask
 // (kCausal: row r of a head is query r % S), or scale then a length mask (kLength: keys at or
-// past lens[r / H] are masked; an empty cache gives a zero row).
+// past lens[r / H] are masked; an empty cache gives a zero row). Columns at or past the row's
+// limit hold kMaskValue whatever the input holds there, so they are not read.
 enum RowMode { kPlain, kCausal, kLength };
 
-template <int MODE, int V>
-__global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_kernel(
-    float* out, const float* in, long long rows, int cols, int S,
-    float scale, const int* __restrict__ lens, int H) {
-  const int lane = threadIdx.x & 63;
-  const long long r = (long long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-  if (r >= rows) return;
-  const float* src = in + r * cols;
-  float* dst = out + r * cols;
-  int limit = cols;  // columns at or past `limit` are masked
-  if constexpr (MODE == kCausal) limit = (int)(r % S) + 1;
+template <int MODE>
+__device__ __forceinline__ int row_limit(unsigned r, int cols, int S, const int* lens, int H) {
+  if constexpr (MODE == kCausal) return (int)(r % (unsigned)S) + 1;
   if constexpr (MODE == kLength) {
-    const int L = lens[r / H];
-    limit = L < 0 ? 0 : (L > cols ? cols : L);
-    if (limit == 0) {  // no keys: a zero row (o = 0, as the decode kernel returns)
-      for (int c = lane; c < cols; c += 64) dst[c] = 0.f;
-      return;
+    const int L = lens[r / (unsigned)H];
+    return L < 0 ? 0 : (L > cols ? cols : L);
+  }
+  return cols;
+}
+
+// The maximum a row starts from: the reference's initial one (cuda/gpu_ops.cu:156), and the
+// masked columns' value where there are any.
+__device__ __forceinline__ float initial_max(int limit, int cols) {
+  return limit < cols ? kMaskValue : -1e30f;
+}
+
+// The weight of a masked column: 0 unless every visible score lies at the mask value's level
+// (mx is the same in every lane).
+__device__ __forceinline__ float masked_weight(float mx) {
+  if (__builtin_amdgcn_readfirstlane(mx > 0.5f * kMaskValue)) return 0.f;
+  return expf(kMaskValue - mx);
+}
+
+// x / sum as q = x inv, corrected once by its exact remainder (inv = 1 / sum): the quotient
+// IEEE division gives, in three operations per element. sum >= 1 or the row is degenerate (0 or
+// NaN, which stays NaN).
+__device__ __forceinline__ float divide(float x, float sum, float inv) {
+  const float q = x * inv;
+  return fmaf(fmaf(-q, sum, x), inv, q);
+}
+
+constexpr int kMaxPieces = 4;  // 16-byte pieces a lane holds of a register row (1,024 columns)
+
+// Rows per wave of the register kernels: four pieces a lane in flight, fewer where that would
+// leave CUs idle (the grid then has fewer than four waves for each of the 1,024 SIMDs).
+int rows_per_wave(long long rows, int pieces) {
+  int n = 4 / pieces;
+  while (n > 1 && rows < 4096LL * n) n >>= 1;
+  return n;
+}
+
+// Softmax of rows of at most 256 NP columns, RPW rows per wave, each read once.
+// [BH 192, S 256] (50 MB) causal, in place: 27 us with the looping kernel below (three passes,
+// two exponentials per element), 19 us here (its 75 MB take 13-15; the exponentials' VALU work
+// does not hide completely under them).
+template <int MODE, int NP, int RPW>
+__global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_reg_kernel(
+    float* out, const float* in, unsigned rows, int cols, int S, float scale,
+    const int* __restrict__ lens, int H) {
+  const int c0 = 4 * (threadIdx.x & 63);
+  const unsigned r0 = wave_row0<RPW>();
+  if (r0 >= rows) return;
+  f32x4 x[RPW][NP];
+  int limit[RPW];
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) {
+    const unsigned r = min(r0 + i, rows - 1);
+    limit[i] = row_limit<MODE>(r, cols, S, lens, H);
+#pragma unroll
+    for (int n = 0; n < NP; ++n)
+      x[i][n] = load_raw(in + (size_t)r * cols, c0 + 256 * n, max(limit[i] - 1, 0), cols);
+  }
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) {
+    if (r0 + i >= rows) return;
+    float* dst = out + (size_t)(r0 + i) * cols;
+    float mx = initial_max(limit[i], cols);
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      x[i][n] = whole_piece(x[i][n], c0 + 256 * n, cols);
+      if constexpr (MODE != kPlain) x[i][n] *= scale;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c0 + 256 * n + e < limit[i]) mx = fmaxf(mx, x[i][n][e]);
+    }
+    mx = wave_max(mx);
+    float sum = 0.f;
+#pragma unroll
+    for (int n = 0; n < NP; ++n)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c0 + 256 * n + e < limit[i]) sum += x[i][n][e] = expf(x[i][n][e] - mx);
+    const float masked = masked_weight(mx);
+    sum = wave_sum(sum) + (limit[i] < cols ? (float)(cols - limit[i]) * masked : 0.f);
+    const float inv = 1.0f / sum;
+    const bool empty = MODE == kLength && limit[i] == 0;  // no keys: a zero row
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      const int c = c0 + 256 * n;
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] = empty ? 0.f : divide(c + e < limit[i] ? x[i][n][e] : masked, sum, inv);
+      if (c < cols) store_piece(dst, c, cols, v);
     }
   }
-  auto value = [&](int c, float x) {
-    if constexpr (MODE == kPlain) return x;
-    const float s = x * scale;
-    return c < limit ? s : kMaskValue;
+}
+
+// Softmax of rows of any length: one row per wave, read again for each reduction.
+template <int MODE>
+__global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_kernel(
+    float* out, const float* in, unsigned rows, int cols, int S,
+    float scale, const int* __restrict__ lens, int H) {
+  const int c0 = 4 * (threadIdx.x & 63);
+  const unsigned r = wave_row0();
+  if (r >= rows) return;
+  const float* src = in + (size_t)r * cols;
+  float* dst = out + (size_t)r * cols;
+  const int limit = row_limit<MODE>(r, cols, S, lens, H);
+  auto visible = [&](auto f) {  // f(piece of scaled values, its first column)
+    for (int c = c0; c < limit; c += 256) {
+      f32x4 v = load_piece(src, c, cols);
+      if constexpr (MODE != kPlain) v *= scale;
+      f(v, c);
+    }
   };
-  float mx = -1e30f;  // the reference's initial max (cuda/gpu_ops.cu:156)
-  read_row<V>(src, cols, lane, [&](int c, float x) { mx = fmaxf(mx, value(c, x)); });
+  float mx = initial_max(limit, cols);
+  visible([&](const f32x4& v, int c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e < limit) mx = fmaxf(mx, v[e]);
+  });
   mx = wave_max(mx);
   float sum = 0.f;
-  read_row<V>(src, cols, lane, [&](int c, float x) { sum += expf(value(c, x) - mx); });
-  sum = wave_sum(sum);
+  visible([&](const f32x4& v, int c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (c + e < limit) sum += expf(v[e] - mx);
+  });
+  const float masked = masked_weight(mx);
+  sum = wave_sum(sum) + (limit < cols ? (float)(cols - limit) * masked : 0.f);
+  const float inv = 1.0f / sum;
+  const bool empty = MODE == kLength && limit == 0;
   // in == out is allowed: each lane writes exactly the columns it reads, after reading them
-  if constexpr (V == 4) {
-    for (int c = lane * 4; c < cols; c += 256) {
-      f32x4 v = *reinterpret_cast<const f32x4*>(src + c);
-      v.x = expf(value(c, v.x) - mx) / sum;
-      v.y = expf(value(c + 1, v.y) - mx) / sum;
-      v.z = expf(value(c + 2, v.z) - mx) / sum;
-      v.w = expf(value(c + 3, v.w) - mx) / sum;
-      *reinterpret_cast<f32x4*>(dst + c) = v;
-    }
-  } else {
-    for (int c = lane; c < cols; c += 64) dst[c] = expf(value(c, src[c]) - mx) / sum;
+  for (int c = c0; c < cols; c += 256) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (c < limit) v = load_piece(src, c, cols);
+    if constexpr (MODE != kPlain) v *= scale;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[e] = empty ? 0.f : divide(c + e < limit ? expf(v[e] - mx) : masked, sum, inv);
+    store_piece(dst, c, cols, v);
   }
 }
 
 // Softmax backward per row: g = p * (dp - sum_j dp_j p_j). ACCUMULATE: din += g (the
 // reference's operator). Otherwise the attention form: din = g, zero past the causal
-// diagonal, times scale (din may be dout).
-template <bool ACCUMULATE>
+// diagonal, times scale (din may be dout). The sum runs over whole rows, whatever p holds past
+// the diagonal. REG: rows of at most 256 NP columns, RPW rows per wave, each read once;
+// otherwise (NP = RPW = 1) any length, the row read twice.
+// [BH 192, S 256], 3 x 50 MB: 36 us with 4-byte loads in two passes, 24.5 us here
+// (6.1 TB/s).
+template <bool ACCUMULATE, bool REG, int NP, int RPW>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_backward_rows_kernel(
-    float* din, const float* dout, const float* __restrict__ p, long long rows, int cols, int S,
+    float* din, const float* dout, const float* __restrict__ p, unsigned rows, int cols, int S,
     float scale) {
-  const int lane = threadIdx.x & 63;
-  const long long r = (long long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
-  if (r >= rows) return;
-  const float* g = dout + r * cols;
-  const float* pr = p + r * cols;
-  float* d = din + r * cols;
-  float dot = 0.f;
-  for (int c = lane; c < cols; c += 64) dot += g[c] * pr[c];
-  dot = wave_sum(dot);
-  const int limit = ACCUMULATE ? cols : (int)(r % S) + 1;
-  for (int c = lane; c < cols; c += 64) {
-    const float v = pr[c] * (g[c] - dot);
-    if constexpr (ACCUMULATE)
-      d[c] += v;
-    else
-      d[c] = c < limit ? v * scale : 0.0f;
+  const int c0 = 4 * (threadIdx.x & 63);
+  const unsigned r0 = wave_row0<RPW>();
+  if (r0 >= rows) return;
+  auto row_dot = [](const f32x4& g, const f32x4& pr, float dot) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dot += g[e] * pr[e];
+    return dot;
+  };
+  auto finish = [&](unsigned r, int c, const f32x4& g, const f32x4& pr, float dot) {
+    const int limit = ACCUMULATE ? cols : (int)(r % (unsigned)S) + 1;
+    float* d = din + (size_t)r * cols;
+    f32x4 v;
+    if constexpr (ACCUMULATE) v = load_piece(d, c, cols);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float t = pr[e] * (g[e] - dot);
+      if constexpr (ACCUMULATE)
+        v[e] += t;
+      else
+        v[e] = c + e < limit ? t * scale : 0.0f;
+    }
+    store_piece(d, c, cols, v);
+  };
+  if constexpr (REG) {
+    f32x4 g[RPW][NP], pr[RPW][NP];
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const unsigned r = min(r0 + i, rows - 1);
+#pragma unroll
+      for (int n = 0; n < NP; ++n) {
+        g[i][n] = load_raw(dout + (size_t)r * cols, c0 + 256 * n, cols - 1, cols);
+        pr[i][n] = load_raw(p + (size_t)r * cols, c0 + 256 * n, cols - 1, cols);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      if (r0 + i >= rows) return;
+      float dot = 0.f;
+#pragma unroll
+      for (int n = 0; n < NP; ++n) {
+        g[i][n] = whole_piece(g[i][n], c0 + 256 * n, cols);
+        pr[i][n] = whole_piece(pr[i][n], c0 + 256 * n, cols);
+        dot = row_dot(g[i][n], pr[i][n], dot);
+      }
+      dot = wave_sum(dot);
+#pragma unroll
+      for (int n = 0; n < NP; ++n)
+        if (c0 + 256 * n < cols) finish(r0 + i, c0 + 256 * n, g[i][n], pr[i][n], dot);
+    }
+  } else {
+    const float *gr = dout + (size_t)r0 * cols, *prow = p + (size_t)r0 * cols;
+    float dot = 0.f;
+    for (int c = c0; c < cols; c += 256)
+      dot = row_dot(load_piece(gr, c, cols), load_piece(prow, c, cols), dot);
+    dot = wave_sum(dot);
+    for (int c = c0; c < cols; c += 256)
+      finish(r0, c, load_piece(gr, c, cols), load_piece(prow, c, cols), dot);
   }
 }
 
@@ -135,96 +317,91 @@ __global__ void scale_kernel(float* __restrict__ x, long long n, float scale) {
 
 // Attention-probability dropout on the materialized path, with the flash kernels' mask
 // (dropout.hpp): element (r, c) of the [BH*S, S] probabilities is row r = bh*S + query and key
-// c. Each lane owns 8 consecutive columns per step, whose keep bits are one Philox block;
-// rows whose columns are not 16-byte pieces take the per-element path (V = 1).
-template <int V, typename F>
-__device__ __forceinline__ void row_groups(const float* row, int cols, int lane,
-                                           const DropParams& dr, long long r, F f) {
-  for (int c0 = 8 * lane; c0 < cols; c0 += 512) {
-    const uint32_t bits = keep8(dr, (uint64_t)r, (uint32_t)c0 >> 3);
-    if constexpr (V == 4) {  // cols % 8 == 0: the group is whole
-      const f32x4 a = *reinterpret_cast<const f32x4*>(row + c0);
-      const f32x4 b = *reinterpret_cast<const f32x4*>(row + c0 + 4);
-      f(c0, a, b, bits);
-    } else {
-      f32x4 a, b;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        a[e] = c0 + e < cols ? row[c0 + e] : 0.f;
-        b[e] = c0 + 4 + e < cols ? row[c0 + 4 + e] : 0.f;
-      }
-      f(c0, a, b, bits);
-    }
-  }
+// c. Each lane owns 8 consecutive columns per step, whose keep bits are one Philox block.
+struct Group8 {
+  float v[8];
+  __device__ __forceinline__ float& operator[](int e) { return v[e]; }
+};
+__device__ __forceinline__ Group8 load_group(const float* row, int c, int cols) {
+  const f32x4 a = load_piece(row, c, cols), b = load_piece(row, c + 4, cols);
+  return Group8{{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}};
 }
-
-template <int V>
-__device__ __forceinline__ void store_group(float* row, int cols, int c0, const f32x4& a,
-                                            const f32x4& b) {
-  if constexpr (V == 4) {
-    *reinterpret_cast<f32x4*>(row + c0) = a;
-    *reinterpret_cast<f32x4*>(row + c0 + 4) = b;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (c0 + e < cols) row[c0 + e] = a[e];
-      if (c0 + 4 + e < cols) row[c0 + 4 + e] = b[e];
-    }
-  }
+__device__ __forceinline__ void store_group(float* row, int c, int cols, Group8& g) {
+  store_piece(row, c, cols, f32x4{g[0], g[1], g[2], g[3]});
+  if (c + 4 < cols) store_piece(row, c + 4, cols, f32x4{g[4], g[5], g[6], g[7]});
 }
 
 // out = p * keep / (1 - p_drop) (the reference's gpu_dropout_forward, cuda/gpu_ops.cu:712-733,
 // with this mask). out may be p.
-template <int V>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void dropout_rows_kernel(
-    float* out, const float* p, long long rows, int cols, DropParams dr) {
-  const int lane = threadIdx.x & 63;
-  const long long r = (long long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
+    float* out, const float* p, unsigned rows, int cols, DropParams dr) {
+  const unsigned r = wave_row0();
   if (r >= rows) return;
-  float* dst = out + r * cols;
-  row_groups<V>(p + r * cols, cols, lane, dr, r, [&](int c0, f32x4 a, f32x4 b, uint32_t bits) {
+  for (int c = 8 * (threadIdx.x & 63); c < cols; c += 512) {
+    Group8 g = load_group(p + (size_t)r * cols, c, cols);
+    const uint32_t bits = keep8(dr, (uint64_t)r, (uint32_t)c >> 3);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      a[e] *= keep_factor(bits, e, dr.scale);
-      b[e] *= keep_factor(bits, 4 + e, dr.scale);
-    }
-    store_group<V>(dst, cols, c0, a, b);
-  });
+    for (int e = 0; e < 8; ++e) g[e] *= keep_factor(bits, e, dr.scale);
+    store_group(out + (size_t)r * cols, c, cols, g);
+  }
 }
 
 // The attention backward's row pass with dropout (src/model.cpp:594-607): dP = dPd * keep /
 // (1 - p_drop) (gpu_dropout_backward, cuda/gpu_ops.cu:736-749), then the softmax backward
-// against the undropped P, zero past the causal diagonal, times scale. ds may be dpd.
-template <int V>
+// against the undropped P, zero past the causal diagonal, times scale. ds may be dpd. NG > 0:
+// rows of at most 512 NG columns, read and their keep bits generated once; NG = 0: any length,
+// both done again for the second pass.
+template <int NG>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void attn_probs_backward_dropout_kernel(
-    float* ds, const float* dpd, const float* __restrict__ p, long long rows, int S,
+    float* ds, const float* dpd, const float* __restrict__ p, unsigned rows, int S,
     float scale, DropParams dr) {
-  const int lane = threadIdx.x & 63;
-  const long long r = (long long)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
+  const int c0 = 8 * (threadIdx.x & 63);
+  const unsigned r = wave_row0();
   if (r >= rows) return;
-  const float* g = dpd + r * S;
-  const float* pr = p + r * S;
-  float* d = ds + r * S;
+  const float *gr = dpd + (size_t)r * S, *pr = p + (size_t)r * S;
+  const int limit = (int)(r % (unsigned)S) + 1;
+  auto undrop = [&](int c) {  // dP of the undropped probabilities
+    Group8 g = load_group(gr, c, S);
+    const uint32_t bits = keep8(dr, (uint64_t)r, (uint32_t)c >> 3);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] *= keep_factor(bits, e, dr.scale);
+    return g;
+  };
+  auto row_dot = [](Group8& g, Group8& q, float dot) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dot += g[e] * q[e];
+    return dot;
+  };
+  auto finish = [&](int c, Group8& g, Group8& q, float dot) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] = c + e < limit ? q[e] * (g[e] - dot) * scale : 0.f;
+    store_group(ds + (size_t)r * S, c, S, g);
+  };
   float dot = 0.f;
-  row_groups<V>(g, S, lane, dr, r, [&](int c0, f32x4 a, f32x4 b, uint32_t bits) {
+  if constexpr (NG > 0) {
+    Group8 g[NG], q[NG];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (c0 + e < S) dot += a[e] * keep_factor(bits, e, dr.scale) * pr[c0 + e];
-      if (c0 + 4 + e < S) dot += b[e] * keep_factor(bits, 4 + e, dr.scale) * pr[c0 + 4 + e];
-    }
-  });
-  dot = wave_sum(dot);
-  const int limit = (int)(r % S) + 1;
-  row_groups<V>(g, S, lane, dr, r, [&](int c0, f32x4 a, f32x4 b, uint32_t bits) {
+    for (int n = 0; n < NG; ++n)
+      if (c0 + 512 * n < S) {
+        q[n] = load_group(pr, c0 + 512 * n, S);
+        g[n] = undrop(c0 + 512 * n);
+        dot = row_dot(g[n], q[n], dot);
+      }
+    dot = wave_sum(dot);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int ca = c0 + e, cb = c0 + 4 + e;
-      a[e] = ca < limit ? pr[ca] * (a[e] * keep_factor(bits, e, dr.scale) - dot) * scale : 0.f;
-      b[e] = cb < limit ? pr[cb] * (b[e] * keep_factor(bits, 4 + e, dr.scale) - dot) * scale
-                        : 0.f;
+    for (int n = 0; n < NG; ++n)
+      if (c0 + 512 * n < S) finish(c0 + 512 * n, g[n], q[n], dot);
+  } else {
+    for (int c = c0; c < S; c += 512) {
+      Group8 g = undrop(c), q = load_group(pr, c, S);
+      dot = row_dot(g, q, dot);
     }
-    store_group<V>(d, S, c0, a, b);
-  });
+    dot = wave_sum(dot);
+    for (int c = c0; c < S; c += 512) {
+      Group8 g = undrop(c), q = load_group(pr, c, S);
+      finish(c, g, q, dot);
+    }
+  }
 }
 
 // The head split and merge (cuda/gpu_ops.cu:426-474), a pure permutation between the
@@ -268,20 +445,52 @@ unsigned row_blocks(long long rows) {
   return (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
 }
 
-bool vec4(const void* a, const void* b, int cols) {
-  return cols % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(b) % 16 == 0;
+// f(pieces, rows per wave) as compile-time constants for rows of 4 to 1,024 columns.
+template <typename F>
+void with_row_shape(long long rows, int cols, F f) {
+  using std::integral_constant;
+  if (cols <= 256) {
+    switch (rows_per_wave(rows, 1)) {
+      case 4: return f(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+      case 2: return f(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+      default: return f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    }
+  }
+  if (cols <= 512) {
+    if (rows_per_wave(rows, 2) == 2)
+      return f(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+    return f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+  }
+  return f(integral_constant<int, 4>{}, integral_constant<int, 1>{});
 }
 
 template <int MODE>
 hipError_t launch_softmax(float* out, const float* in, long long rows, int cols, int S,
                           float scale, const int* lens, int H, hipStream_t stream) {
-  if (vec4(out, in, cols))
-    softmax_rows_kernel<MODE, 4><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-        out, in, rows, cols, S, scale, lens, H);
+  if (cols < 4 || cols > 256 * kMaxPieces)
+    softmax_rows_kernel<MODE><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
+        out, in, (unsigned)rows, cols, S, scale, lens, H);
   else
-    softmax_rows_kernel<MODE, 1><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-        out, in, rows, cols, S, scale, lens, H);
+    with_row_shape(rows, cols, [&](auto np, auto rpw) {
+      softmax_rows_reg_kernel<MODE, np(), rpw()>
+          <<<row_blocks((rows + rpw() - 1) / rpw()), 64 * kRowsPerBlock, 0, stream>>>(
+              out, in, (unsigned)rows, cols, S, scale, lens, H);
+    });
+  return hipGetLastError();
+}
+
+template <bool ACCUMULATE>
+hipError_t launch_softmax_backward(float* din, const float* dout, const float* p, long long rows,
+                                   int cols, int S, float scale, hipStream_t stream) {
+  if (cols < 4 || cols > 256 * kMaxPieces)
+    softmax_backward_rows_kernel<ACCUMULATE, false, 1, 1>
+        <<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(din, dout, p, (unsigned)rows, cols, S, scale);
+  else
+    with_row_shape(rows, cols, [&](auto np, auto rpw) {
+      softmax_backward_rows_kernel<ACCUMULATE, true, np(), rpw()>
+          <<<row_blocks((rows + rpw() - 1) / rpw()), 64 * kRowsPerBlock, 0, stream>>>(
+              din, dout, p, (unsigned)rows, cols, S, scale);
+    });
   return hipGetLastError();
 }
 
@@ -294,9 +503,7 @@ hipError_t launch_softmax_rows(float* out, const float* in, long long rows, int 
 
 hipError_t launch_softmax_backward_rows(float* din, const float* dout, const float* p,
                                         long long rows, int cols, hipStream_t stream) {
-  softmax_backward_rows_kernel<true><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-      din, dout, p, rows, cols, 1, 1.0f);
-  return hipGetLastError();
+  return launch_softmax_backward<true>(din, dout, p, rows, cols, 1, 1.0f, stream);
 }
 
 hipError_t launch_causal_fill(float* m, int n_blocks, int S, float value, hipStream_t stream) {
@@ -317,10 +524,7 @@ hipError_t launch_attention_probs(float* p, int BH, int S, float scale, hipStrea
 
 hipError_t launch_attention_probs_backward(float* ds, const float* dp, const float* p, int BH,
                                            int S, float scale, hipStream_t stream) {
-  const long long rows = (long long)BH * S;
-  softmax_backward_rows_kernel<false><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-      ds, dp, p, rows, S, S, scale);
-  return hipGetLastError();
+  return launch_softmax_backward<false>(ds, dp, p, (long long)BH * S, S, S, scale, stream);
 }
 
 hipError_t launch_decode_probs(float* p, const int* lens, int n_seq, int H, int max_len,
@@ -333,12 +537,7 @@ hipError_t launch_attention_dropout(float* out, const float* p, int BH, int S,
                                    const Dropout& drop, hipStream_t stream) {
   const long long rows = (long long)BH * S;
   const DropParams dr = drop_params(&drop);
-  if (S % 8 == 0 && vec4(out, p, S))
-    dropout_rows_kernel<4><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(out, p, rows, S,
-                                                                                dr);
-  else
-    dropout_rows_kernel<1><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(out, p, rows, S,
-                                                                                dr);
+  dropout_rows_kernel<<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(out, p, (unsigned)rows, S, dr);
   return hipGetLastError();
 }
 
@@ -347,12 +546,15 @@ hipError_t launch_attention_probs_backward_dropout(float* ds, const float* dpd, 
                                                    const Dropout& drop, hipStream_t stream) {
   const long long rows = (long long)BH * S;
   const DropParams dr = drop_params(&drop);
-  if (S % 8 == 0 && vec4(ds, dpd, S) && vec4(p, p, S))
-    attn_probs_backward_dropout_kernel<4><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-        ds, dpd, p, rows, S, scale, dr);
-  else
+  if (S <= 512)
     attn_probs_backward_dropout_kernel<1><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-        ds, dpd, p, rows, S, scale, dr);
+        ds, dpd, p, (unsigned)rows, S, scale, dr);
+  else if (S <= 1024)
+    attn_probs_backward_dropout_kernel<2><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
+        ds, dpd, p, (unsigned)rows, S, scale, dr);
+  else
+    attn_probs_backward_dropout_kernel<0><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
+        ds, dpd, p, (unsigned)rows, S, scale, dr);
   return hipGetLastError();
 }
 

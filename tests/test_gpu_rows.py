@@ -1,0 +1,111 @@
+"""The row kernels of the materialized path at the edges of their shapes: rows that end inside
+a 16-byte piece, one row and several per wave, register rows (4 to 1,024 columns) and looped ones,
+against float64."""
+import numpy as np
+import pytest
+import torch
+
+from dadgpt_amd import attention as A
+
+pytestmark = pytest.mark.gpu
+
+# (columns, rows): 16-byte remainders 0-3, both sides of 256, 512 and 1,024 columns, and row
+# counts that give one, two and four rows per wave with a last wave that is not full.
+SHAPES = [(1, 5), (3, 4099), (4, 9), (5, 16387), (66, 8193), (255, 16389), (256, 16384),
+          (257, 8195), (511, 8193), (512, 4097), (513, 33), (1021, 7), (1024, 5), (1025, 6),
+          (2047, 3)]
+
+
+def _normal(shape, seed, scale=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(shape, generator=g, device="cuda") * scale
+
+
+@pytest.mark.parametrize("cols,rows", SHAPES)
+def test_plain_rows(gpu, cols, rows):
+    """softmax and the accumulating softmax_backward. A probability p = e^(x - max) / sum is off
+    by at most p (|x - max| + 4) 2^-23 <= 6e-7, each product of the backward by 2^-23 of its
+    terms (|g| < 6, and a row sum below 6 in magnitude): 2e-6."""
+    print(f"[case] rows={rows} cols={cols}", flush=True)
+    x, g, d = (_normal((rows, cols), 10 + i, s) for i, s in enumerate((3.0, 1.0, 1.0)))
+    out = torch.full_like(x, float("nan"))
+    A.softmax(out, x, rows, cols)
+    same = x.clone()
+    A.softmax(same, same, rows, cols)
+    assert torch.equal(out, same)
+    p = torch.softmax(x.double(), -1)
+    assert (out.double() - p).abs().max().item() <= 1e-6
+    din = d.clone()
+    A.softmax_backward(din, g, out, rows, cols)
+    o, g6 = out.double(), g.double()
+    want = d.double() + o * (g6 - (g6 * o).sum(-1, keepdim=True))
+    assert (din.double() - want).abs().max().item() <= 2e-6
+
+
+@pytest.mark.parametrize("S,BH", [(1, 3), (3, 5), (4, 2), (63, 70), (64, 260), (130, 127),
+                                  (256, 65), (257, 32), (509, 17), (512, 9), (515, 2), (1023, 1),
+                                  (1030, 1)])
+def test_causal_rows(gpu, S, BH):
+    """attention_probs and attention_probs_backward, without and with dropout (p = 0, whose
+    factors are exactly 1, must give the plain result's values). What lies past the diagonal of
+    the scores does not matter; past that of the probabilities it counts in the row sum."""
+    print(f"[case] BH={BH} S={S}", flush=True)
+    scale = 0.25
+    s, g = _normal((BH, S, S), 20, 6.0), _normal((BH, S, S), 21)
+    upper = torch.ones((S, S), dtype=torch.bool, device="cuda").triu(1)
+    probs = s.masked_fill(upper, float("nan"))
+    A.attention_probs(probs, BH, S, scale)
+    p = torch.softmax((s.double() * scale).masked_fill(upper, float("-inf")), -1)
+    assert (probs.double() - p).abs().max().item() <= 1e-6
+    assert torch.count_nonzero(probs[:, upper]).item() == 0
+    full = probs + 0.01 * upper  # not a causal matrix
+    for pr in (probs, full):
+        ds = torch.full_like(g, float("nan"))
+        A.attention_probs_backward(ds, g, pr, BH, S, scale)
+        p6, g6 = pr.double(), g.double()
+        want = p6 * (g6 - (g6 * p6).sum(-1, keepdim=True)) * scale
+        want.masked_fill_(upper, 0.0)
+        # products and the sum of up to S terms of at most 0.06 past the diagonal
+        tol = 2e-6 * (1 if pr is probs else 1 + 0.06 * S ** 0.5)
+        assert (ds.double() - want).abs().max().item() <= tol
+        drop = torch.full_like(g, float("nan"))
+        A.attention_probs_backward_dropout(drop, g, pr, BH, S, scale, 0.0, 9)
+        assert (drop.double() - want).abs().max().item() <= tol
+        inplace = g.clone()
+        A.attention_probs_backward(inplace, inplace, pr, BH, S, scale)
+        assert torch.equal(inplace, ds)
+    dropped = torch.full_like(g, float("nan"))
+    A.attention_dropout(dropped, probs, BH, S, 0.0, 9)
+    assert torch.equal(dropped, probs)
+
+
+def test_rows_at_the_mask_value(gpu):
+    """Visible scores at and below the mask's -1e9: the masked columns then carry weight, as in
+    the reference's fill-then-softmax."""
+    S = 70
+    s = torch.full((1, S, S), -1e9, device="cuda")
+    s[0, 5] = -2e9
+    s[0, 6] = float("-inf")
+    A.attention_probs(s, 1, S, 1.0)
+    assert torch.equal(s[0, 0], torch.full((S,), np.float32(1.0) / np.float32(S), device="cuda"))
+    want = torch.zeros(S, device="cuda")
+    want[6:] = 1.0 / (S - 6)
+    assert torch.allclose(s[0, 5], want, rtol=1e-6, atol=0)
+    want = torch.zeros(S, device="cuda")
+    want[7:] = 1.0 / (S - 7)
+    assert torch.allclose(s[0, 6], want, rtol=1e-6, atol=0)
+
+
+def test_length_rows(gpu):
+    """decode_probs over rows of 1,022 columns: only the first lens keys, zero past them, a zero
+    row for an empty cache."""
+    n, H, L = 6, 700, 1022
+    s = _normal((n * H, L), 30, 4.0)
+    lens = torch.tensor([1, 0, 513, 1022, 4, 257], dtype=torch.int32, device="cuda")
+    keep = torch.arange(L, device="cuda") < lens.repeat_interleave(H).unsqueeze(1)
+    probs = s.masked_fill(~keep, float("nan"))
+    A.decode_probs(probs, lens, n, H, L, 0.5)
+    p = torch.softmax((s.double() * 0.5).masked_fill(~keep, float("-inf")), -1)
+    p[lens.repeat_interleave(H) == 0] = 0.0
+    assert (probs.double() - p).abs().max().item() <= 1e-6
+    assert torch.count_nonzero(probs[~keep]).item() == 0
