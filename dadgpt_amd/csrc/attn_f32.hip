@@ -17,20 +17,23 @@
 //           exchange). K and V tiles are split once per workgroup as they are staged, into
 //           three bf16 planes each in the bf16 kernels' swizzled layout, read with
 //           ds_read_b128 (K rows) and ds_read_b64_tr_b16 (V^T);
-//  dK/dV    a wave owns 32 keys (lane l holds key l % 32) and walks every later query chunk:
-//           S = Q K^T and dP = dO V^T with K and V in registers (floats, split at each use),
-//           Q and dO as bf16 planes, P and dS in registers, dV^T += dO^T P and
-//           dK^T += Q^T dS; nothing is shared between waves (no atomics);
+//  dK/dV    a wave owns 32 keys (lane l holds key l % 32) and walks the later query chunks:
+//           S = Q K^T and dP = dO V^T with K and V in registers (split once), Q and dO as bf16
+//           planes, P and dS in registers, dV^T += dO^T P and dK^T += Q^T dS (no atomics);
 //  dQ       a wave owns 32 queries again: S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T, with
-//           Q split once, dO split at each use and K, V as bf16 planes;
+//           Q and dO split once and K, V as bf16 planes;
 //  delta    rowsum(dO * O), a separate pass that dK/dV and dQ both read.
-// The next tile is loaded into registers while the current one is on the matrix cores and
-// split into planes as it is stored: 64 rows in the forward, 32 in dK/dV and dQ, where the
-// prefetch registers are needed for the operands.
+// One or two waves share a row group's chunks, by the size of the grid (waves_per_group).
+// The next tile is loaded while the current one is on the matrix cores and split into planes as
+// it is stored: through registers in the forward; in dK/dV and dQ by direct loads into LDS,
+// which leaves the registers to the split operands (splitting dO, K and V once instead of at
+// each use: B16 H12 S1024 backward 606 -> 528 us, bit-identical).
 //
 // The DROP instantiations apply attention-probability dropout with the keep bits of
 // dropout.hpp: the forward and dQ hold keys along registers (keep_words16), dK/dV holds queries
 // along registers (keep_col16).
+#include <type_traits>
+
 #include "common.hpp"
 #include "dropout.hpp"
 #include "kernels.hpp"
@@ -40,13 +43,14 @@
 namespace dadgpt {
 namespace {
 
-constexpr int kWaves = 4;             // waves per workgroup
-// Two workgroups per CU, i.e. at most 256 registers a lane (one wave per SIMD runs the backward
-// ~15% slower). At D = 64 the forward, dQ and dK/dV fit (dK/dV with its plane addresses from
-// LaneLds); the dropout dK/dV spills 19 registers, loop-invariant values reloaded per chunk.
-constexpr int kMinBlocks = 2;
-constexpr int kRows = 32 * kWaves;    // rows (queries or keys) a workgroup owns
-constexpr int kTile = 64;             // rows per staged tile (two 32-row chunks)
+// A workgroup is KG x KS waves: KG row groups of 32 rows (queries, or keys in dK/dV) it owns,
+// and KS waves per group that share its chunks of the other dimension. The staged tile has
+// 32 KS rows; wave (g, s) of a workgroup computes group g against the tile's chunk s, and the KS
+// partial results are merged through LDS at the end.
+constexpr int kGroups = 4;
+constexpr int kRows = 32 * kGroups;  // rows a workgroup owns
+// At most 256 registers a lane (two waves per SIMD; one runs the backward ~15% slower).
+constexpr int wgs_per_cu(int ks) { return 2 / ks; }
 
 // Row (within a 32-row chunk) that score register u of lane half h stands for, when the A
 // operand rows were read through sigma32: 16 * (u / 8) + 8 * h + u % 8.
@@ -81,30 +85,49 @@ __device__ __forceinline__ float exp_acc(float x) {
 // weights below 2^64, the running sums stay far inside fp32 range over any sequence length.
 constexpr float kMaxW = 0x1p64f;
 
-// A TR-row fp32 tile (64 rows in the forward, 32 in the backward kernels, whose registers are
-// scarcer) and its register prefetch: 256 threads, TR*D/1024 16-byte pieces each; rows at or
-// past S read as zeros. Epilogues stage rows at pitch D + 4 floats.
-template <int D, int TR = kTile>
+constexpr int kPitchPad = 4;  // epilogues stage rows of D floats at a pitch of D + 4
+
+// A TR-row fp32 tile and its register prefetch by NT threads, TR*D/(4 NT) 16-byte pieces each;
+// rows at or past S read as zeros.
+template <int D, int TR, int NT>
 struct Tile {
-  static constexpr int kPitch = D + 4;
-  static constexpr int kPieces = TR * D / 4 / 256;
+  static constexpr int kPieces = TR * D / 4 / NT;
+  static constexpr int kThreads = NT;
   f32x4 r[kPieces];
 
   __device__ __forceinline__ void load(const float* src, int row0, int S) {
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
-      const int u = threadIdx.x + 256 * i, row = u / (D / 4), c = u % (D / 4);
+      const int u = threadIdx.x + NT * i, row = u / (D / 4), c = u % (D / 4);
       r[i] = row0 + row < S ? *reinterpret_cast<const f32x4*>(src + (size_t)(row0 + row) * D +
                                                               4 * c)
                             : f32x4{0.f, 0.f, 0.f, 0.f};
     }
   }
-  __device__ __forceinline__ void store(float* lds) const {
+  __device__ __forceinline__ f32x4 piece(int i) const { return r[i]; }
+};
+
+// The same tile prefetched through LDS instead of registers: each lane's pieces travel by direct
+// global -> LDS loads into the lane's own 16-byte slots, so a wave reads back only what it
+// loaded itself and needs no barrier, just its own wait. Rows at or past S read row S-1.
+template <int D, int TR, int NT>
+struct RawTile {
+  static constexpr int kPieces = TR * D / 4 / NT;
+  static constexpr int kThreads = NT;
+  const float* src;
+  float* lds;  // TR * D floats
+  int S, wave, lane;
+  __device__ __forceinline__ void issue(int row0) const {
+    const int left = S - 1 - row0;
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
-      const int u = threadIdx.x + 256 * i, row = u / (D / 4), c = u % (D / 4);
-      *reinterpret_cast<f32x4*>(lds + row * kPitch + 4 * c) = r[i];
+      const int u = NT * i + 64 * wave + lane, row = u / (D / 4), c = u % (D / 4);
+      dma_lds16_sbase(src + (size_t)row0 * D, (uint32_t)(min(row, left) * D + 4 * c) * 4u,
+                      lds + 4 * (NT * i + 64 * wave));
     }
+  }
+  __device__ __forceinline__ f32x4 piece(int i) const {
+    return *reinterpret_cast<const f32x4*>(lds + 4 * (NT * i + 64 * wave + lane));
   }
 };
 
@@ -150,16 +173,17 @@ __device__ __forceinline__ f32x16 mfma_x6(const X3& a, const X3& b, f32x16 acc) 
 // the bf16 kernels (tiles.hpp), so the score operands are ds_read_b128 and the transposed
 // ones ds_read_b64_tr_b16 reads. Each float is split once per workgroup, when the tile is
 // staged, instead of once per wave that reads it.
-template <int D, int TR = kTile>
-__device__ __forceinline__ void store_x3(const Tile<D, TR>& t, bf16* planes) {
+template <int D, int TR, typename T>
+__device__ __forceinline__ void store_x3(const T& t, bf16* planes) {
 #pragma unroll
-  for (int i = 0; i < Tile<D, TR>::kPieces; ++i) {
-    const int u = threadIdx.x + 256 * i, row = u / (D / 4), c = u % (D / 4);
+  for (int i = 0; i < T::kPieces; ++i) {
+    const int u = threadIdx.x + T::kThreads * i, row = u / (D / 4), c = u % (D / 4);
     const int off = rm_off<D>(row, c >> 1) + 4 * (c & 1);  // 4 floats: half a 16-byte chunk
+    const f32x4 x = t.piece(i);
     uint32_t w[3][2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      const float a0 = t.r[i][2 * k], a1 = t.r[i][2 * k + 1];
+      const float a0 = x[2 * k], a1 = x[2 * k + 1];
       const uint32_t p = pack_bf16x2(a0, a1);
       const float b0 = a0 - bf16_lo(p), b1 = a1 - bf16_hi(p);
       const uint32_t q = pack_bf16x2(b0, b1);
@@ -188,7 +212,7 @@ __device__ __forceinline__ void load_split_row(X3 (&x)[D / 16], const float* row
   }
 }
 
-template <int D, int TR = kTile>
+template <int D, int TR>
 __device__ __forceinline__ f32x16 score_tile_p(const bf16* planes, int chunk_row0,
                                                const X3 (&qb)[D / 16], int lane) {
   const int krow = chunk_row0 + sigma32(lane & 31), hi = lane >> 5;
@@ -204,46 +228,7 @@ __device__ __forceinline__ f32x16 score_tile_p(const bf16* planes, int chunk_row
   return acc;
 }
 
-// A global row in the B-operand layout of the score products, as floats: element 8 ds + e is
-// column 16 ds + 8 h + e.
-template <int D>
-__device__ __forceinline__ void load_row_b(float (&x)[D / 2], const float* row, int h) {
-#pragma unroll
-  for (int ds = 0; ds < D / 16; ++ds) {
-    const f32x4 v0 = *reinterpret_cast<const f32x4*>(row + 16 * ds + 8 * h);
-    const f32x4 v1 = *reinterpret_cast<const f32x4*>(row + 16 * ds + 8 * h + 4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[8 * ds + e] = v0[e], x[8 * ds + 4 + e] = v1[e];
-  }
-}
-
-// score_tile_p with the B operand held as floats (the load_split_row layout) and split at
-// each use: for kernels whose registers cannot hold two split rows.
-template <int D, int TR = kTile>
-__device__ __forceinline__ f32x16 score_tile_pf(const bf16* planes, int chunk_row0,
-                                                const float (&bf)[D / 2], int lane) {
-  const int krow = chunk_row0 + sigma32(lane & 31), hi = lane >> 5;
-  f32x16 acc = zero16();
-#pragma unroll
-  for (int ds = 0; ds < D / 16; ++ds) {
-    X3 a;
-#pragma unroll
-    for (int pl = 0; pl < 3; ++pl)
-      a.v[pl] = lds_op(planes + pl * TR * D, rm_off<D>(krow, 2 * ds + hi));
-    float b[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      b[e] = bf[8 * ds + e];
-      // split here, at each use: hoisted out of the tile loop, the splits of a whole row would
-      // hold 1.5x its registers for the kernel's life
-      asm volatile("" : "+v"(b[e]));
-    }
-    acc = mfma_x6(a, split3(b), acc);
-  }
-  return acc;
-}
-
-template <int D, int TR = kTile>
+template <int D, int TR>
 __device__ __forceinline__ void accumulate_t_p(f32x16 (&acc)[D / 32], const bf16* planes,
                                                int chunk_row0, const f32x16& p, int lane) {
 #pragma unroll
@@ -263,11 +248,11 @@ __device__ __forceinline__ void accumulate_t_p(f32x16 (&acc)[D / 32], const bf16
   }
 }
 
-// score_tile_pf and accumulate_t_p at chunk row 0 of TR-row planes, with the addresses from
+// score_tile_p and accumulate_t_p at the start of `planes`, with the addresses from
 // LaneLds (tiles.hpp): the dK/dV kernel's register relief (no spills at D = 64).
 template <int D, int TR>
-__device__ __forceinline__ f32x16 score_tile_pfx(const bf16* planes, const float (&bf)[D / 2],
-                                                 const LaneLds& lo) {
+__device__ __forceinline__ f32x16 score_tile_px(const bf16* planes, const X3 (&b)[D / 16],
+                                                const LaneLds& lo) {
   uint32_t ra[D / 16];
   row_addr_xor<D>(ra, lo.ro);
   f32x16 acc = zero16();
@@ -276,13 +261,7 @@ __device__ __forceinline__ f32x16 score_tile_pfx(const bf16* planes, const float
     X3 a;
 #pragma unroll
     for (int pl = 0; pl < 3; ++pl) a.v[pl] = lds_row_at(planes + pl * TR * D, ra[ds]);
-    float b[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      b[e] = bf[8 * ds + e];
-      asm volatile("" : "+v"(b[e]));
-    }
-    acc = mfma_x6(a, split3(b), acc);
+    acc = mfma_x6(a, b[ds], acc);
   }
   return acc;
 }
@@ -320,7 +299,7 @@ __device__ __forceinline__ void store_rows_t(float* dst, int row0, int S,
   for (int db = 0; db < D / 32; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-      stage[l32 * Tile<D>::kPitch + 32 * db + c32_row(r, h)] = acc[db][r] * mul;
+      stage[l32 * (D + kPitchPad) + 32 * db + c32_row(r, h)] = acc[db][r] * mul;
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's own LDS writes are done
   __builtin_amdgcn_wave_barrier();
   constexpr int kPieces = 32 * D / 4 / 64;
@@ -329,31 +308,63 @@ __device__ __forceinline__ void store_rows_t(float* dst, int row0, int S,
     const int u = lane + 64 * i, row = u / (D / 4), c = u % (D / 4);
     if (row0 + row < S)
       *reinterpret_cast<f32x4*>(dst + (size_t)(row0 + row) * D + 4 * c) =
-          *reinterpret_cast<const f32x4*>(stage + row * Tile<D>::kPitch + 4 * c);
+          *reinterpret_cast<const f32x4*>(stage + row * (D + kPitchPad) + 4 * c);
   }
+}
+
+// Partial sums of the KS waves of a row group, added into the first one's registers through LDS:
+// waves s > 0 write their NA accumulators (`slot`: NA * 16 * 64 floats of the wave's own, lane
+// fastest) and the first wave adds them in order after the barrier, scaled
+// per lane by `mul`.
+template <int NA>
+__device__ __forceinline__ void put_acc(const f32x16 (&acc)[NA], float* slot, int lane) {
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<f32x4*>(slot + ((4 * i + j) * 64 + lane) * 4) =
+          f32x4{acc[i][4 * j], acc[i][4 * j + 1], acc[i][4 * j + 2], acc[i][4 * j + 3]};
+}
+template <int NA>
+__device__ __forceinline__ void add_acc(f32x16 (&acc)[NA], const float* slot, int lane,
+                                        float mul = 1.0f) {
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(slot + ((4 * i + j) * 64 + lane) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][4 * j + e] = fmaf(v[e], mul, acc[i][4 * j + e]);
+    }
 }
 
 // ------------------------------------------------------------------------------ forward
 
-template <int D, bool DROP>
-__global__ __launch_bounds__(64 * kWaves, kMinBlocks) void fwd_f32_kernel(
+template <int D, bool DROP, int KS>
+__global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_kernel(
     float* __restrict__ out, float* __restrict__ lse, const float* __restrict__ q,
     const float* __restrict__ k, const float* __restrict__ v, int S, float scale,
     const DropParams dr) {
-  // K and V tiles as three bf16 planes each; after the tile loop the first holds the
-  // epilogue's fp32 staging rows
-  __shared__ __attribute__((aligned(16))) bf16 skp[3 * kTile * D];
-  __shared__ __attribute__((aligned(16))) bf16 svp[3 * kTile * D];
-  static_assert(3 * kTile * D * 2 >= 2 * 32 * Tile<D>::kPitch * 4, "epilogue staging fits");
+  constexpr int NT = 64 * kGroups * KS, TR = 64, CPT = 2 / KS;  // chunks per tile and wave
+  // K and V tiles as three bf16 planes each; after the tile loop they hold the second waves'
+  // partial results, then the epilogue's fp32 staging rows
+  constexpr int kPlane = 3 * TR * D;
+  __shared__ __attribute__((aligned(16))) bf16 planes[2 * kPlane];
+  bf16 *skp = planes, *svp = planes + kPlane;
+  constexpr int kPart = (D / 32) * 1024 + 128;  // a partial: O, m and l (floats)
+  constexpr int kStage = 32 * (D + kPitchPad);  // a wave's staged rows (floats)
+  static_assert(4 * kPlane >= 4 * kGroups * (KS > 1 && kPart > kStage ? kPart : kStage),
+                "partials and staging fit");
   const int bh = blockIdx.x;
   const int blk = gridDim.y - 1 - blockIdx.y;  // longest query blocks first
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar
+  const int grp = wave % kGroups, sub = wave / kGroups;
   const size_t base = (size_t)bh * S * D;
-  const int q0 = blk * kRows + 32 * wave;  // the wave's first query
-  const int qi = q0 + l32;                 // this lane's query
+  const int q0 = blk * kRows + 32 * grp;  // the wave's first query
+  const int qi = q0 + l32;                // this lane's query
   const int last = min(S, (blk + 1) * kRows) - 1;  // the workgroup's last query
-  const int n_tiles = last / kTile + 1;
+  const int n_tiles = last / TR + 1;
 
   X3 qb[D / 16];  // the lane's query row, split
   load_split_row<D>(qb, q + base + (size_t)min(qi, S - 1) * D, h);
@@ -362,23 +373,24 @@ __global__ __launch_bounds__(64 * kWaves, kMinBlocks) void fwd_f32_kernel(
   for (int db = 0; db < D / 32; ++db) o[db] = zero16();
   float m = neg_inf(), lh = 0.f;  // running maximum; this lane half's sum of weights
 
-  Tile<D> tk, tv;
+  Tile<D, TR, NT> tk, tv;
   tk.load(k + base, 0, S);
   tv.load(v + base, 0, S);
   for (int t = 0; t < n_tiles; ++t) {
     __syncthreads();  // the previous tile's reads are done
-    store_x3<D>(tk, skp);
-    store_x3<D>(tv, svp);
+    store_x3<D, TR>(tk, skp);
+    store_x3<D, TR>(tv, svp);
     __syncthreads();
     if (t + 1 < n_tiles) {  // next tile in flight during this one
-      tk.load(k + base, (t + 1) * kTile, S);
-      tv.load(v + base, (t + 1) * kTile, S);
+      tk.load(k + base, (t + 1) * TR, S);
+      tv.load(v + base, (t + 1) * TR, S);
     }
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int key0 = t * kTile + 32 * c;
+    for (int i = 0; i < CPT; ++i) {
+      const int c = KS == 1 ? i : sub;
+      const int key0 = t * TR + 32 * c;
       if (key0 > q0 + 31) continue;  // wave-uniform: the whole chunk is in the future
-      f32x16 s = score_tile_p<D>(skp, 32 * c, qb, lane);
+      f32x16 s = score_tile_p<D, TR>(skp, 32 * c, qb, lane);
       // only the chunk whose first key is the wave's first query holds keys after a query
       // (or past S); waves are 32-query aligned, so it is the one with key0 == q0
       const bool diag = key0 == q0;
@@ -425,14 +437,37 @@ __global__ __launch_bounds__(64 * kWaves, kMinBlocks) void fwd_f32_kernel(
       if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qi, key0, h);
 #pragma unroll
       for (int u = 0; u < 16; ++u) s[u] = DROP ? w[u] * keep_factor(keep, u, dr) : w[u];
-      accumulate_t_p<D>(o, svp, 32 * c, s, lane);
+      accumulate_t_p<D, TR>(o, svp, 32 * c, s, lane);
     }
+  }
+  __syncthreads();  // every wave is done with the tiles: they hold partials and staging now
+  float* slot = reinterpret_cast<float*>(planes) + grp * (KS > 1 && kPart > kStage ? kPart : kStage);
+  if constexpr (KS == 2) {
+    // (m, l, O) of the group's second wave: rescaled to the larger maximum and added. A wave
+    // that saw no chunk has m = -inf and zeros, which get weight 0.
+    float* ml = slot + (D / 32) * 1024;
+    if (sub == 1) {
+      put_acc(o, slot, lane);
+      ml[lane] = m;
+      ml[64 + lane] = lh;
+    }
+    __syncthreads();
+    if (sub == 1) return;
+    const float m1 = ml[lane], mn = fmaxf(m, m1);
+    const float a0 = m == neg_inf() ? 0.f : exp_acc(m - mn);
+    const float a1 = m1 == neg_inf() ? 0.f : exp_acc(m1 - mn);
+    m = mn;
+    lh = lh * a0 + ml[64 + lane] * a1;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[db][r] *= a0;
+    add_acc(o, slot, lane, a1);
+    __builtin_amdgcn_wave_barrier();
   }
   const float l = sum_halves(lh);
   if (h == 0 && qi < S) lse[(size_t)bh * S + qi] = m + logf(l);
-  __syncthreads();  // every wave is done with the tiles: reuse sk as per-wave staging
-  float* stage = reinterpret_cast<float*>(wave < 2 ? skp : svp) + (wave & 1) * 32 * Tile<D>::kPitch;
-  store_rows_t<D>(out + base, q0, S, o, 1.0f / l, stage, lane);
+  store_rows_t<D>(out + base, q0, S, o, 1.0f / l, slot, lane);
 }
 
 // ----------------------------------------------------------------------------- backward
@@ -458,188 +493,245 @@ __global__ __launch_bounds__(256) void delta_f32_kernel(float* __restrict__ delt
   }
 }
 
-template <int D, bool DROP>
-__global__ __launch_bounds__(64 * kWaves, kMinBlocks) void dkdv_f32_kernel(
+// LDS of the backward kernels (bytes): two streamed tiles of 32 KS rows as three bf16 planes
+// each, and raw; afterwards the partials and staging of the epilogue (`acc` accumulators a wave).
+template <int D, int KS>
+struct BwdLds {
+  static constexpr int TR = 32 * KS, kPlane = 3 * TR * D;
+  static constexpr int kBytes = 2 * kPlane * 2 + 2 * TR * D * 4;
+  static constexpr int slot_floats(int acc) {
+    const int stage = 32 * (D + kPitchPad), part = acc * 1024;
+    return KS > 1 && part > stage ? part : stage;
+  }
+};
+
+template <int D, bool DROP, int KS>
+__global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dkdv_f32_kernel(
     float* __restrict__ dk, float* __restrict__ dv, const float* __restrict__ q,
     const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ dout,
     const float* __restrict__ lse, const float* __restrict__ delta, int S, float scale,
     const DropParams dr) {
-  // Q and dO tiles of TR rows as three bf16 planes each (see the forward); each array also
-  // holds two waves' epilogue staging
-  constexpr int TR = 32;
-  constexpr int kLds = 3 * TR * D > 4 * 32 * Tile<D>::kPitch ? 3 * TR * D
-                                                               : 4 * 32 * Tile<D>::kPitch;
-  __shared__ __attribute__((aligned(16))) bf16 sqp[kLds];
-  __shared__ __attribute__((aligned(16))) bf16 sgp[kLds];
+  // Q and dO tiles: planes and raw
+  using Lds = BwdLds<D, KS>;
+  constexpr int TR = Lds::TR, NT = 64 * kGroups * KS;
+  __shared__ __attribute__((aligned(16))) char smem[Lds::kBytes];
+  bf16 *sqp = reinterpret_cast<bf16*>(smem), *sgp = sqp + Lds::kPlane;
+  float* raw = reinterpret_cast<float*>(sgp + Lds::kPlane);
+  constexpr int kSlot = Lds::slot_floats(2 * (D / 32));
+  static_assert(kGroups * kSlot * 4 <= Lds::kBytes, "partials and staging fit");
   // per query row of the tile: lse, and delta * scale
   __shared__ __attribute__((aligned(16))) float sl[TR], sd[TR];
   const int bh = blockIdx.x, blk = blockIdx.y;  // early key blocks see the most queries: first
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar
+  const int grp = wave % kGroups, sub = wave / kGroups;
   const size_t base = (size_t)bh * S * D;
-  const int k0 = blk * kRows + 32 * wave;  // the wave's first key
-  const int kj = k0 + l32;                 // this lane's key
+  const int k0 = blk * kRows + 32 * grp;  // the wave's first key
+  const int kj = k0 + l32;                // this lane's key
   const int t0 = (blk * kRows) / TR;  // first query tile with a query >= the first key
   const int n_tiles = (S + TR - 1) / TR;
 
-  // the lane's K and V rows (score-product B layout), split at each use
-  float kf[D / 2], vf[D / 2];
-  load_row_b<D>(kf, k + base + (size_t)min(kj, S - 1) * D, h);
-  load_row_b<D>(vf, v + base + (size_t)min(kj, S - 1) * D, h);
-  f32x16 dka[D / 32], dva[D / 32];
+  X3 kb[D / 16], vb[D / 16];  // the lane's K and V rows (score-product B layout), split
+  load_split_row<D>(kb, k + base + (size_t)min(kj, S - 1) * D, h);
+  load_split_row<D>(vb, v + base + (size_t)min(kj, S - 1) * D, h);
+  f32x16 da[2 * (D / 32)];  // dV^T, then dK^T
+  f32x16(&dva)[D / 32] = reinterpret_cast<f32x16(&)[D / 32]>(da[0]);
+  f32x16(&dka)[D / 32] = reinterpret_cast<f32x16(&)[D / 32]>(da[D / 32]);
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db) dka[db] = zero16(), dva[db] = zero16();
+  for (int i = 0; i < 2 * (D / 32); ++i) da[i] = zero16();
 
-  static_assert(TR == 32, "one chunk per tile");
   const LaneLds lo = lane_lds<D>(lane);
-  Tile<D, TR> tq, tg;
+  const RawTile<D, TR, NT> tq{q + base, raw, S, wave, lane},
+      tg{dout + base, raw + TR * D, S, wave, lane};
   float pl = 0.f, pd = 0.f;
   auto load_stats = [&](int row0) {
     const int r = row0 + (threadIdx.x & (TR - 1));
     pl = r < S ? lse[(size_t)bh * S + r] : 0.f;
     pd = r < S ? delta[(size_t)bh * S + r] : 0.f;
   };
-  tq.load(q + base, t0 * TR, S);
-  tg.load(dout + base, t0 * TR, S);
+  tq.issue(t0 * TR);
+  tg.issue(t0 * TR);
   load_stats(t0 * TR);
   for (int t = t0; t < n_tiles; ++t) {
-    __syncthreads();
+    wait_vm_lds<0>();  // this wave's pieces of the tile
+    __syncthreads();   // every wave is done with the previous tile's planes
     store_x3<D, TR>(tq, sqp);
     store_x3<D, TR>(tg, sgp);
     if (threadIdx.x < TR) sl[threadIdx.x] = pl, sd[threadIdx.x] = pd * scale;
     __syncthreads();
     if (t + 1 < n_tiles) {
-      tq.load(q + base, (t + 1) * TR, S);
-      tg.load(dout + base, (t + 1) * TR, S);
+      tq.issue((t + 1) * TR);
+      tg.issue((t + 1) * TR);
       load_stats((t + 1) * TR);
     }
+    const int qrow0 = t * TR + 32 * sub;
+    // wave-uniform: every query of the chunk precedes every key, or lies past S
+    if (qrow0 + 31 < k0 || (KS > 1 && qrow0 >= S)) continue;
+    const bf16 *qc = sqp + 32 * sub * D, *gc = sgp + 32 * sub * D;
+    // lane (l32, h), register u: query qrow0 + reg_row(u, h), key kj
+    f32x16 s = score_tile_px<D, TR>(qc, kb, lo);   // Q K^T
+    f32x16 dp = score_tile_px<D, TR>(gc, vb, lo);  // dO V^T
+    uint32_t keep = 0;
+    if constexpr (DROP) keep = keep_col16(dr, (uint64_t)bh * S + qrow0, k0, lane);
+    // Statistics of the chunk's rows 32 sub + reg_row(u, h): registers 8j..8j+7 are the 8
+    // consecutive rows 32 sub + 16j + 8h .., two 16-byte LDS reads each.
+    // keys after a query, or rows past S, only where the chunk reaches the wave's first
+    // keys or S (wave-uniform)
+    const bool mask = qrow0 < k0 + 31 || qrow0 + 31 >= S;
 #pragma unroll
-    for (int c = 0; c < TR / 32; ++c) {
-      const int qrow0 = t * TR + 32 * c;
-      if (qrow0 + 31 < k0) continue;  // wave-uniform: every query of the chunk precedes every key
-      // lane (l32, h), register u: query qrow0 + reg_row(u, h), key kj
-      f32x16 s = score_tile_pfx<D, TR>(sqp, kf, lo);   // Q K^T
-      f32x16 dp = score_tile_pfx<D, TR>(sgp, vf, lo);  // dO V^T
-      uint32_t keep = 0;
-      if constexpr (DROP) keep = keep_col16(dr, (uint64_t)bh * S + qrow0, k0, lane);
-      // Statistics of the chunk's rows 32c + reg_row(u, h): registers 8j..8j+7 are the 8
-      // consecutive rows 32c + 16j + 8h .., two 16-byte LDS reads each.
-      // keys after a query, or rows past S, only where the chunk reaches the wave's first
-      // keys or S (wave-uniform)
-      const bool mask = qrow0 < k0 + 31 || qrow0 + 31 >= S;
+    for (int g4 = 0; g4 < 4; ++g4) {
+      // registers 4 g4 .. 4 g4 + 3 are the consecutive rows 32 sub + 16(g4/2) + 8h + 4(g4%2) ..;
+      // their statistics are read here, four at a time, rather than all ahead of the loop
+      const int r = 32 * sub + 16 * (g4 >> 1) + 8 * h + 4 * (g4 & 1);
+      asm volatile("" ::: "memory");
+      const f32x4 ls = *reinterpret_cast<const f32x4*>(sl + r);
+      const f32x4 ds = *reinterpret_cast<const f32x4*>(sd + r);
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        // registers 4 g4 .. 4 g4 + 3 are the consecutive rows 32c + 16(g4/2) + 8h + 4(g4%2) ..;
-        // their statistics are read here, four at a time, rather than all ahead of the loop
-        const int r = 32 * c + 16 * (g4 >> 1) + 8 * h + 4 * (g4 & 1);
-        asm volatile("" ::: "memory");
-        const f32x4 ls = *reinterpret_cast<const f32x4*>(sl + r);
-        const f32x4 ds = *reinterpret_cast<const f32x4*>(sd + r);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int u = 4 * g4 + e;
-          const int qrow = qrow0 + reg_row(u, h);
-          float p = exp_acc(fmaf(s[u], scale, -ls[e]));
-          if (mask && !(kj <= qrow && qrow < S)) p = 0.f;
-          float g = dp[u];
-          if constexpr (DROP) {
-            const float f = keep_factor(keep, u, dr.scale);
-            g *= f;
-            s[u] = p * f;  // the probability that multiplied V
-          } else {
-            s[u] = p;
-          }
-          dp[u] = p * fmaf(g, scale, -ds[e]);  // P (dP - delta) scale
+      for (int e = 0; e < 4; ++e) {
+        const int u = 4 * g4 + e;
+        const int qrow = qrow0 + reg_row(u, h);
+        float p = exp_acc(fmaf(s[u], scale, -ls[e]));
+        if (mask && !(kj <= qrow && qrow < S)) p = 0.f;
+        float g = dp[u];
+        if constexpr (DROP) {
+          const float f = keep_factor(keep, u, dr.scale);
+          g *= f;
+          s[u] = p * f;  // the probability that multiplied V
+        } else {
+          s[u] = p;
         }
+        dp[u] = p * fmaf(g, scale, -ds[e]);  // P (dP - delta) scale
       }
-      accumulate_t_px<D, TR>(dva, sgp, s, lo);   // dV^T += dO^T P
-      accumulate_t_px<D, TR>(dka, sqp, dp, lo);  // dK^T += Q^T dS
     }
+    accumulate_t_px<D, TR>(dva, gc, s, lo);   // dV^T += dO^T P
+    accumulate_t_px<D, TR>(dka, qc, dp, lo);  // dK^T += Q^T dS
   }
   __syncthreads();
-  float* stage = reinterpret_cast<float*>(wave < 2 ? sqp : sgp) + (wave & 1) * 32 * Tile<D>::kPitch;
-  store_rows_t<D>(dk + base, k0, S, dka, 1.0f, stage, lane);
-  store_rows_t<D>(dv + base, k0, S, dva, 1.0f, stage, lane);  // after the wave's dK reads
+  float* slot = reinterpret_cast<float*>(smem) + grp * kSlot;
+  if constexpr (KS == 2) {
+    if (sub == 1) put_acc(da, slot, lane);
+    __syncthreads();
+    if (sub == 1) return;
+    add_acc(da, slot, lane);
+    __builtin_amdgcn_wave_barrier();
+  }
+  store_rows_t<D>(dk + base, k0, S, dka, 1.0f, slot, lane);
+  store_rows_t<D>(dv + base, k0, S, dva, 1.0f, slot, lane);  // after the wave's dK reads
 }
 
-template <int D, bool DROP>
-__global__ __launch_bounds__(64 * kWaves, kMinBlocks) void dq_f32_kernel(
+template <int D, bool DROP, int KS>
+__global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dq_f32_kernel(
     float* __restrict__ dq, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ dout, const float* __restrict__ lse,
     const float* __restrict__ delta, int S, float scale, const DropParams dr) {
-  // K and V tiles of TR rows as three bf16 planes each (see the forward); each array also
-  // holds two waves' epilogue staging
-  constexpr int TR = 32;
-  constexpr int kLds = 3 * TR * D > 4 * 32 * Tile<D>::kPitch ? 3 * TR * D
-                                                               : 4 * 32 * Tile<D>::kPitch;
-  __shared__ __attribute__((aligned(16))) bf16 skp[kLds];
-  __shared__ __attribute__((aligned(16))) bf16 svp[kLds];
+  // K and V tiles: planes and raw
+  using Lds = BwdLds<D, KS>;
+  constexpr int TR = Lds::TR, NT = 64 * kGroups * KS;
+  __shared__ __attribute__((aligned(16))) char smem[Lds::kBytes];
+  bf16 *skp = reinterpret_cast<bf16*>(smem), *svp = skp + Lds::kPlane;
+  float* raw = reinterpret_cast<float*>(svp + Lds::kPlane);
+  constexpr int kSlot = Lds::slot_floats(D / 32);
+  static_assert(kGroups * kSlot * 4 <= Lds::kBytes, "partials and staging fit");
   const int bh = blockIdx.x;
   const int blk = gridDim.y - 1 - blockIdx.y;  // longest query blocks first
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar
+  const int grp = wave % kGroups, sub = wave / kGroups;
   const size_t base = (size_t)bh * S * D;
-  const int q0 = blk * kRows + 32 * wave;
+  const int q0 = blk * kRows + 32 * grp;
   const int qi = q0 + l32;
   const int qc = min(qi, S - 1);
   const int last = min(S, (blk + 1) * kRows) - 1;
   const int n_tiles = last / TR + 1;
 
-  // the lane's Q row split once, its dO row (columns 16 ds + 8 h + 0..7) split at each use
-  X3 qb[D / 16];
+  X3 qb[D / 16], gb[D / 16];  // the lane's Q and dO rows (score-product B layout), split
   load_split_row<D>(qb, q + base + (size_t)qc * D, h);
-  float gf[D / 2];
-  load_row_b<D>(gf, dout + base + (size_t)qc * D, h);
+  load_split_row<D>(gb, dout + base + (size_t)qc * D, h);
   const float my_lse = lse[(size_t)bh * S + qc];
   const float my_dscale = delta[(size_t)bh * S + qc] * scale;
   f32x16 acc[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) acc[db] = zero16();
 
-  Tile<D, TR> tk, tv;
-  tk.load(k + base, 0, S);
-  tv.load(v + base, 0, S);
+  const RawTile<D, TR, NT> tk{k + base, raw, S, wave, lane},
+      tv{v + base, raw + TR * D, S, wave, lane};
+  tk.issue(0);
+  tv.issue(0);
   for (int t = 0; t < n_tiles; ++t) {
-    __syncthreads();
+    wait_vm_lds<0>();  // this wave's pieces of the tile
+    __syncthreads();   // every wave is done with the previous tile's planes
     store_x3<D, TR>(tk, skp);
     store_x3<D, TR>(tv, svp);
     __syncthreads();
     if (t + 1 < n_tiles) {
-      tk.load(k + base, (t + 1) * TR, S);
-      tv.load(v + base, (t + 1) * TR, S);
+      tk.issue((t + 1) * TR);
+      tv.issue((t + 1) * TR);
+    }
+    const int key0 = t * TR + 32 * sub;
+    if (key0 > q0 + 31) continue;  // wave-uniform: the whole chunk is in the future
+    // lane (l32, h), register u: query qi, key key0 + reg_row(u, h)
+    f32x16 s = score_tile_p<D, TR>(skp, 32 * sub, qb, lane);   // K Q^T
+    f32x16 dp = score_tile_p<D, TR>(svp, 32 * sub, gb, lane);  // V dO^T
+    KeepWords16 keep = {};
+    if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qi, key0, h);
+    // only the chunk whose first key is the wave's first query holds keys after a query (or
+    // past S): waves are 32-query aligned
+    const bool diag = key0 == q0;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s[u] = exp_acc(fmaf(s[u], scale, -my_lse));  // P
+    if (diag) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (key0 + reg_row(u, h) > qi) s[u] = 0.f;
     }
 #pragma unroll
-    for (int c = 0; c < TR / 32; ++c) {
-      const int key0 = t * TR + 32 * c;
-      if (key0 > q0 + 31) continue;
-      // lane (l32, h), register u: query qi, key key0 + reg_row(u, h)
-      f32x16 s = score_tile_p<D, TR>(skp, 32 * c, qb, lane);   // K Q^T
-      f32x16 dp = score_tile_pf<D, TR>(svp, 32 * c, gf, lane);  // V dO^T
-      KeepWords16 keep = {};
-      if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qi, key0, h);
-      // only the chunk whose first key is the wave's first query holds keys after a query (or
-      // past S): waves are 32-query aligned
-      const bool diag = key0 == q0;
-#pragma unroll
-      for (int u = 0; u < 16; ++u) s[u] = exp_acc(fmaf(s[u], scale, -my_lse));  // P
-      if (diag) {
-#pragma unroll
-        for (int u = 0; u < 16; ++u)
-          if (key0 + reg_row(u, h) > qi) s[u] = 0.f;
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const float p = s[u];
-        float g = dp[u];
-        if constexpr (DROP) g *= keep_factor(keep, u, dr);
-        s[u] = p * fmaf(g, scale, -my_dscale);  // P (dP - delta) scale
-      }
-      accumulate_t_p<D, TR>(acc, skp, 32 * c, s, lane);  // dQ^T += K^T dS^T
+    for (int u = 0; u < 16; ++u) {
+      const float p = s[u];
+      float g = dp[u];
+      if constexpr (DROP) g *= keep_factor(keep, u, dr);
+      s[u] = p * fmaf(g, scale, -my_dscale);  // P (dP - delta) scale
     }
+    accumulate_t_p<D, TR>(acc, skp, 32 * sub, s, lane);  // dQ^T += K^T dS^T
   }
   __syncthreads();
-  float* stage = reinterpret_cast<float*>(wave < 2 ? skp : svp) + (wave & 1) * 32 * Tile<D>::kPitch;
-  store_rows_t<D>(dq + base, q0, S, acc, 1.0f, stage, lane);
+  float* slot = reinterpret_cast<float*>(smem) + grp * kSlot;
+  if constexpr (KS == 2) {
+    if (sub == 1) put_acc(acc, slot, lane);
+    __syncthreads();
+    if (sub == 1) return;
+    add_acc(acc, slot, lane);
+    __builtin_amdgcn_wave_barrier();
+  }
+  store_rows_t<D>(dq + base, q0, S, acc, 1.0f, slot, lane);
+}
+
+// Waves per row group. With one, a workgroup walks its chunks four waves wide, two workgroups
+// to a CU; a grid of no more workgroups than that (all of them start at once) lasts as long as
+// the longest one's chain, so each group then gets a second wave and the chain is half as long.
+// B4 H12 S1024 D64 (384 workgroups): forward 64.6 -> 49.6 us, backward 197 -> 162 us; B8 H8
+// (512): 68.9 -> 60.8, 212 -> 196. Larger grids keep the CUs busy anyway and would pay for the
+// wider barrier and the merge: 640 workgroups 141 -> 147 and 453 -> 468 us, B16 H12 S1024 (1,536)
+// 165 -> 186 and 528 -> 600 us. Up to three chunks (S <= 96) there is too little to share: S 65
+// backward 27.7 -> 29.5 us, S 100 34.5 -> 33.3.
+int waves_per_group(int BH, int S) {
+  const long long wgs = (long long)BH * ((S + kRows - 1) / kRows);
+  return S > 96 && wgs <= 2LL * device_cus() ? 2 : 1;
+}
+
+// f(whether to drop, waves per row group) as compile-time constants.
+template <typename F>
+void with_shape(int BH, int S, bool drop, F f) {
+  const bool two = waves_per_group(BH, S) == 2;
+  auto with_drop = [&](auto d) {
+    if (two)
+      f(d, std::integral_constant<int, 2>{});
+    else
+      f(d, std::integral_constant<int, 1>{});
+  };
+  if (drop)
+    with_drop(std::true_type{});
+  else
+    with_drop(std::false_type{});
 }
 
 template <int D>
@@ -647,10 +739,10 @@ hipError_t fwd_f32_t(float* out, float* lse, const float* q, const float* k, con
                      int BH, int S, float scale, hipStream_t stream, const Dropout* drop) {
   const dim3 grid(BH, (S + kRows - 1) / kRows);
   const DropParams dr = drop_params(drop);
-  if (drop != nullptr)
-    fwd_f32_kernel<D, true><<<grid, 64 * kWaves, 0, stream>>>(out, lse, q, k, v, S, scale, dr);
-  else
-    fwd_f32_kernel<D, false><<<grid, 64 * kWaves, 0, stream>>>(out, lse, q, k, v, S, scale, dr);
+  with_shape(BH, S, drop != nullptr, [&](auto drop_c, auto ks) {
+    fwd_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(out, lse, q, k, v,
+                                                                             S, scale, dr);
+  });
   return hipGetLastError();
 }
 
@@ -667,21 +759,16 @@ hipError_t bwd_f32_t(float* dq, float* dk, float* dv, float* delta, const float*
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const dim3 grid(BH, (S + kRows - 1) / kRows);
-  if (drop != nullptr)
-    dkdv_f32_kernel<D, true><<<grid, 64 * kWaves, 0, stream>>>(dk, dv, q, k, v, dout, lse,
-                                                               delta, S, scale, dr);
-  else
-    dkdv_f32_kernel<D, false><<<grid, 64 * kWaves, 0, stream>>>(dk, dv, q, k, v, dout, lse,
-                                                                delta, S, scale, dr);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (drop != nullptr)
-    dq_f32_kernel<D, true><<<grid, 64 * kWaves, 0, stream>>>(dq, q, k, v, dout, lse, delta, S,
-                                                             scale, dr);
-  else
-    dq_f32_kernel<D, false><<<grid, 64 * kWaves, 0, stream>>>(dq, q, k, v, dout, lse, delta, S,
-                                                              scale, dr);
-  return hipGetLastError();
+  with_shape(BH, S, drop != nullptr, [&](auto drop_c, auto ks) {
+    dkdv_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(
+        dk, dv, q, k, v, dout, lse, delta, S, scale, dr);
+    e = hipGetLastError();
+    if (e != hipSuccess) return;
+    dq_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(
+        dq, q, k, v, dout, lse, delta, S, scale, dr);
+    e = hipGetLastError();
+  });
+  return e;
 }
 
 }  // namespace

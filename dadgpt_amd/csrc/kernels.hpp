@@ -54,6 +54,9 @@ struct Dropout {
   uint64_t seed;
 };
 
+// Compute units of the current device (cached per device; 0 if unknown).
+int device_cus();
+
 // Causal flash forward, bf16 in/out, fp32 logsumexp (natural log) [BH, S]. q, k, v, out as
 // `layout` places them (tensors kTQ, kTK, kTV, kTO), D in {32,64}. With `drop`, the
 // probabilities multiplying V are dropped (the logsumexp is that of the undropped scores).
