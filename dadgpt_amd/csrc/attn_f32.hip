@@ -23,7 +23,7 @@
 //  dQ       a wave owns 32 queries again: S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T, with
 //           Q and dO split once and K, V as bf16 planes;
 //  delta    rowsum(dO * O), a separate pass that dK/dV and dQ both read.
-// One or two waves share a row group's chunks, by the size of the grid (waves_per_group).
+// One or two waves share a row group's chunks, by the size of the grid (f32_waves_per_group).
 // The next tile is loaded while the current one is on the matrix cores and split into planes as
 // it is stored: through registers in the forward; in dK/dV and dQ by direct loads into LDS,
 // which leaves the registers to the split operands (splitting dO, K and V once instead of at
@@ -143,14 +143,23 @@ struct X3 {
   bf16x8 v[3];
 };
 
+// pack_bf16x2 for a word whose halves are taken apart again: opaque, because the compiler would
+// otherwise convert the low half a second time instead of shifting it out of the word (48 of
+// dK/dV's 576 VALU instructions per chunk).
+__device__ __forceinline__ uint32_t pack_once(float lo, float hi) {
+  uint32_t w = pack_bf16x2(lo, hi);
+  asm("" : "+v"(w));
+  return w;
+}
+
 __device__ __forceinline__ X3 split3(const float (&x)[8]) {
   u32x4 w[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float a0 = x[2 * i], a1 = x[2 * i + 1];
-    const uint32_t p = pack_bf16x2(a0, a1);
+    const uint32_t p = pack_once(a0, a1);
     const float b0 = a0 - bf16_lo(p), b1 = a1 - bf16_hi(p);  // exact
-    const uint32_t q = pack_bf16x2(b0, b1);
+    const uint32_t q = pack_once(b0, b1);
     const float c0 = b0 - bf16_lo(q), c1 = b1 - bf16_hi(q);  // exact
     w[0][i] = p;
     w[1][i] = q;
@@ -184,9 +193,9 @@ __device__ __forceinline__ void store_x3(const T& t, bf16* planes) {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const float a0 = x[2 * k], a1 = x[2 * k + 1];
-      const uint32_t p = pack_bf16x2(a0, a1);
+      const uint32_t p = pack_once(a0, a1);
       const float b0 = a0 - bf16_lo(p), b1 = a1 - bf16_hi(p);
-      const uint32_t q = pack_bf16x2(b0, b1);
+      const uint32_t q = pack_once(b0, b1);
       w[0][k] = p;
       w[1][k] = q;
       w[2][k] = pack_bf16x2(b0 - bf16_lo(q), b1 - bf16_hi(q));
@@ -312,32 +321,6 @@ __device__ __forceinline__ void store_rows_t(float* dst, int row0, int S,
   }
 }
 
-// Partial sums of the KS waves of a row group, added into the first one's registers through LDS:
-// waves s > 0 write their NA accumulators (`slot`: NA * 16 * 64 floats of the wave's own, lane
-// fastest) and the first wave adds them in order after the barrier, scaled
-// per lane by `mul`.
-template <int NA>
-__device__ __forceinline__ void put_acc(const f32x16 (&acc)[NA], float* slot, int lane) {
-#pragma unroll
-  for (int i = 0; i < NA; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<f32x4*>(slot + ((4 * i + j) * 64 + lane) * 4) =
-          f32x4{acc[i][4 * j], acc[i][4 * j + 1], acc[i][4 * j + 2], acc[i][4 * j + 3]};
-}
-template <int NA>
-__device__ __forceinline__ void add_acc(f32x16 (&acc)[NA], const float* slot, int lane,
-                                        float mul = 1.0f) {
-#pragma unroll
-  for (int i = 0; i < NA; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(slot + ((4 * i + j) * 64 + lane) * 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[i][4 * j + e] = fmaf(v[e], mul, acc[i][4 * j + e]);
-    }
-}
-
 // ------------------------------------------------------------------------------ forward
 
 template <int D, bool DROP, int KS>
@@ -447,7 +430,7 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
     // that saw no chunk has m = -inf and zeros, which get weight 0.
     float* ml = slot + (D / 32) * 1024;
     if (sub == 1) {
-      put_acc(o, slot, lane);
+      put_acc(o, reinterpret_cast<AccLds*>(slot), lane);
       ml[lane] = m;
       ml[64 + lane] = lh;
     }
@@ -462,7 +445,7 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[db][r] *= a0;
-    add_acc(o, slot, lane, a1);
+    add_acc(o, reinterpret_cast<const AccLds*>(slot), lane, a1);
     __builtin_amdgcn_wave_barrier();
   }
   const float l = sum_halves(lh);
@@ -534,6 +517,13 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dkdv_f32_ke
   X3 kb[D / 16], vb[D / 16];  // the lane's K and V rows (score-product B layout), split
   load_split_row<D>(kb, k + base + (size_t)min(kj, S - 1) * D, h);
   load_split_row<D>(vb, v + base + (size_t)min(kj, S - 1) * D, h);
+#pragma unroll
+  for (int ds = 0; ds < D / 16; ++ds)
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) {
+      asm volatile("" : "+v"(kb[ds].v[pl]));
+      asm volatile("" : "+v"(vb[ds].v[pl]));
+    }
   f32x16 da[2 * (D / 32)];  // dV^T, then dK^T
   f32x16(&dva)[D / 32] = reinterpret_cast<f32x16(&)[D / 32]>(da[0]);
   f32x16(&dka)[D / 32] = reinterpret_cast<f32x16(&)[D / 32]>(da[D / 32]);
@@ -578,41 +568,48 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dkdv_f32_ke
     // keys after a query, or rows past S, only where the chunk reaches the wave's first
     // keys or S (wave-uniform)
     const bool mask = qrow0 < k0 + 31 || qrow0 + 31 >= S;
+    // (the mask's compares and selects, 80 instructions, only in the instance that needs them)
+    auto weights = [&](auto masked) {
 #pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      // registers 4 g4 .. 4 g4 + 3 are the consecutive rows 32 sub + 16(g4/2) + 8h + 4(g4%2) ..;
-      // their statistics are read here, four at a time, rather than all ahead of the loop
-      const int r = 32 * sub + 16 * (g4 >> 1) + 8 * h + 4 * (g4 & 1);
-      asm volatile("" ::: "memory");
-      const f32x4 ls = *reinterpret_cast<const f32x4*>(sl + r);
-      const f32x4 ds = *reinterpret_cast<const f32x4*>(sd + r);
+      for (int g4 = 0; g4 < 4; ++g4) {
+        // registers 4 g4 .. 4 g4 + 3 are the consecutive rows 32 sub + 16(g4/2) + 8h + 4(g4%2) ..;
+        // their statistics are read here, four at a time, rather than all ahead of the loop
+        const int r = 32 * sub + 16 * (g4 >> 1) + 8 * h + 4 * (g4 & 1);
+        asm volatile("" ::: "memory");
+        const f32x4 ls = *reinterpret_cast<const f32x4*>(sl + r);
+        const f32x4 ds = *reinterpret_cast<const f32x4*>(sd + r);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int u = 4 * g4 + e;
-        const int qrow = qrow0 + reg_row(u, h);
-        float p = exp_acc(fmaf(s[u], scale, -ls[e]));
-        if (mask && !(kj <= qrow && qrow < S)) p = 0.f;
-        float g = dp[u];
-        if constexpr (DROP) {
-          const float f = keep_factor(keep, u, dr.scale);
-          g *= f;
-          s[u] = p * f;  // the probability that multiplied V
-        } else {
-          s[u] = p;
+        for (int e = 0; e < 4; ++e) {
+          const int u = 4 * g4 + e;
+          const int qrow = qrow0 + reg_row(u, h);
+          float p = exp_acc(fmaf(s[u], scale, -ls[e]));
+          if (masked() && !(kj <= qrow && qrow < S)) p = 0.f;
+          float g = dp[u];
+          if constexpr (DROP) {
+            const float f = keep_factor(keep, u, dr.scale);
+            g *= f;
+            s[u] = p * f;  // the probability that multiplied V
+          } else {
+            s[u] = p;
+          }
+          dp[u] = p * fmaf(g, scale, -ds[e]);  // P (dP - delta) scale
         }
-        dp[u] = p * fmaf(g, scale, -ds[e]);  // P (dP - delta) scale
       }
-    }
+    };
+    if (mask)
+      weights(std::true_type{});
+    else
+      weights(std::false_type{});
     accumulate_t_px<D, TR>(dva, gc, s, lo);   // dV^T += dO^T P
     accumulate_t_px<D, TR>(dka, qc, dp, lo);  // dK^T += Q^T dS
   }
   __syncthreads();
   float* slot = reinterpret_cast<float*>(smem) + grp * kSlot;
   if constexpr (KS == 2) {
-    if (sub == 1) put_acc(da, slot, lane);
+    if (sub == 1) put_acc(da, reinterpret_cast<AccLds*>(slot), lane);
     __syncthreads();
     if (sub == 1) return;
-    add_acc(da, slot, lane);
+    add_acc(da, reinterpret_cast<const AccLds*>(slot), lane);
     __builtin_amdgcn_wave_barrier();
   }
   store_rows_t<D>(dk + base, k0, S, dka, 1.0f, slot, lane);
@@ -696,10 +693,10 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dq_f32_kern
   __syncthreads();
   float* slot = reinterpret_cast<float*>(smem) + grp * kSlot;
   if constexpr (KS == 2) {
-    if (sub == 1) put_acc(acc, slot, lane);
+    if (sub == 1) put_acc(acc, reinterpret_cast<AccLds*>(slot), lane);
     __syncthreads();
     if (sub == 1) return;
-    add_acc(acc, slot, lane);
+    add_acc(acc, reinterpret_cast<const AccLds*>(slot), lane);
     __builtin_amdgcn_wave_barrier();
   }
   store_rows_t<D>(dq + base, q0, S, acc, 1.0f, slot, lane);
@@ -708,20 +705,21 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dq_f32_kern
 // Waves per row group. With one, a workgroup walks its chunks four waves wide, two workgroups
 // to a CU; a grid of no more workgroups than that (all of them start at once) lasts as long as
 // the longest one's chain, so each group then gets a second wave and the chain is half as long.
+// (all figures before the mask branch and pack_once below, which took another 2-7%)
 // B4 H12 S1024 D64 (384 workgroups): forward 64.6 -> 49.6 us, backward 197 -> 162 us; B8 H8
 // (512): 68.9 -> 60.8, 212 -> 196. Larger grids keep the CUs busy anyway and would pay for the
 // wider barrier and the merge: 640 workgroups 141 -> 147 and 453 -> 468 us, B16 H12 S1024 (1,536)
 // 165 -> 186 and 528 -> 600 us. Up to three chunks (S <= 96) there is too little to share: S 65
 // backward 27.7 -> 29.5 us, S 100 34.5 -> 33.3.
-int waves_per_group(int BH, int S) {
+int f32_waves_per_group(int BH, int S) {
   const long long wgs = (long long)BH * ((S + kRows - 1) / kRows);
   return S > 96 && wgs <= 2LL * device_cus() ? 2 : 1;
 }
 
 // f(whether to drop, waves per row group) as compile-time constants.
 template <typename F>
-void with_shape(int BH, int S, bool drop, F f) {
-  const bool two = waves_per_group(BH, S) == 2;
+void with_f32_shape(int BH, int S, bool drop, F f) {
+  const bool two = f32_waves_per_group(BH, S) == 2;
   auto with_drop = [&](auto d) {
     if (two)
       f(d, std::integral_constant<int, 2>{});
@@ -739,7 +737,7 @@ hipError_t fwd_f32_t(float* out, float* lse, const float* q, const float* k, con
                      int BH, int S, float scale, hipStream_t stream, const Dropout* drop) {
   const dim3 grid(BH, (S + kRows - 1) / kRows);
   const DropParams dr = drop_params(drop);
-  with_shape(BH, S, drop != nullptr, [&](auto drop_c, auto ks) {
+  with_f32_shape(BH, S, drop != nullptr, [&](auto drop_c, auto ks) {
     fwd_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(out, lse, q, k, v,
                                                                              S, scale, dr);
   });
@@ -759,7 +757,7 @@ hipError_t bwd_f32_t(float* dq, float* dk, float* dv, float* delta, const float*
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const dim3 grid(BH, (S + kRows - 1) / kRows);
-  with_shape(BH, S, drop != nullptr, [&](auto drop_c, auto ks) {
+  with_f32_shape(BH, S, drop != nullptr, [&](auto drop_c, auto ks) {
     dkdv_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(
         dk, dv, q, k, v, dout, lse, delta, S, scale, dr);
     e = hipGetLastError();

@@ -10,12 +10,31 @@
 // 32- or a 64-bank LDS.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
 namespace dadgpt {
 
 constexpr int kTileRows = 64;
+
+// f(strided, dropped, waves per group) as compile-time constants (dropout is contiguous only).
+template <typename F>
+void with_shape(int waves_per_group, bool drop, bool strided, F f) {
+  auto with_waves = [&](auto s, auto d) {
+    if (waves_per_group == 2)
+      f(s, d, std::integral_constant<int, 2>{});
+    else
+      f(s, d, std::integral_constant<int, 1>{});
+  };
+  if (drop)
+    with_waves(std::false_type{}, std::true_type{});
+  else if (strided)
+    with_waves(std::true_type{}, std::false_type{});
+  else
+    with_waves(std::false_type{}, std::false_type{});
+}
 
 // Where tensor t's rows of slice bh lie. STRIDED = false is the contiguous [BH, S, D] layout
 // with every offset a compile-time multiple of D; STRIDED = true reads the layout (kernels.hpp).
@@ -295,6 +314,34 @@ __device__ __forceinline__ void store_rows_staged(bf16* dst, int pitch, int rows
     if (r < rows_valid)
       __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst + (size_t)r * pitch + c * 8));
   }
+}
+
+// Partial accumulators passed between waves through LDS, one 32x32 block as four 16-byte pieces
+// a lane, lane fastest (no bank conflicts): put_acc writes a wave's NA blocks, add_acc adds them
+// to another wave's, times the lane's `mul`.
+struct AccLds {
+  f32x4 piece[4][64];
+};
+template <int NA>
+__device__ __forceinline__ void put_acc(const f32x16 (&acc)[NA], AccLds* slot, int lane) {
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      slot[i].piece[j][lane] =
+          f32x4{acc[i][4 * j], acc[i][4 * j + 1], acc[i][4 * j + 2], acc[i][4 * j + 3]};
+}
+template <int NA>
+__device__ __forceinline__ void add_acc(f32x16 (&acc)[NA], const AccLds* slot, int lane,
+                                        float mul = 1.0f) {
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 v = slot[i].piece[j][lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][4 * j + e] = fmaf(v[e], mul, acc[i][4 * j + e]);
+    }
 }
 
 // s_waitcnt: vector-memory count <= N and every LDS operation done (gfx9 encoding: vmcnt in
