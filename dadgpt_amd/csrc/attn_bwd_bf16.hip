@@ -19,6 +19,8 @@
 // Masking runs only in the blocks that straddle the diagonal, behind a uniform branch around
 // the instructions that zero P. The streamed tiles (Q and dO for dK/dV, K and V for dQ) are
 // double-buffered in LDS through direct global->LDS loads, one tile ahead of the compute.
+// On small grids (KS = 2, waves_per_group) a workgroup owns 64 rows instead of 128 and two waves
+// share each 32-row group, taking one chunk of every tile each; their sums are merged at the end.
 // STRIDED and DROP instantiations as in the forward: per-tensor strides, and dropout with
 // the keep bits regenerated (dV from P keep/(1-p), dS = P (dP keep/(1-p) - delta)).
 #include "common.hpp"
@@ -231,13 +233,13 @@ __device__ __forceinline__ void dkdv_block(bool mask, f32x16 (&dkacc)[D / 32],
   }
 }
 
-template <int D, bool STRIDED, bool DROP>
+template <int D, bool STRIDED, bool DROP, int KS>
 __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocksNoDrop) void dkdv_bf16_kernel(
     bf16* __restrict__ dk, bf16* __restrict__ dv, const bf16* __restrict__ q,
     const bf16* __restrict__ k, const bf16* __restrict__ v, const bf16* __restrict__ dout,
     const float* __restrict__ lse, const float* __restrict__ delta, int S, float c,
     float lse_mul, float dk_mul, const AttnLayout L, const DropParams dr) {
-  constexpr int KB = kKW * kWaves;
+  constexpr int kGroups = kWaves / KS, KB = kKW * kGroups;  // key groups, keys
   constexpr int DS = D / 16, DB = D / 32;
   // Q and dO tiles, double-buffered (constant buffer indices in the unrolled loop; see the
   // forward kernel), and per wave and buffer the tile's lse and delta rows, converted in place
@@ -253,6 +255,7 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
+  const int grp = wave % kGroups, sub = wave / kGroups;
   const Slice<D, STRIDED> sl(L, bh, S);
   const bf16* qg = sl.base(q, kTQ);
   const bf16* dog = sl.base(dout, kTDO);
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
   const float* lseg = lse + (size_t)bh * S;
   const float* delg = delta + (size_t)bh * S;
 
-  const int kw0 = kblk * KB + wave * kKW;
+  const int kw0 = kblk * KB + grp * kKW;
   const int key = kw0 + l32;
   const int t_first = (kblk * KB) / kTileRows;
   const int t_end = (S - 1) / kTileRows + 1;
@@ -317,8 +320,8 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
       st[cb][1][lane] = -st[cb][1][lane];
       const bool edge = r0 + kTileRows > S;
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
-        const int qlo = r0 + 32 * qb;  // first query of the block
+      for (int i = 0; i < 2 / KS; ++i) {
+        const int qb = KS == 1 ? i : sub, qlo = r0 + 32 * qb;  // first query of the block
         if (qlo + 31 < kw0) continue;   // every key of the wave is after every query
         uint32_t keep = 0;
         if constexpr (DROP) keep = keep_col16(dr, (uint64_t)bh * S + qlo, kw0, lane);
@@ -336,13 +339,36 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
     if (t + 1 < t_end) tile(t + 1, sq[1], sdo[1], 1, sq[0], sdo[0], 0);
   }
 
-  // the tiles are free after the last barrier: each wave stages its 32 rows in its quarter
-  // of sq (dK) and sdo (dV)
-  if (kw0 < S) {
-    store_rows_staged<D>(sl.row(dk, kTDK, kw0), sl.pitch(kTDK), S - kw0, dkacc, dk_mul,
-                         &sq[0][0] + wave * kKW * D, lane);
-    store_rows_staged<D>(sl.row(dv, kTDV, kw0), sl.pitch(kTDV), S - kw0, dvacc, 1.0f,
-                         &sdo[0][0] + wave * kKW * D, lane);
+  // the tiles are free after the last barrier
+  if constexpr (KS == 1) {
+    // each wave stages its 32 rows in its quarter of sq (dK) and sdo (dV)
+    if (kw0 < S) {
+      store_rows_staged<D>(sl.row(dk, kTDK, kw0), sl.pitch(kTDK), S - kw0, dkacc, dk_mul,
+                           &sq[0][0] + wave * kKW * D, lane);
+      store_rows_staged<D>(sl.row(dv, kTDV, kw0), sl.pitch(kTDV), S - kw0, dvacc, 1.0f,
+                           &sdo[0][0] + wave * kKW * D, lane);
+    }
+  } else {
+    // The group's two waves exchange partials: the first finishes dK, the second dV, each in
+    // the group's slot of sq / sdo (partials in, rows staged out).
+    static_assert(sizeof(sq) >= kGroups * DB * sizeof(AccLds), "a group's partials fit");
+    AccLds* slot_k = reinterpret_cast<AccLds*>(&sq[0][0]) + grp * DB;
+    AccLds* slot_v = reinterpret_cast<AccLds*>(&sdo[0][0]) + grp * DB;
+    if (sub == 1)
+      put_acc(dkacc, slot_k, lane);
+    else
+      put_acc(dvacc, slot_v, lane);
+    __syncthreads();
+    if (kw0 >= S) return;
+    if (sub == 0) {
+      add_acc(dkacc, slot_k, lane);
+      store_rows_staged<D>(sl.row(dk, kTDK, kw0), sl.pitch(kTDK), S - kw0, dkacc, dk_mul,
+                           reinterpret_cast<bf16*>(slot_k), lane);
+    } else {
+      add_acc(dvacc, slot_v, lane);
+      store_rows_staged<D>(sl.row(dv, kTDV, kw0), sl.pitch(kTDV), S - kw0, dvacc, 1.0f,
+                           reinterpret_cast<bf16*>(slot_v), lane);
+    }
   }
 }
 
@@ -417,13 +443,13 @@ __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
 // dQ for one query block per wave; the kernel also computes delta = rowsum(dO * O) of its
 // rows (from the dO operands it holds and one load of O) and writes it for the dK/dV kernel,
 // so the backward needs no separate delta pass.
-template <int D, bool STRIDED, bool DROP>
+template <int D, bool STRIDED, bool DROP, int KS>
 __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(
     bf16* __restrict__ dq, float* __restrict__ delta, const bf16* __restrict__ q,
     const bf16* __restrict__ k, const bf16* __restrict__ v, const bf16* __restrict__ dout,
     const bf16* __restrict__ out, const float* __restrict__ lse, int S, float scale_log2,
     float scale, const AttnLayout L, const DropParams dr) {
-  constexpr int QB = kQW * kWaves;
+  constexpr int kGroups = kWaves / KS, QB = kQW * kGroups;  // query groups, queries
   constexpr int DS = D / 16, DB = D / 32;
   // K and V tiles, double-buffered (constant buffer indices; see the forward kernel).
   __shared__ __attribute__((aligned(16))) bf16 sk[2][kTileRows * D];
@@ -435,12 +461,13 @@ __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
+  const int grp = wave % kGroups, sub = wave / kGroups;
   const Slice<D, STRIDED> sl(L, bh, S);
   const bf16* kg = sl.base(k, kTK);
   const bf16* vg = sl.base(v, kTV);
   const int kp = sl.pitch(kTK), vp = sl.pitch(kTV);  // row pitches of the streamed tiles
 
-  const int q0 = qblk * QB + wave * kQW;
+  const int q0 = qblk * QB + grp * kQW;
   const int qrow = q0 + l32;
   const int wg_last = min(S, (qblk + 1) * QB) - 1;
   const int n_tiles = wg_last / kTileRows + 1;
@@ -487,7 +514,7 @@ __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(
       dpart += bf16_lo(a[w]) * bf16_lo(o[w]) + bf16_hi(a[w]) * bf16_hi(o[w]);
   }
   const float dlt = sum_halves(dpart);
-  if (hi == 0 && qrow < S) delta[(size_t)bh * S + qrow] = dlt;
+  if (hi == 0 && qrow < S && sub == 0) delta[(size_t)bh * S + qrow] = dlt;
 
   auto tile = [&](int t, const bf16* ck, const bf16* cv, bf16* nk, bf16* nv) {
     const int k0 = t * kTileRows;
@@ -497,8 +524,8 @@ __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(
     }
     if (q0 < S) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const int klo = k0 + 32 * kb;        // first key of the chunk
+      for (int i = 0; i < 2 / KS; ++i) {
+        const int kb = KS == 1 ? i : sub, klo = k0 + 32 * kb;  // first key of the chunk
         if (klo > q0 + kQW - 1) continue;    // every key after every query of the wave
         KeepWords16 keep = {};
         if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qrow, klo, hi);
@@ -515,9 +542,17 @@ __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(
     if (t + 1 < n_tiles) tile(t + 1, sk[1], sv[1], sk[0], sv[0]);
   }
 
+  if constexpr (KS == 2) {  // the group's second wave adds to the first
+    static_assert(sizeof(sk) >= kGroups * DB * sizeof(AccLds), "a group's partials fit");
+    AccLds* slot = reinterpret_cast<AccLds*>(&sk[0][0]) + grp * DB;
+    if (sub == 1) put_acc(dqacc, slot, lane);
+    __syncthreads();
+    if (sub == 1) return;
+    add_acc(dqacc, slot, lane);
+  }
   if (q0 < S)
     store_rows_staged<D>(sl.row(dq, kTDQ, q0), sl.pitch(kTDQ), S - q0, dqacc, scale,
-                         &sk[0][0] + wave * kQW * D, lane);
+                         &sk[0][0] + (KS == 1 ? wave : grp * 2) * kQW * D, lane);
 }
 
 template <int D>
@@ -542,34 +577,27 @@ hipError_t launch_bwd_bf16_t(bf16* dq, bf16* dk, bf16* dv, float* delta, const b
   // P = exp2(S * scale * log2(e) - lse * log2(e)) holds for either sign of the scale.
   const float sl2 = scale * kLog2e;
   if (phases & kBwdDq) {
-    constexpr int QB = kQW * kWaves;
-    const dim3 grid(BH, (S + QB - 1) / QB);
-    if (drop != nullptr)
-      dq_bf16_kernel<D, false, true><<<grid, 64 * kWaves, 0, stream>>>(
-          dq, delta, q, k, v, dout, out, lse, S, sl2, scale, L, dr);
-    else if (contiguous)
-      dq_bf16_kernel<D, false, false><<<grid, 64 * kWaves, 0, stream>>>(
-          dq, delta, q, k, v, dout, out, lse, S, sl2, scale, L, dr);
-    else
-      dq_bf16_kernel<D, true, false><<<grid, 64 * kWaves, 0, stream>>>(
-          dq, delta, q, k, v, dout, out, lse, S, sl2, scale, L, dr);
+    with_shape(waves_per_group(BH, S, D, drop != nullptr), drop != nullptr, !contiguous,
+               [&](auto strided, auto dropped, auto ks) {
+                 constexpr int QB = kQW * kWaves / ks();
+                 const dim3 grid(BH, (S + QB - 1) / QB);
+                 dq_bf16_kernel<D, strided(), dropped(), ks()><<<grid, 64 * kWaves, 0, stream>>>(
+                     dq, delta, q, k, v, dout, out, lse, S, sl2, scale, L, dr);
+               });
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   if (phases & kBwdDkdv) {
-    constexpr int KB = kKW * kWaves;
     // s = S - lse/scale needs a nonzero scale: a zero one (P = exp(-lse)) runs with 1e-30,
     // whose S*scale terms are then below fp32 resolution next to lse/scale.
     const float se = scale != 0.f ? scale : 1e-30f;
-    const dim3 grid(BH, (S + KB - 1) / KB);
-    if (drop != nullptr)
-      dkdv_bf16_kernel<D, false, true><<<grid, 64 * kWaves, 0, stream>>>(
-          dk, dv, q, k, v, dout, lse, delta, S, se * kLog2e, -1.0f / se, scale, L, dr);
-    else if (contiguous)
-      dkdv_bf16_kernel<D, false, false><<<grid, 64 * kWaves, 0, stream>>>(
-          dk, dv, q, k, v, dout, lse, delta, S, se * kLog2e, -1.0f / se, scale, L, dr);
-    else
-      dkdv_bf16_kernel<D, true, false><<<grid, 64 * kWaves, 0, stream>>>(
-          dk, dv, q, k, v, dout, lse, delta, S, se * kLog2e, -1.0f / se, scale, L, dr);
+    with_shape(waves_per_group(BH, S, D, drop != nullptr), drop != nullptr, !contiguous,
+               [&](auto strided, auto dropped, auto ks) {
+                 constexpr int KB = kKW * kWaves / ks();
+                 const dim3 grid(BH, (S + KB - 1) / KB);
+                 dkdv_bf16_kernel<D, strided(), dropped(), ks()>
+                     <<<grid, 64 * kWaves, 0, stream>>>(dk, dv, q, k, v, dout, lse, delta, S,
+                                                        se * kLog2e, -1.0f / se, scale, L, dr);
+               });
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   return e;

@@ -4,7 +4,9 @@
 //
 // Work decomposition: one workgroup = WAVES waves x NQB*32 queries of one (b,h) slice; it
 // walks the 64-key tiles up to its last query (causal tile skipping). Each wave owns NQB
-// 32-query MFMA blocks and handles each key tile as two 32-key chunks. Per chunk and wave, on
+// 32-query MFMA blocks and handles each key tile as two 32-key chunks; on small grids (KS = 2,
+// waves_per_group) a workgroup owns half the queries, two waves share each query block, taking
+// one chunk of every tile each, and their (m, l, O) are merged at the end. Per chunk and wave, on
 // v_mfma_f32_32x32x16_bf16:
 //   S^T[key][query] = K . Q^T   A = K rows from LDS (rows loaded through sigma32), B = Q held
 //                               in registers for the whole kernel; one K operand read feeds
@@ -219,7 +221,7 @@ __device__ __forceinline__ void fwd_softmax_pv(f32x16 (&s)[NQB], f32x16 (&oacc)[
       for (int i = 0; i < NQB; ++i) oacc[i][db] = mfma32(va[db][j], pb[i][j], oacc[i][db]);
 }
 
-template <int D, bool STRIDED, bool DROP>
+template <int D, bool STRIDED, bool DROP, int KS>
 __global__ __launch_bounds__(64 * kWaves, kMinBlocks)
 __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_kernel(
     bf16* __restrict__ out, float* __restrict__ lse, const bf16* __restrict__ q,
@@ -227,7 +229,7 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
     int negate_q, int snake, const AttnLayout L, const DropParams dr) {
   // scale_log2 = |scale| * log2(e); a negative scale is applied by negating Q (exact in bf16),
   // so the row max of the raw scores is the row max of the scaled ones.
-  constexpr int QB = kQW * kWaves;
+  constexpr int kGroups = kWaves / KS, QB = kQW * kGroups;  // query groups, queries
   constexpr int DS = D / 16;  // 16-wide K-steps along D
   constexpr int DB = D / 32;  // 32-row blocks of O^T
   // K and V tiles, double-buffered: tile t is read while t+1 is in flight. With the tile loop
@@ -237,6 +239,8 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
   __shared__ __attribute__((aligned(16))) bf16 sv[2][kTileRows * D];
   __shared__ f32x4 smask[4][64];
   static_assert(kWaves * kQW <= 2 * kTileRows, "the epilogue stages every wave's rows in sk");
+  static_assert(KS == 1 || sizeof(sk) >= kGroups * (D / 32) * sizeof(AccLds),
+                "the second waves' partials fit sk");
 
   // Dispatch order: longest (latest) query blocks first, (b,h) fastest. With `snake` > 0 (a grid
   // that fits on the CUs in one round) every other group of `snake` workgroups in dispatch
@@ -255,13 +259,14 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar
   const int l32 = lane & 31, hi = lane >> 5;
+  const int grp = wave % kGroups, sub = wave / kGroups;
   const Slice<D, STRIDED> sl(L, bh, S);
   const bf16* qg = sl.base(q, kTQ);
   const bf16* kg = sl.base(k, kTK);
   const bf16* vg = sl.base(v, kTV);
   const int qp = sl.pitch(kTQ), kp = sl.pitch(kTK), vp = sl.pitch(kTV);  // row pitches
 
-  const int q0 = qblk * QB + wave * kQW;
+  const int q0 = qblk * QB + grp * kQW;
   const int wg_last = min(S, (qblk + 1) * QB) - 1;
   const int n_tiles = wg_last / kTileRows + 1;
 
@@ -319,16 +324,16 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
       // One 32-key chunk at a time (holding both chunks' scores at once measured no faster
       // and costs registers); the other waves on the SIMD cover the operand reads' latency.
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const int c0 = k0 + 32 * kb;
+      for (int i = 0; i < 2 / KS; ++i) {
+        const int kb = KS == 1 ? i : sub, c0 = k0 + 32 * kb;
         if (c0 > q0 + kQW - 1) break;  // every key of the chunk after every query
         bf16x8 ka[DS], va[DB][2];
         f32x16 sc[kNQB];
         KeepWords16 keep[kNQB] = {};
         if constexpr (DROP) {
 #pragma unroll
-          for (int i = 0; i < kNQB; ++i)
-            keep[i] = keep_words16(dr, (uint64_t)bh * S + q0 + 32 * i + l32, c0, hi);
+          for (int n = 0; n < kNQB; ++n)
+            keep[n] = keep_words16(dr, (uint64_t)bh * S + q0 + 32 * n + l32, c0, hi);
         }
         fwd_k_ops<D>(ka, ck, kb, lane);
         // the chunk whose first key is the wave's first query is the one to mask
@@ -350,6 +355,27 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
     if (t + 1 < n_tiles) tile(t + 1, sk[1], sv[1], sk[0], sv[0]);
   }
 
+  if constexpr (KS == 2) {
+    // (m, l, O) of the group's second wave: rescaled to the larger maximum and added. A wave
+    // that saw no chunk of the row has m = -inf and zeros, which get weight 2^-inf = 0.
+    AccLds* slot = reinterpret_cast<AccLds*>(&sk[0][0]) + grp * DB;
+    float* ml = reinterpret_cast<float*>(&smask[0][0]) + grp * 128;
+    if (sub == 1) {
+      put_acc(oacc[0], slot, lane);
+      ml[lane] = mrun[0];
+      ml[64 + lane] = lrun[0];
+    }
+    __syncthreads();
+    if (sub == 1) return;
+    const float m1 = ml[lane], mn = fmaxf(mrun[0], m1);
+    const float a0 = fast_exp2(mrun[0] - mn), a1 = fast_exp2(m1 - mn);
+    mrun[0] = mn;
+    lrun[0] = lrun[0] * a0 + ml[64 + lane] * a1;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) oacc[0][db] *= a0;
+    add_acc(oacc[0], slot, lane, a1);
+  }
+
   // ---- epilogue: O = O^T / l, lse = ln2 * (m + log2 l) ----
 #pragma unroll
   for (int i = 0; i < kNQB; ++i) {
@@ -359,7 +385,7 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
     // the tiles are free after the last barrier: each wave stages its rows in its quarter of sk
     if (q0 + 32 * i < S)
       store_rows_staged<D>(sl.row(out, kTO, q0 + 32 * i), sl.pitch(kTO), S - q0 - 32 * i,
-                           oacc[i], inv, &sk[0][0] + (wave * kNQB + i) * 32 * D, lane);
+                           oacc[i], inv, &sk[0][0] + (KS == 1 ? wave : grp * 2) * 32 * D * kNQB + i * 32 * D, lane);
     if (qrow < S && hi == 0) lse[(size_t)bh * S + qrow] = (mrun[i] + __log2f(l)) * kLn2;
   }
 }
@@ -368,29 +394,25 @@ template <int D>
 hipError_t launch_fwd_bf16_t(bf16* out, float* lse, const bf16* q, const bf16* k, const bf16* v,
                              int BH, int S, float scale, const AttnLayout& L,
                              const Dropout* drop, hipStream_t stream) {
-  constexpr int QB = kQW * kWaves;
-  dim3 grid(BH, (S + QB - 1) / QB);
-  // Snake order only for grids of at most kMinBlocks workgroups per CU (all resident at once,
-  // the dispatcher dealing each CU the same number): measured 2% faster at B8 H12 T1024 (768
-  // workgroups, 3 per CU) and 6% slower at B16 (1,536).
   const int cus = device_cus();
-  const int snake =
-      cus > 0 && (long long)grid.x * grid.y <= (long long)cus * kMinBlocks ? cus : 0;
   // Masked scores are -inf and exponentiate as exp2(-inf * c - m), so c must be positive: a
   // zero scale (uniform attention) runs with c = 1e-30: every score below 1e22 in magnitude
   // then has |s*c - m| < 2^-25, an fp32 weight of exactly 1.
   const float c = fmaxf(fabsf(scale) * kLog2e, 1e-30f);
   const DropParams dr = drop_params(drop);
-  if (drop != nullptr) {  // contiguous layout only (checked by the caller)
-    fwd_bf16_kernel<D, false, true><<<grid, 64 * kWaves, 0, stream>>>(out, lse, q, k, v, S, c,
-                                                                      scale < 0.f, snake, L, dr);
-  } else if (is_contiguous(L, S, D)) {
-    fwd_bf16_kernel<D, false, false><<<grid, 64 * kWaves, 0, stream>>>(out, lse, q, k, v, S, c,
-                                                                       scale < 0.f, snake, L, dr);
-  } else {
-    fwd_bf16_kernel<D, true, false><<<grid, 64 * kWaves, 0, stream>>>(out, lse, q, k, v, S, c,
-                                                                      scale < 0.f, snake, L, dr);
-  }
+  auto launch = [&](auto strided, auto dropped, auto ks) {
+    constexpr int QB = kQW * kWaves / ks();
+    const dim3 grid(BH, (S + QB - 1) / QB);
+    // Snake order only for grids of at most kMinBlocks workgroups per CU (all resident at once,
+    // the dispatcher dealing each CU the same number): measured 2% faster at B8 H12 T1024 (768
+    // workgroups, 3 per CU) and 6% slower at B16 (1,536).
+    const int snake =
+        cus > 0 && (long long)grid.x * grid.y <= (long long)cus * kMinBlocks ? cus : 0;
+    fwd_bf16_kernel<D, strided(), dropped(), ks()><<<grid, 64 * kWaves, 0, stream>>>(
+        out, lse, q, k, v, S, c, scale < 0.f, snake, L, dr);
+  };
+  // dropout: contiguous layout only (checked by the caller)
+  with_shape(waves_per_group(BH, S, D, drop != nullptr), drop != nullptr, !is_contiguous(L, S, D), launch);
   return hipGetLastError();
 }
 

@@ -57,6 +57,38 @@ struct Dropout {
 // Compute units of the current device (cached per device; 0 if unknown).
 int device_cus();
 
+// Waves per 32-row group in the bf16 kernels. A workgroup is four waves over 64-row tiles: with
+// one wave per group it owns 128 rows (queries, or keys in dK/dV), each wave taking both
+// 32-row chunks of a tile; with two it owns 64, two waves taking one chunk of each tile and
+// merging at the end. Two make the chain of the longest workgroup half as long and its stream
+// twice as expensive per row, so they pay where a grid is so small that it lasts as long as that
+// chain, and cost 5-15% where the CUs are full anyway. Measured, one wave -> two, forward /
+// backward us (BH x S, D = 64): 48 x 1024 17.4 -> 14.0 / 48 -> 38.6, 64 x 1024 18.2 -> 17.9 /
+// 54.0 -> 54.4, 72 x 1024 19.2 -> 19.8 / 56 -> 59; 24 x 2048 29 -> 22.5 / 84 -> 66, 36 x 2048
+// 32.2 -> 32.2 / 96 -> 95; 12 x 4096 53 -> 40 / 157 -> 120; 128 x 512 11.2 -> 11.0 / 32 -> 38;
+// 96 x 384 9.3 -> 8.5 / 24.2 -> 22.5, 128 x 320 8.3 -> 7.8 / 21.7 -> 21.2, hence the line at two
+// 128-row workgroups per CU, one more per head counted. Short sequences (S <= 256, at most two
+// tiles' worth of chain to save) need one 64-row workgroup per CU: 128 x 128 5.5 -> 5.2 /
+// 13.2 -> 11.7, 192 x 128 5.6 -> 5.7 / 13.5 -> 13.8; one tile (S <= 64) has nothing to share. At
+// D = 32, where half the registers leave more workgroups resident, and with dropout, whose
+// generator lengthens the chain, the line lies further out: D = 32 72 x 1024 14.4 -> 12.8 /
+// 37 -> 32, 96 x 1024 14.4 -> 14.6 / 39.3 -> 38.3; dropout 96 x 1024 32 -> 31 / 99 -> 92,
+// 128 x 1024 35.3 -> 37.5 / 110 -> 115, 128 x 512 14.6 -> 14.6 / 41.1 -> 42.7.
+inline int waves_per_group(int BH, int S, int D, bool drop) {
+  if (S <= 64) return 1;
+  const long long cus = device_cus(), wgs = (long long)BH * ((S + 127) / 128 + 1);
+  bool two;
+  if (D == 32)
+    two = wgs <= 3 * cus;
+  else if (S <= 256)
+    two = (long long)BH * ((S + 63) / 64) <= cus;
+  else if (drop && S > 512)
+    two = 2 * wgs <= 7 * cus;
+  else
+    two = wgs <= 2 * cus;
+  return two ? 2 : 1;
+}
+
 // Causal flash forward, bf16 in/out, fp32 logsumexp (natural log) [BH, S]. q, k, v, out as
 // `layout` places them (tensors kTQ, kTK, kTV, kTO), D in {32,64}. With `drop`, the
 // probabilities multiplying V are dropped (the logsumexp is that of the undropped scores).

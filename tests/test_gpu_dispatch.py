@@ -58,3 +58,51 @@ F32_SHAPES = [(3, 96, 64), (3, 97, 64), (2, 129, 64), (5, 160, 32), (1, 500, 64)
 def test_f32_shapes(gpu, BH, S, D):
     """The fp32 kernels' bounds (1e-5) hold against float64 whatever the split."""
     _check(BH, S, D, torch.float32, (1e-5,) * 5)
+
+
+# One or two waves per row group in the bf16 kernels: one tile and two (S 64, 65), the short rule
+# (S 128, 256) and the long one (S 257, 800, 1000) on both sides of their lines at 256 CUs, tiles
+# that end inside a chunk, and more heads than a round of workgroups.
+BF16_SHAPES = [(1, 64, 64), (1, 65, 64), (3, 95, 64), (2, 97, 32), (128, 128, 64), (129, 128, 64),
+               (64, 256, 64), (65, 250, 64), (128, 257, 64), (129, 330, 64), (64, 800, 64),
+               (74, 790, 64), (24, 2047, 64), (384, 100, 32), (385, 70, 32), (96, 800, 32),
+               (110, 800, 32)]
+BF16_TOLS = (2e-2, 1e-3, 5e-2, 5e-2, 5e-2)
+
+
+@pytest.mark.parametrize("BH,S,D", BF16_SHAPES)
+def test_bf16_shapes(gpu, BH, S, D):
+    """The bf16 kernels' bounds against float64 (of the same bf16 inputs) whatever the split."""
+    _check(BH, S, D, torch.bfloat16, BF16_TOLS)
+
+
+@pytest.mark.parametrize("BH,S", [(2, 70), (5, 300), (99, 520), (150, 520)])
+def test_bf16_dropout_and_strided_shapes(gpu, BH, S):
+    """The dropout instantiations at p = 0 give the plain results, and the strided ones the
+    contiguous ones', on both sides of the lines that differ between them: to the rounding of
+    another summation order, 2^-8 of the values' scale (outputs and gradients below 8)."""
+    print(f"[case] dropout / strided BH={BH} S={S}", flush=True)
+    D, tol = 64, 8 * 2.0 ** -8
+    q, k, v, dout = _inputs(BH, S, D, torch.bfloat16, S)
+    scale = A.default_scale(D)
+    out, lse = A.attention_forward(q, k, v, scale)
+    want = (out, lse) + A.attention_backward(dout, out, lse, q, k, v, scale)[:3]
+
+    def close(got):
+        for x, y in zip(got, want):
+            assert (x.float() - y.float()).abs().max().item() <= tol
+
+    o2, l2, delta = torch.empty_like(out), torch.empty_like(lse), torch.empty_like(lse)
+    A.flash_attention_forward_bf16_dropout(o2, l2, q, k, v, BH, S, D, scale, 0.0, 5)
+    grads = [torch.empty_like(q) for _ in range(3)]
+    A.flash_attention_backward_bf16_dropout(*grads, delta, dout, o2, l2, q, k, v, BH, S, D, scale,
+                                            0.0, 5)
+    close((o2, l2, *grads))
+    tokens = [x.view(1, BH, S, D).transpose(1, 2).contiguous().transpose(1, 2)
+              for x in (q, k, v, dout)]
+    o3 = torch.empty_like(tokens[0])
+    l3 = torch.empty_like(lse)
+    A.flash_attention_forward_bf16_strided(o3, l3, *tokens[:3], scale)
+    g3 = [torch.empty_like(tokens[0]) for _ in range(3)]
+    A.flash_attention_backward_bf16_strided(*g3, delta, tokens[3], o3, l3, *tokens[:3], scale)
+    close((o3.reshape(BH, S, D), l3, *[x.reshape(BH, S, D) for x in g3]))
