@@ -176,8 +176,17 @@ def _ptr(t) -> int | None:
     return t.data_ptr()
 
 
+# The current stream's handle without the Stream object that torch.cuda.current_stream() makes
+# (0.2 us a call against 2.8), where torch has the accessors.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream_ptr(stream) -> int | None:
     if stream is None:
+        if _raw_stream is not None and _current_device is not None \
+                and torch.cuda.is_initialized():
+            return _raw_stream(_current_device()) or None
         stream = torch.cuda.current_stream()
     return stream.cuda_stream or None
 
@@ -197,6 +206,37 @@ def _require(t, name, dtype, numel, device=None):
         raise ValueError(f"{name} has {t.numel()} elements, needs {numel}")
 
 
+def _ptrs(dtype, numel, tensors, names) -> list:
+    """Device addresses of `tensors`, each held to _require (None passes as None). The checks of
+    plain tensors run here on their own; whatever fails one, subclasses included, goes to
+    _require for its verdict."""
+    ptrs = []
+    for t, name in zip(tensors, names):
+        if not (type(t) is torch.Tensor and t.dtype is dtype and t.is_cuda and t.is_contiguous()
+                and t.numel() >= numel):
+            _require(t, name, dtype, numel)
+        ptrs.append(None if t is None else t.data_ptr())
+    return ptrs
+
+
+_FWD_NAMES = ("out", "q", "k", "v")
+_BWD_NAMES = ("dq", "dk", "dv", "dout", "out", "q", "k", "v")
+
+
+def _forward_ptrs(dtype, out, lse, q, k, v, BH, S, d_head):
+    """The checked addresses of a contiguous forward, in the C ABI's order."""
+    o, pq, pk, pv = _ptrs(dtype, BH * S * d_head, (out, q, k, v), _FWD_NAMES)
+    return (o, *_ptrs(torch.float32, BH * S, (lse,), ("lse",)), pq, pk, pv)
+
+
+def _backward_ptrs(dtype, dq, dk, dv, delta, dout, out, lse, q, k, v, BH, S, d_head):
+    """The checked addresses of a contiguous backward, in the C ABI's order."""
+    gq, gk, gv, do, o, pq, pk, pv = _ptrs(dtype, BH * S * d_head,
+                                          (dq, dk, dv, dout, out, q, k, v), _BWD_NAMES)
+    dl, ls = _ptrs(torch.float32, BH * S, (delta, lse), ("delta", "lse"))
+    return (gq, gk, gv, dl, do, o, ls, pq, pk, pv)
+
+
 # --------------------------------------------------------------- reference-named wrappers
 
 def flash_attention_supported(d_head: int) -> bool:
@@ -207,80 +247,51 @@ def flash_attention_supported(d_head: int) -> bool:
 def flash_attention_forward(out, lse, q, k, v, BH: int, S: int, d_head: int, scale: float,
                             stream=None) -> None:
     """gpu_flash_attention_forward (cuda/gpu_ops.cuh:116-117). fp32 buffers, overwritten."""
-    n = BH * S * d_head
-    for t, nm in ((out, "out"), (q, "q"), (k, "k"), (v, "v")):
-        _require(t, nm, torch.float32, n)
-    _require(lse, "lse", torch.float32, BH * S)
+    ptrs = _forward_ptrs(torch.float32, out, lse, q, k, v, BH, S, d_head)
     _check(lib().dadgpt_flash_attention_forward_async(
-        _ptr(out), _ptr(lse), _ptr(q), _ptr(k), _ptr(v), BH, S, d_head, scale,
-        _stream_ptr(stream)))
+        *ptrs, BH, S, d_head, scale, _stream_ptr(stream)))
 
 
 def flash_attention_backward(dq, dk, dv, delta, dout, out, lse, q, k, v, BH: int, S: int,
                              d_head: int, scale: float, stream=None) -> None:
     """gpu_flash_attention_backward (cuda/gpu_ops.cuh:119-122). Writes dq, dk, dv and the
     delta scratch."""
-    n = BH * S * d_head
-    for t, nm in ((dq, "dq"), (dk, "dk"), (dv, "dv"), (dout, "dout"), (out, "out"),
-                  (q, "q"), (k, "k"), (v, "v")):
-        _require(t, nm, torch.float32, n)
-    _require(delta, "delta", torch.float32, BH * S)
-    _require(lse, "lse", torch.float32, BH * S)
+    ptrs = _backward_ptrs(torch.float32, dq, dk, dv, delta, dout, out, lse, q, k, v, BH, S, d_head)
     _check(lib().dadgpt_flash_attention_backward_async(
-        _ptr(dq), _ptr(dk), _ptr(dv), _ptr(delta), _ptr(dout), _ptr(out), _ptr(lse), _ptr(q),
-        _ptr(k), _ptr(v), BH, S, d_head, scale, _stream_ptr(stream)))
+        *ptrs, BH, S, d_head, scale, _stream_ptr(stream)))
 
 
 def flash_attention_forward_bf16(out, lse, q, k, v, BH: int, S: int, d_head: int,
                                  scale: float, stream=None) -> None:
-    n = BH * S * d_head
-    for t, nm in ((out, "out"), (q, "q"), (k, "k"), (v, "v")):
-        _require(t, nm, torch.bfloat16, n)
-    _require(lse, "lse", torch.float32, BH * S)
+    ptrs = _forward_ptrs(torch.bfloat16, out, lse, q, k, v, BH, S, d_head)
     _check(lib().dadgpt_flash_attention_forward_bf16(
-        _ptr(out), _ptr(lse), _ptr(q), _ptr(k), _ptr(v), BH, S, d_head, scale,
-        _stream_ptr(stream)))
+        *ptrs, BH, S, d_head, scale, _stream_ptr(stream)))
 
 
 def flash_attention_backward_bf16(dq, dk, dv, delta, dout, out, lse, q, k, v, BH: int, S: int,
                                   d_head: int, scale: float, stream=None) -> None:
-    n = BH * S * d_head
-    for t, nm in ((dq, "dq"), (dk, "dk"), (dv, "dv"), (dout, "dout"), (out, "out"),
-                  (q, "q"), (k, "k"), (v, "v")):
-        _require(t, nm, torch.bfloat16, n)
-    _require(delta, "delta", torch.float32, BH * S)
-    _require(lse, "lse", torch.float32, BH * S)
+    ptrs = _backward_ptrs(torch.bfloat16, dq, dk, dv, delta, dout, out, lse, q, k, v, BH, S,
+                          d_head)
     _check(lib().dadgpt_flash_attention_backward_bf16(
-        _ptr(dq), _ptr(dk), _ptr(dv), _ptr(delta), _ptr(dout), _ptr(out), _ptr(lse), _ptr(q),
-        _ptr(k), _ptr(v), BH, S, d_head, scale, _stream_ptr(stream)))
+        *ptrs, BH, S, d_head, scale, _stream_ptr(stream)))
 
 
 def flash_attention_forward_dropout(out, lse, q, k, v, BH: int, S: int, d_head: int,
                                     scale: float, dropout_p: float, seed: int,
                                     stream=None) -> None:
     """fp32 forward with attention-probability dropout (the reference's precision)."""
-    n = BH * S * d_head
-    for t, nm in ((out, "out"), (q, "q"), (k, "k"), (v, "v")):
-        _require(t, nm, torch.float32, n)
-    _require(lse, "lse", torch.float32, BH * S)
+    ptrs = _forward_ptrs(torch.float32, out, lse, q, k, v, BH, S, d_head)
     _check(lib().dadgpt_flash_attention_forward_dropout(
-        _ptr(out), _ptr(lse), _ptr(q), _ptr(k), _ptr(v), BH, S, d_head, scale, dropout_p,
-        seed & 0xFFFFFFFFFFFFFFFF, _stream_ptr(stream)))
+        *ptrs, BH, S, d_head, scale, dropout_p, seed & 0xFFFFFFFFFFFFFFFF, _stream_ptr(stream)))
 
 
 def flash_attention_backward_dropout(dq, dk, dv, delta, dout, out, lse, q, k, v, BH: int,
                                      S: int, d_head: int, scale: float, dropout_p: float,
                                      seed: int, stream=None) -> None:
     """fp32 backward of flash_attention_forward_dropout with the same (dropout_p, seed)."""
-    n = BH * S * d_head
-    for t, nm in ((dq, "dq"), (dk, "dk"), (dv, "dv"), (dout, "dout"), (out, "out"),
-                  (q, "q"), (k, "k"), (v, "v")):
-        _require(t, nm, torch.float32, n)
-    _require(delta, "delta", torch.float32, BH * S)
-    _require(lse, "lse", torch.float32, BH * S)
+    ptrs = _backward_ptrs(torch.float32, dq, dk, dv, delta, dout, out, lse, q, k, v, BH, S, d_head)
     _check(lib().dadgpt_flash_attention_backward_dropout(
-        _ptr(dq), _ptr(dk), _ptr(dv), _ptr(delta), _ptr(dout), _ptr(out), _ptr(lse), _ptr(q),
-        _ptr(k), _ptr(v), BH, S, d_head, scale, dropout_p, seed & 0xFFFFFFFFFFFFFFFF,
+        *ptrs, BH, S, d_head, scale, dropout_p, seed & 0xFFFFFFFFFFFFFFFF,
         _stream_ptr(stream)))
 
 
@@ -289,28 +300,19 @@ def flash_attention_forward_bf16_dropout(out, lse, q, k, v, BH: int, S: int, d_h
                                          stream=None) -> None:
     """bf16 forward with attention-probability dropout (the reference's materialized path
     with dropout, src/model.cpp:406-416, fused); the mask is a function of (seed, position)."""
-    n = BH * S * d_head
-    for t, nm in ((out, "out"), (q, "q"), (k, "k"), (v, "v")):
-        _require(t, nm, torch.bfloat16, n)
-    _require(lse, "lse", torch.float32, BH * S)
+    ptrs = _forward_ptrs(torch.bfloat16, out, lse, q, k, v, BH, S, d_head)
     _check(lib().dadgpt_flash_attention_forward_bf16_dropout(
-        _ptr(out), _ptr(lse), _ptr(q), _ptr(k), _ptr(v), BH, S, d_head, scale, dropout_p,
-        seed & 0xFFFFFFFFFFFFFFFF, _stream_ptr(stream)))
+        *ptrs, BH, S, d_head, scale, dropout_p, seed & 0xFFFFFFFFFFFFFFFF, _stream_ptr(stream)))
 
 
 def flash_attention_backward_bf16_dropout(dq, dk, dv, delta, dout, out, lse, q, k, v, BH: int,
                                           S: int, d_head: int, scale: float, dropout_p: float,
                                           seed: int, stream=None) -> None:
     """The backward of flash_attention_forward_bf16_dropout with the same (dropout_p, seed)."""
-    n = BH * S * d_head
-    for t, nm in ((dq, "dq"), (dk, "dk"), (dv, "dv"), (dout, "dout"), (out, "out"),
-                  (q, "q"), (k, "k"), (v, "v")):
-        _require(t, nm, torch.bfloat16, n)
-    _require(delta, "delta", torch.float32, BH * S)
-    _require(lse, "lse", torch.float32, BH * S)
+    ptrs = _backward_ptrs(torch.bfloat16, dq, dk, dv, delta, dout, out, lse, q, k, v, BH, S,
+                          d_head)
     _check(lib().dadgpt_flash_attention_backward_bf16_dropout(
-        _ptr(dq), _ptr(dk), _ptr(dv), _ptr(delta), _ptr(dout), _ptr(out), _ptr(lse), _ptr(q),
-        _ptr(k), _ptr(v), BH, S, d_head, scale, dropout_p, seed & 0xFFFFFFFFFFFFFFFF,
+        *ptrs, BH, S, d_head, scale, dropout_p, seed & 0xFFFFFFFFFFFFFFFF,
         _stream_ptr(stream)))
 
 
@@ -326,23 +328,28 @@ def flash_attention_backward_bf16_phase(phase: int, dq, dk, dv, delta, dout, out
 # ------------------------------------------------ strided layouts (no split/merge passes)
 
 def _head_view(t, name, shape=None):
-    """A bf16 device view [B, H, S, d_head] whose rows are contiguous -> its strides."""
+    """A bf16 device view [B, H, S, d_head] whose rows are contiguous -> its strides (batch,
+    head, row)."""
     if not isinstance(t, torch.Tensor) or not t.is_cuda or t.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be a bfloat16 device tensor")
-    if t.dim() != 4 or t.stride(3) != 1:
+    strides = t.stride()
+    if len(strides) != 4 or strides[3] != 1:
         raise ValueError(f"{name} must be a [B, H, S, d_head] view with contiguous rows")
-    if shape is not None and tuple(t.shape) != tuple(shape):
+    if shape is not None and t.shape != shape:
         raise ValueError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
-    return HeadStrides(t.stride(0), t.stride(1), t.stride(2))
+    return strides[:3]
+
+
+_Strides4, _Strides8 = HeadStrides * 4, HeadStrides * 8
 
 
 def flash_attention_forward_bf16_strided(out, lse, q, k, v, scale: float, stream=None) -> None:
     """Forward over [B, H, S, d_head] views of any row placement (e.g. heads sliced out of
     the token-major projection output, or a KV cache's first S rows); lse [B*H, S] fp32.
     Replaces split_heads + flash forward + merge_heads (src/model.cpp:384-392,423-424)."""
-    B, H, S, D = q.shape
-    st = (HeadStrides * 4)(*[_head_view(t, nm, (B, H, S, D))
-                             for t, nm in ((q, "q"), (k, "k"), (v, "v"), (out, "out"))])
+    shape = B, H, S, D = q.shape
+    st = _Strides4(_head_view(q, "q", shape), _head_view(k, "k", shape),
+                   _head_view(v, "v", shape), _head_view(out, "out", shape))
     _require(lse, "lse", torch.float32, B * H * S)
     _check(lib().dadgpt_flash_attention_forward_bf16_strided(
         _ptr(out), _ptr(lse), _ptr(q), _ptr(k), _ptr(v), B, H, S, D, scale, st,
@@ -353,10 +360,11 @@ def flash_attention_backward_bf16_strided(dq, dk, dv, delta, dout, out, lse, q, 
                                           scale: float, stream=None) -> None:
     """Backward over [B, H, S, d_head] views (see flash_attention_forward_bf16_strided);
     replaces split_heads + flash backward + 3 merge_heads (src/model.cpp:564-576,619-624)."""
-    B, H, S, D = q.shape
-    views = ((q, "q"), (k, "k"), (v, "v"), (out, "out"), (dout, "dout"), (dq, "dq"),
-             (dk, "dk"), (dv, "dv"))
-    st = (HeadStrides * 8)(*[_head_view(t, nm, (B, H, S, D)) for t, nm in views])
+    shape = B, H, S, D = q.shape
+    st = _Strides8(_head_view(q, "q", shape), _head_view(k, "k", shape),
+                   _head_view(v, "v", shape), _head_view(out, "out", shape),
+                   _head_view(dout, "dout", shape), _head_view(dq, "dq", shape),
+                   _head_view(dk, "dk", shape), _head_view(dv, "dv", shape))
     _require(delta, "delta", torch.float32, B * H * S)
     _require(lse, "lse", torch.float32, B * H * S)
     _check(lib().dadgpt_flash_attention_backward_bf16_strided(
@@ -408,18 +416,17 @@ def decode_attention(out, q, k_cache, v_cache, lens, n_seq, n_heads, max_len, d_
     dt = q.dtype
     if dt not in (torch.bfloat16, torch.float32):
         raise TypeError("decode_attention: q must be bfloat16 or float32")
-    _require(q, "q", dt, n_seq * n_heads * d_head)
-    _require(out, "out", dt, n_seq * n_heads * d_head)
-    _require(k_cache, "k_cache", dt, n_seq * n_heads * max_len * d_head)
-    _require(v_cache, "v_cache", dt, n_seq * n_heads * max_len * d_head)
-    _require(lens, "lens", torch.int32, n_seq)
+    rows = n_seq * n_heads
+    pq, po = _ptrs(dt, rows * d_head, (q, out), ("q", "out"))
+    pk, pv = _ptrs(dt, rows * max_len * d_head, (k_cache, v_cache), ("k_cache", "v_cache"))
+    pl, = _ptrs(torch.int32, n_seq, (lens,), ("lens",))
     if workspace is not None and (not workspace.is_cuda or not workspace.is_contiguous()):
         raise ValueError("workspace must be a contiguous device tensor")
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     fn = (lib().dadgpt_decode_attention_bf16 if dt == torch.bfloat16
           else lib().dadgpt_decode_attention_f32)
-    _check(fn(_ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(lens), n_seq, n_heads,
-              max_len, d_head, scale, _ptr(workspace), ws_bytes, _stream_ptr(stream)))
+    _check(fn(po, pq, pk, pv, pl, n_seq, n_heads, max_len, d_head, scale, _ptr(workspace),
+              ws_bytes, _stream_ptr(stream)))
 
 
 # --------------------------------------------------------------- allocating conveniences
@@ -435,14 +442,12 @@ def decode_attention_noalloc(out, q, k_cache, v_cache, lens, n_seq, n_heads, max
     (DECODE_NOALLOC_SCRATCH_BYTES) holds the split-cache partials, so the call allocates
     nothing. Calls that overlap in time on one device race on that scratch."""
     dt = torch.bfloat16
-    _require(q, "q", dt, n_seq * n_heads * d_head)
-    _require(out, "out", dt, n_seq * n_heads * d_head)
-    _require(k_cache, "k_cache", dt, n_seq * n_heads * max_len * d_head)
-    _require(v_cache, "v_cache", dt, n_seq * n_heads * max_len * d_head)
-    _require(lens, "lens", torch.int32, n_seq)
+    rows = n_seq * n_heads
+    pq, po = _ptrs(dt, rows * d_head, (q, out), ("q", "out"))
+    pk, pv = _ptrs(dt, rows * max_len * d_head, (k_cache, v_cache), ("k_cache", "v_cache"))
+    pl, = _ptrs(torch.int32, n_seq, (lens,), ("lens",))
     _check(lib().dadgpt_decode_attention_bf16_noalloc(
-        _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(lens), n_seq, n_heads, max_len,
-        d_head, scale, _stream_ptr(stream)))
+        po, pq, pk, pv, pl, n_seq, n_heads, max_len, d_head, scale, _stream_ptr(stream)))
 
 
 # ---------------------------------------------------------------- materialized attention

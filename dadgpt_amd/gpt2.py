@@ -145,7 +145,7 @@ def _check(status: int) -> None:
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_attn._stream_ptr(None))
 
 
 # ------------------------------------------------------------------------------ GEMMs
