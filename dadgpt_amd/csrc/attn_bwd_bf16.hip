@@ -9,8 +9,9 @@
 //   dK/dV kernel   key-major; per 32-query block:  S = Q K^T, dP = dO V^T,
 //                  P = exp(S*scale - lse), dS = P (dP - delta),
 //                  dV^T += dO^T P, dK^T += Q^T dS                    (attention.cu:87-152)
-//   delta kernel   delta as a pass of its own (profiling and the phase API)
+//   delta kernel   delta as a pass of its own (the phase API; long rows on small grids)
 //
+// Small and medium grids run both in one launch (bwd_plan): dK/dV workgroups first, then dQ ones.
 // Both MFMA kernels own their outputs outright (no atomics, bitwise repeatable). The score
 // tiles use the same sigma32 row permutation as the forward so that P and dS feed the next
 // MFMA as B operands from registers; the operands that must be read along the score dimension
@@ -233,35 +234,87 @@ __device__ __forceinline__ void dkdv_block(bool mask, f32x16 (&dkacc)[D / 32],
   }
 }
 
-template <int D, bool STRIDED, bool DROP, int KS>
-__global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocksNoDrop) void dkdv_bf16_kernel(
-    bf16* __restrict__ dk, bf16* __restrict__ dv, const bf16* __restrict__ q,
-    const bf16* __restrict__ k, const bf16* __restrict__ v, const bf16* __restrict__ dout,
-    const float* __restrict__ lse, const float* __restrict__ delta, int S, float c,
-    float lse_mul, float dk_mul, const AttnLayout L, const DropParams dr) {
+// What a backward kernel works on.
+struct BwdArgs {
+  bf16 *dq, *dk, *dv;
+  float* delta;
+  const bf16 *q, *k, *v, *dout, *out;
+  const float* lse;
+  int S;
+  float scale, scale_log2;      // dQ: the scale, and times log2(e)
+  float c, lse_mul;             // dK/dV: nonzero scale times log2(e), and -1/scale
+  AttnLayout L;
+  DropParams dr;
+};
+
+// LDS of a workgroup: two streamed tiles (Q and dO, or K and V), double-buffered (constant
+// buffer indices in the unrolled loop; see the forward kernel).
+template <int D>
+struct BwdTiles {
+  __attribute__((aligned(16))) bf16 a[2][kTileRows * D];
+  __attribute__((aligned(16))) bf16 b[2][kTileRows * D];
+};
+// dK/dV: per wave and buffer the tile's lse and delta rows, converted in place to -lse/scale and
+// -delta: each wave loads and converts its own copy, so the conversion needs no barrier.
+struct BwdStats {
+  __attribute__((aligned(16))) float row[kWaves][2][2][kTileRows];
+};
+
+// delta of rows row0 .. S-1 into LDS, for a dK/dV workgroup that runs beside the dQ ones
+// instead of after them (the order of the sum differs from dQ's): 16 bytes of a row per lane,
+// four groups of rows in flight.
+template <int D, bool STRIDED>
+__device__ __forceinline__ void delta_rows(float* delta, const Slice<D, STRIDED>& sl,
+                                           const bf16* dout, const bf16* out, int row0, int S) {
+  constexpr int LPR = D / 8, ROWS = 64 * kWaves / LPR, N = 4;
+  const int part = threadIdx.x % LPR;
+  for (int r0 = row0 + (int)threadIdx.x / LPR; r0 - (int)threadIdx.x / LPR < S; r0 += N * ROWS) {
+    u32x4 g[N], o[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = min(r0 + i * ROWS, S - 1);
+      g[i] = ld_g128u(sl.row(dout, kTDO, r) + part * 8);
+      o[i] = ld_g128u(sl.row(out, kTO, r) + part * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      float acc = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        acc += bf16_lo(g[i][w]) * bf16_lo(o[i][w]) + bf16_hi(g[i][w]) * bf16_hi(o[i][w]);
+      acc = lanes::group_sum<LPR>(acc);
+      const int r = r0 + i * ROWS;
+      if (part == 0 && r < S) delta[r - row0] = acc;
+    }
+  }
+}
+
+// One workgroup's dK and dV. OWN_DELTA: delta is computed here, into own_delta (one float for
+// each row from the first tile on); otherwise it is read from a.delta.
+template <int D, bool STRIDED, bool DROP, int KS, bool OWN_DELTA>
+__device__ __forceinline__ void dkdv_workgroup(const BwdArgs& a, int bh, int kblk,
+                                               BwdTiles<D>& tiles, BwdStats& stats,
+                                               float* own_delta) {
   constexpr int kGroups = kWaves / KS, KB = kKW * kGroups;  // key groups, keys
   constexpr int DS = D / 16, DB = D / 32;
-  // Q and dO tiles, double-buffered (constant buffer indices in the unrolled loop; see the
-  // forward kernel), and per wave and buffer the tile's lse and delta rows, converted in place
-  // to -lse/scale and -delta: each wave loads and converts its own copy, so the conversion
-  // needs no barrier.
-  __shared__ __attribute__((aligned(16))) bf16 sq[2][kTileRows * D];
-  __shared__ __attribute__((aligned(16))) bf16 sdo[2][kTileRows * D];
-  __shared__ __attribute__((aligned(16))) float sst[kWaves][2][2][kTileRows];
+  auto& sq = tiles.a;
+  auto& sdo = tiles.b;
   static_assert(kWaves * kKW <= 2 * kTileRows, "the epilogue stages every wave's rows in sq");
+  const bf16 *q = a.q, *k = a.k, *v = a.v, *dout = a.dout;
+  bf16 *dk = a.dk, *dv = a.dv;
+  const int S = a.S;
+  const DropParams& dr = a.dr;
 
-  const int bh = blockIdx.x;
-  const int kblk = blockIdx.y;  // key block 0 sees the most query tiles: dispatched first
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
   const int grp = wave % kGroups, sub = wave / kGroups;
-  const Slice<D, STRIDED> sl(L, bh, S);
+  const Slice<D, STRIDED> sl(a.L, bh, S);
   const bf16* qg = sl.base(q, kTQ);
   const bf16* dog = sl.base(dout, kTDO);
   const int qp = sl.pitch(kTQ), dop = sl.pitch(kTDO);  // row pitches of the streamed tiles
-  const float* lseg = lse + (size_t)bh * S;
-  const float* delg = delta + (size_t)bh * S;
+  const float* lseg = a.lse + (size_t)bh * S;
+  const float* delg = a.delta + (size_t)bh * S;
 
   const int kw0 = kblk * KB + grp * kKW;
   const int key = kw0 + l32;
@@ -294,16 +347,18 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
   uint32_t qoff[Dma::PER_WAVE], dooff[Dma::PER_WAVE];
   Dma::offsets(qoff, wave, lane, qp);
   Dma::offsets(dooff, wave, lane, dop);
-  float(*st)[2][kTileRows] = sst[wave];
+  float(*st)[2][kTileRows] = stats.row[wave];
   auto issue = [&](int t, bf16* nq, bf16* ndo, int buf) {
     Dma::template load_any<true>(nq, qg, t * kTileRows, S, qoff, wave, lane, qp);
     Dma::template load_any<true>(ndo, dog, t * kTileRows, S, dooff, wave, lane, dop);
     dma_row64(st[buf][0], lseg, t * kTileRows, S, lane);
-    dma_row64(st[buf][1], delg, t * kTileRows, S, lane);
+    if constexpr (!OWN_DELTA) dma_row64(st[buf][1], delg, t * kTileRows, S, lane);
   };
   // The first tile loads alongside the operands above: one wait covers all of them (the
   // compiler, which does not see the direct loads, then has nothing left to wait for).
   issue(t_first, sq[0], sdo[0], 0);
+  if constexpr (OWN_DELTA)
+    delta_rows<D, STRIDED>(own_delta, sl, dout, a.out, t_first * kTileRows, S);
   wait_vm_lds<0>();
   __builtin_amdgcn_s_barrier();
 
@@ -316,8 +371,9 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
     if (t + 1 < t_end) issue(t + 1, nq, ndo, nb);
     if (kw0 < S && r0 + kTileRows - 1 >= kw0) {
       // -lse/scale and -delta (this wave's copy; its LDS accesses complete in order)
-      st[cb][0][lane] *= lse_mul;
-      st[cb][1][lane] = -st[cb][1][lane];
+      st[cb][0][lane] *= a.lse_mul;
+      st[cb][1][lane] = OWN_DELTA ? -own_delta[min(r0 + lane, S - 1) - t_first * kTileRows]
+                                  : -st[cb][1][lane];
       const bool edge = r0 + kTileRows > S;
 #pragma unroll
       for (int i = 0; i < 2 / KS; ++i) {
@@ -327,7 +383,7 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
         if constexpr (DROP) keep = keep_col16(dr, (uint64_t)bh * S + qlo, kw0, lane);
         // some key after some query, or rows past S: mask
         dkdv_block<D, DROP, XA>(edge || qlo < kw0 + kKW - 1, dkacc, dvacc, kop, vop, cq, cdo,
-                                st[cb][0], st[cb][1], qb, key - r0, S - r0, lane, c, keep,
+                                st[cb][0], st[cb][1], qb, key - r0, S - r0, lane, a.c, keep,
                                 dr.scale, lo);
       }
     }
@@ -343,7 +399,7 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
   if constexpr (KS == 1) {
     // each wave stages its 32 rows in its quarter of sq (dK) and sdo (dV)
     if (kw0 < S) {
-      store_rows_staged<D>(sl.row(dk, kTDK, kw0), sl.pitch(kTDK), S - kw0, dkacc, dk_mul,
+      store_rows_staged<D>(sl.row(dk, kTDK, kw0), sl.pitch(kTDK), S - kw0, dkacc, a.scale,
                            &sq[0][0] + wave * kKW * D, lane);
       store_rows_staged<D>(sl.row(dv, kTDV, kw0), sl.pitch(kTDV), S - kw0, dvacc, 1.0f,
                            &sdo[0][0] + wave * kKW * D, lane);
@@ -362,7 +418,7 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
     if (kw0 >= S) return;
     if (sub == 0) {
       add_acc(dkacc, slot_k, lane);
-      store_rows_staged<D>(sl.row(dk, kTDK, kw0), sl.pitch(kTDK), S - kw0, dkacc, dk_mul,
+      store_rows_staged<D>(sl.row(dk, kTDK, kw0), sl.pitch(kTDK), S - kw0, dkacc, a.scale,
                            reinterpret_cast<bf16*>(slot_k), lane);
     } else {
       add_acc(dvacc, slot_v, lane);
@@ -370,6 +426,15 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
                            reinterpret_cast<bf16*>(slot_v), lane);
     }
   }
+}
+
+template <int D, bool STRIDED, bool DROP, int KS>
+__global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocksNoDrop) void dkdv_bf16_kernel(
+    const BwdArgs a) {
+  __shared__ BwdTiles<D> tiles;
+  __shared__ BwdStats stats;
+  // key block 0 sees the most query tiles: dispatched first
+  dkdv_workgroup<D, STRIDED, DROP, KS, false>(a, blockIdx.x, blockIdx.y, tiles, stats, nullptr);
 }
 
 // ---------------------------------------------------------------- dQ
@@ -443,26 +508,27 @@ __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
 // dQ for one query block per wave; the kernel also computes delta = rowsum(dO * O) of its
 // rows (from the dO operands it holds and one load of O) and writes it for the dK/dV kernel,
 // so the backward needs no separate delta pass.
-template <int D, bool STRIDED, bool DROP, int KS>
-__global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(
-    bf16* __restrict__ dq, float* __restrict__ delta, const bf16* __restrict__ q,
-    const bf16* __restrict__ k, const bf16* __restrict__ v, const bf16* __restrict__ dout,
-    const bf16* __restrict__ out, const float* __restrict__ lse, int S, float scale_log2,
-    float scale, const AttnLayout L, const DropParams dr) {
+template <int D, bool STRIDED, bool DROP, int KS, bool WRITE_DELTA>
+__device__ __forceinline__ void dq_workgroup(const BwdArgs& a, int bh, int qblk,
+                                             BwdTiles<D>& tiles) {
   constexpr int kGroups = kWaves / KS, QB = kQW * kGroups;  // query groups, queries
   constexpr int DS = D / 16, DB = D / 32;
-  // K and V tiles, double-buffered (constant buffer indices; see the forward kernel).
-  __shared__ __attribute__((aligned(16))) bf16 sk[2][kTileRows * D];
-  __shared__ __attribute__((aligned(16))) bf16 sv[2][kTileRows * D];
+  auto& sk = tiles.a;
+  auto& sv = tiles.b;
   static_assert(kWaves * kQW <= 2 * kTileRows, "the epilogue stages every wave's rows in sk");
+  const bf16 *q = a.q, *k = a.k, *v = a.v, *dout = a.dout, *out = a.out;
+  bf16* dq = a.dq;
+  float* delta = a.delta;
+  const float* lse = a.lse;
+  const int S = a.S;
+  const float scale_log2 = a.scale_log2, scale = a.scale;
+  const DropParams& dr = a.dr;
 
-  const int bh = blockIdx.x;
-  const int qblk = gridDim.y - 1 - blockIdx.y;  // longest (latest) query blocks dispatch first
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi = lane >> 5;
   const int grp = wave % kGroups, sub = wave / kGroups;
-  const Slice<D, STRIDED> sl(L, bh, S);
+  const Slice<D, STRIDED> sl(a.L, bh, S);
   const bf16* kg = sl.base(k, kTK);
   const bf16* vg = sl.base(v, kTV);
   const int kp = sl.pitch(kTK), vp = sl.pitch(kTV);  // row pitches of the streamed tiles
@@ -508,13 +574,13 @@ __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) {
     asm volatile("" : "+v"(oop[ds]));
-    const u32x4 a = as_u32x4(doop[ds]), o = as_u32x4(oop[ds]);
+    const u32x4 g = as_u32x4(doop[ds]), o = as_u32x4(oop[ds]);
 #pragma unroll
     for (int w = 0; w < 4; ++w)
-      dpart += bf16_lo(a[w]) * bf16_lo(o[w]) + bf16_hi(a[w]) * bf16_hi(o[w]);
+      dpart += bf16_lo(g[w]) * bf16_lo(o[w]) + bf16_hi(g[w]) * bf16_hi(o[w]);
   }
   const float dlt = sum_halves(dpart);
-  if (hi == 0 && qrow < S && sub == 0) delta[(size_t)bh * S + qrow] = dlt;
+  if (WRITE_DELTA && hi == 0 && qrow < S && sub == 0) delta[(size_t)bh * S + qrow] = dlt;
 
   auto tile = [&](int t, const bf16* ck, const bf16* cv, bf16* nk, bf16* nv) {
     const int k0 = t * kTileRows;
@@ -555,6 +621,65 @@ __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(
                          &sk[0][0] + (KS == 1 ? wave : grp * 2) * kQW * D, lane);
 }
 
+template <int D, bool STRIDED, bool DROP, int KS>
+__global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(const BwdArgs a) {
+  __shared__ BwdTiles<D> tiles;
+  // longest (latest) query blocks dispatch first
+  dq_workgroup<D, STRIDED, DROP, KS, true>(a, blockIdx.x, gridDim.y - 1 - blockIdx.y, tiles);
+}
+
+// ---------------------------------------------------------------- both in one launch
+// Grid (BH, key blocks + query blocks): dK/dV workgroups first (the longer chains), then the dQ
+// ones. OWN_DELTA: the dK/dV workgroups compute delta of their rows themselves (up to
+// kOwnDeltaMaxS of them) and the dQ workgroups write it; otherwise a pass before has.
+constexpr int kOwnDeltaMaxS = 1024;
+template <int D, bool STRIDED, bool DROP, int KS, bool OWN_DELTA>
+__global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocksNoDrop) void bwd_bf16_kernel(
+    const BwdArgs a) {
+  __shared__ BwdTiles<D> tiles;
+  __shared__ BwdStats stats;
+  __shared__ float own_delta[OWN_DELTA ? kOwnDeltaMaxS : 1];
+  const int n = gridDim.y / 2, y = blockIdx.y;  // as many key blocks as query blocks
+  if (y < n)
+    dkdv_workgroup<D, STRIDED, DROP, KS, OWN_DELTA>(a, blockIdx.x, y, tiles, stats, own_delta);
+  else
+    dq_workgroup<D, STRIDED, DROP, KS, OWN_DELTA>(a, blockIdx.x, 2 * n - 1 - y, tiles);
+}
+
+// How a backward is launched: dQ, then dK/dV (kSeparate); both in one launch with delta
+// computed where it is needed (kOneOwnDelta); or a delta pass, then both (kOneAfterDelta).
+enum BwdLaunch { kSeparate, kOneOwnDelta, kOneAfterDelta };
+struct BwdPlan {
+  BwdLaunch how;
+  int waves_per_group;
+};
+
+// One launch saves a kernel's start and end (~4 us) and lets the dQ workgroups fill the CUs that
+// the dK/dV ones leave idle at the end of their chains. It pays up to about four 128-row
+// workgroups of each kind per CU (one more per head counted), and whatever the batch for S <=
+// 256; beyond, the CUs are full and recomputing delta costs more. Separate -> one launch, us
+// (BH x S, D = 64): 128 x 128 11.5 -> 7.8, 192 x 256 20.0 -> 15.4, 24 x 1024 32.8 -> 24.5,
+// 96 x 1024 67 -> 60, 128 x 1024 83 -> 80, 24 x 4096 211 -> 192, 12 x 4096 127 -> 102, 768 x 256
+// 62 -> 60.5; on the other side 256 x 512 55.7 -> 56.7, 192 x 1024 115 -> 122. With dropout, whose
+// kernel holds two workgroups per CU where dQ alone holds three, the line for long rows is
+// nearer: 24 x 1024 44 -> 33, 40 x 1024 46 -> 44, 64 x 1024 67 -> 68, 96 x 1024 98 -> 107. Up to
+// 1,024 rows the dK/dV workgroups compute delta themselves (96 x 1024: 59 against 61 us with the
+// pass).
+// Two waves per row group then pay only while the grid, twice as large now, still fits on the
+// CUs, or for long chains up to twice that (one wave -> two): 64 x 256 10.8 -> 10.4, 24 x 1024
+// 30.4 -> 24.5, 96 x 512 21.4 -> 24.4, 64 x 800 31.2 -> 33.2, 24 x 2048 61 -> 57; 128 x 128
+// 7.7 -> 8.0.
+BwdPlan bwd_plan(int BH, int S, int D, bool drop) {
+  const long long cus = device_cus(), rows64 = (long long)BH * ((S + 63) / 64),
+                  wgs = (long long)BH * ((S + 127) / 128 + 1);
+  const bool one = drop && S > 512 ? 2 * wgs <= 3 * cus : S <= 256 || 2 * wgs <= 9 * cus;
+  if (!one) return {kSeparate, waves_per_group(BH, S, D, drop)};
+  const bool two = S > 64 && (S <= 128    ? 2 * rows64 <= cus
+                              : S < 1024 ? 2 * rows64 <= 3 * cus
+                                         : rows64 <= 3 * cus);
+  return {S <= kOwnDeltaMaxS ? kOneOwnDelta : kOneAfterDelta, two ? 2 : 1};
+}
+
 template <int D>
 hipError_t launch_bwd_bf16_t(bf16* dq, bf16* dk, bf16* dv, float* delta, const bf16* dout,
                              const bf16* out, const float* lse, const bf16* q, const bf16* k,
@@ -563,7 +688,10 @@ hipError_t launch_bwd_bf16_t(bf16* dq, bf16* dk, bf16* dv, float* delta, const b
   hipError_t e = hipSuccess;
   const bool contiguous = is_contiguous(L, S, D);
   const DropParams dr = drop_params(drop);  // dropout: contiguous layout only (caller checks)
-  if (phases & kBwdDelta) {
+  const BwdPlan plan = phases == kBwdAll
+                           ? bwd_plan(BH, S, D, drop != nullptr)
+                           : BwdPlan{kSeparate, waves_per_group(BH, S, D, drop != nullptr)};
+  if ((phases & kBwdDelta) || plan.how == kOneAfterDelta) {
     const long long rows = (long long)BH * S;
     const int row_blocks = (S + 31) / 32;
     if (contiguous)
@@ -574,32 +702,35 @@ hipError_t launch_bwd_bf16_t(bf16* dq, bf16* dk, bf16* dv, float* delta, const b
           delta, dout, out, S, rows, row_blocks, L);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  // P = exp2(S * scale * log2(e) - lse * log2(e)) holds for either sign of the scale.
-  const float sl2 = scale * kLog2e;
-  if (phases & kBwdDq) {
-    with_shape(waves_per_group(BH, S, D, drop != nullptr), drop != nullptr, !contiguous,
-               [&](auto strided, auto dropped, auto ks) {
-                 constexpr int QB = kQW * kWaves / ks();
-                 const dim3 grid(BH, (S + QB - 1) / QB);
-                 dq_bf16_kernel<D, strided(), dropped(), ks()><<<grid, 64 * kWaves, 0, stream>>>(
-                     dq, delta, q, k, v, dout, out, lse, S, sl2, scale, L, dr);
-               });
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  if (phases & kBwdDkdv) {
-    // s = S - lse/scale needs a nonzero scale: a zero one (P = exp(-lse)) runs with 1e-30,
-    // whose S*scale terms are then below fp32 resolution next to lse/scale.
-    const float se = scale != 0.f ? scale : 1e-30f;
-    with_shape(waves_per_group(BH, S, D, drop != nullptr), drop != nullptr, !contiguous,
-               [&](auto strided, auto dropped, auto ks) {
-                 constexpr int KB = kKW * kWaves / ks();
-                 const dim3 grid(BH, (S + KB - 1) / KB);
-                 dkdv_bf16_kernel<D, strided(), dropped(), ks()>
-                     <<<grid, 64 * kWaves, 0, stream>>>(dk, dv, q, k, v, dout, lse, delta, S,
-                                                        se * kLog2e, -1.0f / se, scale, L, dr);
-               });
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
+  // dQ: P = exp2(S * scale * log2(e) - lse * log2(e)) holds for either sign of the scale. dK/dV:
+  // s = S - lse/scale needs a nonzero scale: a zero one (P = exp(-lse)) runs with 1e-30, whose
+  // S*scale terms are then below fp32 resolution next to lse/scale.
+  const float se = scale != 0.f ? scale : 1e-30f;
+  const BwdArgs args{dq, dk, dv, delta, q,     k,     v,          dout,
+                     out, lse, S, scale, scale * kLog2e, se * kLog2e, -1.0f / se, L, dr};
+  const int ks = plan.waves_per_group;
+  const unsigned blocks = (unsigned)((S + 32 * kWaves / ks - 1) / (32 * kWaves / ks));
+  with_shape(ks, drop != nullptr, !contiguous, [&](auto strided, auto dropped, auto w) {
+    if (plan.how == kOneOwnDelta)
+      bwd_bf16_kernel<D, strided(), dropped(), w(), true>
+          <<<dim3(BH, 2 * blocks), 64 * kWaves, 0, stream>>>(args);
+    else if (plan.how == kOneAfterDelta)
+      bwd_bf16_kernel<D, strided(), dropped(), w(), false>
+          <<<dim3(BH, 2 * blocks), 64 * kWaves, 0, stream>>>(args);
+    if (plan.how != kSeparate) {
+      e = hipGetLastError();
+      return;
+    }
+    const dim3 grid(BH, blocks);
+    if (phases & kBwdDq) {
+      dq_bf16_kernel<D, strided(), dropped(), w()><<<grid, 64 * kWaves, 0, stream>>>(args);
+      if ((e = hipGetLastError()) != hipSuccess) return;
+    }
+    if (phases & kBwdDkdv) {
+      dkdv_bf16_kernel<D, strided(), dropped(), w()><<<grid, 64 * kWaves, 0, stream>>>(args);
+      e = hipGetLastError();
+    }
+  });
   return e;
 }
 

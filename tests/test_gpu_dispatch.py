@@ -66,7 +66,11 @@ def test_f32_shapes(gpu, BH, S, D):
 BF16_SHAPES = [(1, 64, 64), (1, 65, 64), (3, 95, 64), (2, 97, 32), (128, 128, 64), (129, 128, 64),
                (64, 256, 64), (65, 250, 64), (128, 257, 64), (129, 330, 64), (64, 800, 64),
                (74, 790, 64), (24, 2047, 64), (384, 100, 32), (385, 70, 32), (96, 800, 32),
-               (110, 800, 32)]
+               (110, 800, 32),
+               # the backward in one launch or two: delta held for up to 1,024 rows, its own pass
+               # past them, the line in heads x length, and the one for two waves
+               (3, 1024, 64), (3, 1025, 64), (2, 1030, 32), (128, 1000, 64), (129, 1000, 64),
+               (192, 500, 64), (300, 270, 64), (48, 511, 64), (49, 511, 64), (600, 200, 32)]
 BF16_TOLS = (2e-2, 1e-3, 5e-2, 5e-2, 5e-2)
 
 
@@ -76,7 +80,7 @@ def test_bf16_shapes(gpu, BH, S, D):
     _check(BH, S, D, torch.bfloat16, BF16_TOLS)
 
 
-@pytest.mark.parametrize("BH,S", [(2, 70), (5, 300), (99, 520), (150, 520)])
+@pytest.mark.parametrize("BH,S", [(2, 70), (5, 300), (99, 520), (150, 520), (3, 1030), (30, 600), (100, 257), (60, 700)])
 def test_bf16_dropout_and_strided_shapes(gpu, BH, S):
     """The dropout instantiations at p = 0 give the plain results, and the strided ones the
     contiguous ones', on both sides of the lines that differ between them: to the rounding of
