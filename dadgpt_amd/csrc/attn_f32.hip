@@ -22,8 +22,10 @@
 //           planes, P and dS in registers, dV^T += dO^T P and dK^T += Q^T dS (no atomics);
 //  dQ       a wave owns 32 queries again: S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T, with
 //           Q and dO split once and K, V as bf16 planes;
-//  delta    rowsum(dO * O), a separate pass that dK/dV and dQ both read.
-// One or two waves share a row group's chunks, by the size of the grid (f32_waves_per_group).
+//  delta    rowsum(dO * O), computed by the backward's workgroups or, for long rows, by a pass of
+//           its own.
+// dK/dV and dQ are workgroups of one launch. One or two waves share a row group's chunks, by the
+// size of the grid (fwd_waves_per_group, bwd_waves_per_group).
 // The next tile is loaded while the current one is on the matrix cores and split into planes as
 // it is stored: through registers in the forward; in dK/dV and dQ by direct loads into LDS,
 // which leaves the registers to the split operands (splitting dO, K and V once instead of at
@@ -488,23 +490,65 @@ struct BwdLds {
   }
 };
 
-template <int D, bool DROP, int KS>
-__global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dkdv_f32_kernel(
-    float* __restrict__ dk, float* __restrict__ dv, const float* __restrict__ q,
-    const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ dout,
-    const float* __restrict__ lse, const float* __restrict__ delta, int S, float scale,
-    const DropParams dr) {
+// What a backward kernel works on.
+struct F32BwdArgs {
+  float *dq, *dk, *dv, *delta;
+  const float *q, *k, *v, *dout, *out, *lse;
+  int S;
+  float scale;
+  DropParams dr;
+};
+// LDS of a workgroup: the tiles, and per query row of a dK/dV tile lse and delta * scale.
+template <int D, int KS>
+struct F32BwdShared {
+  __attribute__((aligned(16))) char tiles[BwdLds<D, KS>::kBytes];
+  __attribute__((aligned(16))) float sl[32 * KS], sd[32 * KS];
+};
+
+// delta of rows row0 .. S-1 into LDS, by the whole workgroup: D/4 lanes per row, one 16-byte
+// piece each, four groups of rows in flight.
+template <int D, int NT>
+__device__ __forceinline__ void delta_rows(float* delta, const float* dout, const float* out,
+                                           int row0, int S) {
+  constexpr int LPR = D / 4, ROWS = NT / LPR, N = 4;
+  const int c = threadIdx.x % LPR, lr = threadIdx.x / LPR;
+  for (int b0 = row0; b0 < S; b0 += N * ROWS) {
+    f32x4 g[N], o[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const size_t r = min(b0 + i * ROWS + lr, S - 1);
+      g[i] = *reinterpret_cast<const f32x4*>(dout + r * D + 4 * c);
+      o[i] = *reinterpret_cast<const f32x4*>(out + r * D + 4 * c);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      float acc = g[i][0] * o[i][0] + g[i][1] * o[i][1] + g[i][2] * o[i][2] + g[i][3] * o[i][3];
+      acc = lanes::group_sum<LPR>(acc);
+      const int r = b0 + i * ROWS + lr;
+      if (c == 0 && r < S) delta[r - row0] = acc;
+    }
+  }
+}
+
+// One workgroup's dK and dV. OWN_DELTA: delta is computed here, into own_delta (a float for each
+// row from the first tile on); otherwise it is read from a.delta.
+template <int D, bool DROP, int KS, bool OWN_DELTA>
+__device__ __forceinline__ void dkdv_f32_workgroup(const F32BwdArgs& a, int bh, int blk,
+                                                   F32BwdShared<D, KS>& sm, float* own_delta) {
   // Q and dO tiles: planes and raw
   using Lds = BwdLds<D, KS>;
   constexpr int TR = Lds::TR, NT = 64 * kGroups * KS;
-  __shared__ __attribute__((aligned(16))) char smem[Lds::kBytes];
+  char* smem = sm.tiles;
   bf16 *sqp = reinterpret_cast<bf16*>(smem), *sgp = sqp + Lds::kPlane;
   float* raw = reinterpret_cast<float*>(sgp + Lds::kPlane);
   constexpr int kSlot = Lds::slot_floats(2 * (D / 32));
   static_assert(kGroups * kSlot * 4 <= Lds::kBytes, "partials and staging fit");
-  // per query row of the tile: lse, and delta * scale
-  __shared__ __attribute__((aligned(16))) float sl[TR], sd[TR];
-  const int bh = blockIdx.x, blk = blockIdx.y;  // early key blocks see the most queries: first
+  float *sl = sm.sl, *sd = sm.sd;
+  const float *q = a.q, *k = a.k, *v = a.v, *dout = a.dout, *lse = a.lse, *delta = a.delta;
+  float *dk = a.dk, *dv = a.dv;
+  const int S = a.S;
+  const float scale = a.scale;
+  const DropParams& dr = a.dr;
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar
   const int grp = wave % kGroups, sub = wave / kGroups;
@@ -537,17 +581,25 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dkdv_f32_ke
   auto load_stats = [&](int row0) {
     const int r = row0 + (threadIdx.x & (TR - 1));
     pl = r < S ? lse[(size_t)bh * S + r] : 0.f;
-    pd = r < S ? delta[(size_t)bh * S + r] : 0.f;
+    if constexpr (OWN_DELTA)
+      pd = 0.f;  // read from own_delta as the tile is staged
+    else
+      pd = r < S ? delta[(size_t)bh * S + r] : 0.f;
   };
   tq.issue(t0 * TR);
   tg.issue(t0 * TR);
   load_stats(t0 * TR);
+  if constexpr (OWN_DELTA)
+    delta_rows<D, NT>(own_delta, dout + base, a.out + base, t0 * TR, S);
   for (int t = t0; t < n_tiles; ++t) {
     wait_vm_lds<0>();  // this wave's pieces of the tile
     __syncthreads();   // every wave is done with the previous tile's planes
     store_x3<D, TR>(tq, sqp);
     store_x3<D, TR>(tg, sgp);
-    if (threadIdx.x < TR) sl[threadIdx.x] = pl, sd[threadIdx.x] = pd * scale;
+    if (threadIdx.x < TR) {
+      if constexpr (OWN_DELTA) pd = own_delta[min(t * TR + (int)threadIdx.x, S - 1) - t0 * TR];
+      sl[threadIdx.x] = pl, sd[threadIdx.x] = pd * scale;
+    }
     __syncthreads();
     if (t + 1 < n_tiles) {
       tq.issue((t + 1) * TR);
@@ -616,21 +668,23 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dkdv_f32_ke
   store_rows_t<D>(dv + base, k0, S, dva, 1.0f, slot, lane);  // after the wave's dK reads
 }
 
-template <int D, bool DROP, int KS>
-__global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dq_f32_kernel(
-    float* __restrict__ dq, const float* __restrict__ q, const float* __restrict__ k,
-    const float* __restrict__ v, const float* __restrict__ dout, const float* __restrict__ lse,
-    const float* __restrict__ delta, int S, float scale, const DropParams dr) {
+// One workgroup's dQ. OWN_DELTA: delta of its rows is computed here and written; otherwise read.
+template <int D, bool DROP, int KS, bool OWN_DELTA>
+__device__ __forceinline__ void dq_f32_workgroup(const F32BwdArgs& a, int bh, int blk,
+                                                 F32BwdShared<D, KS>& sm) {
   // K and V tiles: planes and raw
   using Lds = BwdLds<D, KS>;
   constexpr int TR = Lds::TR, NT = 64 * kGroups * KS;
-  __shared__ __attribute__((aligned(16))) char smem[Lds::kBytes];
+  char* smem = sm.tiles;
   bf16 *skp = reinterpret_cast<bf16*>(smem), *svp = skp + Lds::kPlane;
   float* raw = reinterpret_cast<float*>(svp + Lds::kPlane);
   constexpr int kSlot = Lds::slot_floats(D / 32);
   static_assert(kGroups * kSlot * 4 <= Lds::kBytes, "partials and staging fit");
-  const int bh = blockIdx.x;
-  const int blk = gridDim.y - 1 - blockIdx.y;  // longest query blocks first
+  const float *q = a.q, *k = a.k, *v = a.v, *dout = a.dout, *lse = a.lse;
+  float *dq = a.dq, *delta = a.delta;
+  const int S = a.S;
+  const float scale = a.scale;
+  const DropParams& dr = a.dr;
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar
   const int grp = wave % kGroups, sub = wave / kGroups;
@@ -645,7 +699,25 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dq_f32_kern
   load_split_row<D>(qb, q + base + (size_t)qc * D, h);
   load_split_row<D>(gb, dout + base + (size_t)qc * D, h);
   const float my_lse = lse[(size_t)bh * S + qc];
-  const float my_dscale = delta[(size_t)bh * S + qc] * scale;
+  float my_delta;
+  if constexpr (OWN_DELTA) {
+    const float* g = dout + base + (size_t)qc * D + 8 * h;
+    const float* o = a.out + base + (size_t)qc * D + 8 * h;
+    float part = 0.f;
+#pragma unroll
+    for (int ds = 0; ds < D / 16; ++ds)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(g + 16 * ds + e);
+        const f32x4 y = *reinterpret_cast<const f32x4*>(o + 16 * ds + e);
+        part += x[0] * y[0] + x[1] * y[1] + x[2] * y[2] + x[3] * y[3];
+      }
+    my_delta = sum_halves(part);
+    if (h == 0 && qi < S && sub == 0) delta[(size_t)bh * S + qi] = my_delta;
+  } else {
+    my_delta = delta[(size_t)bh * S + qc];
+  }
+  const float my_dscale = my_delta * scale;
   f32x16 acc[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) acc[db] = zero16();
@@ -702,24 +774,51 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void dq_f32_kern
   store_rows_t<D>(dq + base, q0, S, acc, 1.0f, slot, lane);
 }
 
+// The backward is one launch: grid (BH, key blocks + query blocks), dK/dV workgroups first (the
+// longer chains), then the dQ ones, which fill the CUs as those run out. As two launches, each
+// with its own start, end and half-idle last round (B4 H12 S1024 / B1 H24 S1024 / B16 H12 S256,
+// us): 158 -> 143, 140 -> 86, 68 -> 55; where the CUs are full anyway (B16 H12 S1024) 532 -> 527.
+// OWN_DELTA: both kinds compute delta themselves, which saves the small grids a launch (4 x 64:
+// 10.0 -> 8.3 us); past kOwnDeltaMaxS rows, where dK/dV would read O and dO once per key block
+// more, a pass before does it (96 x 1024: 268 against 263.5 us).
+constexpr int kOwnDeltaMaxS = 512;
+template <int D, bool DROP, int KS, bool OWN_DELTA>
+__global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void bwd_f32_kernel(
+    const F32BwdArgs a) {
+  __shared__ F32BwdShared<D, KS> sm;
+  __shared__ float own_delta[OWN_DELTA ? kOwnDeltaMaxS : 1];
+  const int n = gridDim.y / 2, y = blockIdx.y;  // as many key blocks as query blocks
+  if (y < n)
+    dkdv_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, y, sm, own_delta);
+  else
+    dq_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, 2 * n - 1 - y, sm);
+}
+
 // Waves per row group. With one, a workgroup walks its chunks four waves wide, two workgroups
 // to a CU; a grid of no more workgroups than that (all of them start at once) lasts as long as
 // the longest one's chain, so each group then gets a second wave and the chain is half as long.
-// (all figures before the mask branch and pack_once below, which took another 2-7%)
-// B4 H12 S1024 D64 (384 workgroups): forward 64.6 -> 49.6 us, backward 197 -> 162 us; B8 H8
-// (512): 68.9 -> 60.8, 212 -> 196. Larger grids keep the CUs busy anyway and would pay for the
-// wider barrier and the merge: 640 workgroups 141 -> 147 and 453 -> 468 us, B16 H12 S1024 (1,536)
-// 165 -> 186 and 528 -> 600 us. Up to three chunks (S <= 96) there is too little to share: S 65
-// backward 27.7 -> 29.5 us, S 100 34.5 -> 33.3.
-int f32_waves_per_group(int BH, int S) {
-  const long long wgs = (long long)BH * ((S + kRows - 1) / kRows);
-  return S > 96 && wgs <= 2LL * device_cus() ? 2 : 1;
+// Past one workgroup per CU the gain shrinks with the chain's length. Forward, one -> two (us):
+// 128 x 256 (256 workgroups) 21.0 -> 18.4, 48 x 1024 (384) 64.6 -> 49.6, 64 x 1024 (512) 68.8 ->
+// 64.7, 96 x 512 (384) 37.8 -> 32.7; 128 x 512 (512) 38.1 -> 39.0, 128 x 300 (384) 24.8 -> 27.3,
+// 40 x 2048 (640) 141 -> 147, 192 x 1024 165 -> 186; up to three chunks (S <= 96) there is too
+// little to share.
+int fwd_waves_per_group(int BH, int S) {
+  const long long wgs = (long long)BH * ((S + kRows - 1) / kRows), cus = device_cus();
+  const long long most = S >= 768 ? 4 * cus : S >= 512 ? 3 * cus : 2 * cus;  // halves of a CU
+  return S > 96 && 2 * wgs <= most ? 2 : 1;
+}
+// The backward's grid holds two workgroups per 128 rows, so its line is at half as many rows:
+// 24 x 1024 (192 of each kind) 120 -> 86, 128 x 128 22.6 -> 19.6, 48 x 1024 (384) 143 -> 150,
+// 96 x 512 81 -> 94. Short sequences: 4 x 64 8.4 -> 7.2, 192 x 64 15.5 -> 20.6.
+int bwd_waves_per_group(int BH, int S) {
+  const long long wgs = (long long)BH * ((S + kRows - 1) / kRows), cus = device_cus();
+  return wgs <= (S > 96 ? cus : cus / 4) ? 2 : 1;
 }
 
 // f(whether to drop, waves per row group) as compile-time constants.
 template <typename F>
-void with_f32_shape(int BH, int S, bool drop, F f) {
-  const bool two = f32_waves_per_group(BH, S) == 2;
+void with_f32_shape(int waves_per_group, bool drop, F f) {
+  const bool two = waves_per_group == 2;
   auto with_drop = [&](auto d) {
     if (two)
       f(d, std::integral_constant<int, 2>{});
@@ -737,7 +836,7 @@ hipError_t fwd_f32_t(float* out, float* lse, const float* q, const float* k, con
                      int BH, int S, float scale, hipStream_t stream, const Dropout* drop) {
   const dim3 grid(BH, (S + kRows - 1) / kRows);
   const DropParams dr = drop_params(drop);
-  with_f32_shape(BH, S, drop != nullptr, [&](auto drop_c, auto ks) {
+  with_f32_shape(fwd_waves_per_group(BH, S), drop != nullptr, [&](auto drop_c, auto ks) {
     fwd_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(out, lse, q, k, v,
                                                                              S, scale, dr);
   });
@@ -749,21 +848,22 @@ hipError_t bwd_f32_t(float* dq, float* dk, float* dv, float* delta, const float*
                      const float* out, const float* lse, const float* q, const float* k,
                      const float* v, int BH, int S, float scale, hipStream_t stream,
                      const Dropout* drop) {
-  const DropParams dr = drop_params(drop);
-  const long long rows = (long long)BH * S;
-  const long long blocks = (rows * (D / 4) + 255) / 256;
-  delta_f32_kernel<D><<<(unsigned)(blocks < 16384 ? blocks : 16384), 256, 0, stream>>>(
-      delta, dout, out, rows);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const dim3 grid(BH, (S + kRows - 1) / kRows);
-  with_f32_shape(BH, S, drop != nullptr, [&](auto drop_c, auto ks) {
-    dkdv_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(
-        dk, dv, q, k, v, dout, lse, delta, S, scale, dr);
-    e = hipGetLastError();
-    if (e != hipSuccess) return;
-    dq_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(
-        dq, q, k, v, dout, lse, delta, S, scale, dr);
+  const F32BwdArgs args{dq, dk, dv, delta, q, k, v, dout, out, lse, S, scale, drop_params(drop)};
+  const bool own = S <= kOwnDeltaMaxS;
+  hipError_t e = hipSuccess;
+  if (!own) {
+    const long long rows = (long long)BH * S, blocks = (rows * (D / 4) + 255) / 256;
+    delta_f32_kernel<D><<<(unsigned)(blocks < 16384 ? blocks : 16384), 256, 0, stream>>>(
+        delta, dout, out, rows);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  const dim3 grid(BH, 2 * ((S + kRows - 1) / kRows));
+  with_f32_shape(bwd_waves_per_group(BH, S), drop != nullptr, [&](auto drop_c, auto ks) {
+    constexpr int threads = 64 * kGroups * ks();
+    if (own)
+      bwd_f32_kernel<D, drop_c(), ks(), true><<<grid, threads, 0, stream>>>(args);
+    else
+      bwd_f32_kernel<D, drop_c(), ks(), false><<<grid, threads, 0, stream>>>(args);
     e = hipGetLastError();
   });
   return e;

@@ -48,10 +48,13 @@ def _check(BH, S, D, dtype, tols):
         assert torch.isfinite(x).all().item() and torch.equal(x, y)
 
 
-# One or two waves per row group: S on both sides of three chunks (96), and grids of 512 and
-# more 128-row workgroups (two per CU of 256) around the line.
+# One or two waves per row group: S on both sides of three chunks (96), grids of 256, 384 and 512
+# 128-row workgroups (the forward's lines on 256 CUs by length), 256 (the backward's) and 64 (its
+# line for short sequences), and delta held for up to 512 rows or in its own pass.
 F32_SHAPES = [(3, 96, 64), (3, 97, 64), (2, 129, 64), (5, 160, 32), (1, 500, 64), (64, 1000, 64),
-              (65, 1000, 64), (128, 385, 32), (129, 390, 32), (512, 100, 64), (513, 100, 32)]
+              (65, 1000, 64), (128, 385, 32), (129, 390, 32), (512, 100, 64), (513, 100, 32),
+              (64, 40, 64), (65, 33, 64), (32, 1000, 64), (33, 1000, 32), (3, 512, 64),
+              (3, 513, 64), (86, 300, 64), (85, 300, 64), (76, 600, 32), (77, 600, 64)]
 
 
 @pytest.mark.parametrize("BH,S,D", F32_SHAPES)
