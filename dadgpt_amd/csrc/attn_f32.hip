@@ -276,6 +276,23 @@ __device__ __forceinline__ f32x16 score_tile_px(const bf16* planes, const X3 (&b
   }
   return acc;
 }
+// score_tile_px with the lower planes of the B operand in LDS (`blo`, by lane).
+template <int D, int TR>
+__device__ __forceinline__ f32x16 score_tile_pxl(const bf16* planes, const bf16x8 (&b0)[D / 16],
+                                                 const bf16x8 (*blo)[2][64], int lane,
+                                                 const LaneLds& lo) {
+  uint32_t ra[D / 16];
+  row_addr_xor<D>(ra, lo.ro);
+  f32x16 acc = zero16();
+#pragma unroll
+  for (int ds = 0; ds < D / 16; ++ds) {
+    X3 a;
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) a.v[pl] = lds_row_at(planes + pl * TR * D, ra[ds]);
+    acc = mfma_x6(a, X3{{b0[ds], blo[ds][0][lane], blo[ds][1][lane]}}, acc);
+  }
+  return acc;
+}
 template <int D, int TR>
 __device__ __forceinline__ void accumulate_t_px(f32x16 (&acc)[D / 32], const bf16* planes,
                                                 const f32x16& p, const LaneLds& lo) {
@@ -503,6 +520,8 @@ template <int D, int KS>
 struct F32BwdShared {
   __attribute__((aligned(16))) char tiles[BwdLds<D, KS>::kBytes];
   __attribute__((aligned(16))) float sl[32 * KS], sd[32 * KS];
+  // dK/dV at D = 64: the lower planes of the groups' V rows, by lane
+  bf16x8 vlo[kGroups][D == 64 ? D / 16 : 1][2][64];
 };
 
 // delta of rows row0 .. S-1 into LDS, by the whole workgroup: D/4 lanes per row, one 16-byte
@@ -558,16 +577,30 @@ __device__ __forceinline__ void dkdv_f32_workgroup(const F32BwdArgs& a, int bh, 
   const int t0 = (blk * kRows) / TR;  // first query tile with a query >= the first key
   const int n_tiles = (S + TR - 1) / TR;
 
-  X3 kb[D / 16], vb[D / 16];  // the lane's K and V rows (score-product B layout), split
+  // The lane's K and V rows (score-product B layout), split. At D = 64 V's lower planes go to LDS,
+  // which the two waves of a group share (published by the first barrier): with all six planes
+  // in registers (96 of 256) the loop spilled and the compiler could not move the softmax under
+  // the dP products (B16 H12 S1024 513 -> 498 us, with dropout B4 180 -> 153; at D = 32, where
+  // they fit, the LDS reads cost 4%).
+  constexpr bool kVLds = D == 64;
+  X3 kb[D / 16], vb[D / 16];
   load_split_row<D>(kb, k + base + (size_t)min(kj, S - 1) * D, h);
   load_split_row<D>(vb, v + base + (size_t)min(kj, S - 1) * D, h);
+  bf16x8 vb0[D / 16];
 #pragma unroll
-  for (int ds = 0; ds < D / 16; ++ds)
+  for (int ds = 0; ds < D / 16; ++ds) {
+    vb0[ds] = vb[ds].v[0];
+    if constexpr (kVLds) {
+      if (sub == 0) sm.vlo[grp][ds][0][lane] = vb[ds].v[1], sm.vlo[grp][ds][1][lane] = vb[ds].v[2];
+      asm volatile("" : "+v"(vb0[ds]));
+    }
+    // not to be split again inside the loop
 #pragma unroll
     for (int pl = 0; pl < 3; ++pl) {
       asm volatile("" : "+v"(kb[ds].v[pl]));
-      asm volatile("" : "+v"(vb[ds].v[pl]));
+      if constexpr (!kVLds) asm volatile("" : "+v"(vb[ds].v[pl]));
     }
+  }
   f32x16 da[2 * (D / 32)];  // dV^T, then dK^T
   f32x16(&dva)[D / 32] = reinterpret_cast<f32x16(&)[D / 32]>(da[0]);
   f32x16(&dka)[D / 32] = reinterpret_cast<f32x16(&)[D / 32]>(da[D / 32]);
@@ -612,46 +645,48 @@ __device__ __forceinline__ void dkdv_f32_workgroup(const F32BwdArgs& a, int bh, 
     const bf16 *qc = sqp + 32 * sub * D, *gc = sgp + 32 * sub * D;
     // lane (l32, h), register u: query qrow0 + reg_row(u, h), key kj
     f32x16 s = score_tile_px<D, TR>(qc, kb, lo);   // Q K^T
-    f32x16 dp = score_tile_px<D, TR>(gc, vb, lo);  // dO V^T
+    f32x16 dp;  // dO V^T
+    if constexpr (kVLds)
+      dp = score_tile_pxl<D, TR>(gc, vb0, sm.vlo[grp], lane, lo);
+    else
+      dp = score_tile_px<D, TR>(gc, vb, lo);
     uint32_t keep = 0;
     if constexpr (DROP) keep = keep_col16(dr, (uint64_t)bh * S + qrow0, k0, lane);
-    // Statistics of the chunk's rows 32 sub + reg_row(u, h): registers 8j..8j+7 are the 8
-    // consecutive rows 32 sub + 16j + 8h .., two 16-byte LDS reads each.
+    // P in place of S, under the dP products: registers 8j..8j+7 are the 8 consecutive rows
+    // 32 sub + 16j + 8h .., their statistics two 16-byte LDS reads each
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const f32x4 ls =
+          *reinterpret_cast<const f32x4*>(sl + 32 * sub + 16 * (g4 >> 1) + 8 * h + 4 * (g4 & 1));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[4 * g4 + e] = exp_acc(fmaf(s[4 * g4 + e], scale, -ls[e]));
+    }
     // keys after a query, or rows past S, only where the chunk reaches the wave's first
     // keys or S (wave-uniform)
-    const bool mask = qrow0 < k0 + 31 || qrow0 + 31 >= S;
-    // (the mask's compares and selects, 80 instructions, only in the instance that needs them)
-    auto weights = [&](auto masked) {
+    if (qrow0 < k0 + 31 || qrow0 + 31 >= S) {
 #pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        // registers 4 g4 .. 4 g4 + 3 are the consecutive rows 32 sub + 16(g4/2) + 8h + 4(g4%2) ..;
-        // their statistics are read here, four at a time, rather than all ahead of the loop
-        const int r = 32 * sub + 16 * (g4 >> 1) + 8 * h + 4 * (g4 & 1);
-        asm volatile("" ::: "memory");
-        const f32x4 ls = *reinterpret_cast<const f32x4*>(sl + r);
-        const f32x4 ds = *reinterpret_cast<const f32x4*>(sd + r);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int u = 4 * g4 + e;
-          const int qrow = qrow0 + reg_row(u, h);
-          float p = exp_acc(fmaf(s[u], scale, -ls[e]));
-          if (masked() && !(kj <= qrow && qrow < S)) p = 0.f;
-          float g = dp[u];
-          if constexpr (DROP) {
-            const float f = keep_factor(keep, u, dr.scale);
-            g *= f;
-            s[u] = p * f;  // the probability that multiplied V
-          } else {
-            s[u] = p;
-          }
-          dp[u] = p * fmaf(g, scale, -ds[e]);  // P (dP - delta) scale
-        }
+      for (int u = 0; u < 16; ++u) {
+        const int qrow = qrow0 + reg_row(u, h);
+        s[u] = kj <= qrow && qrow < S ? s[u] : 0.f;
       }
-    };
-    if (mask)
-      weights(std::true_type{});
-    else
-      weights(std::false_type{});
+    }
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const f32x4 ds =
+          *reinterpret_cast<const f32x4*>(sd + 32 * sub + 16 * (g4 >> 1) + 8 * h + 4 * (g4 & 1));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int u = 4 * g4 + e;
+        const float p = s[u];
+        float g = dp[u];
+        if constexpr (DROP) {
+          const float f = keep_factor(keep, u, dr.scale);
+          g *= f;
+          s[u] = p * f;  // the probability that multiplied V
+        }
+        dp[u] = p * fmaf(g, scale, -ds[e]);  // P (dP - delta) scale
+      }
+    }
     accumulate_t_px<D, TR>(dva, gc, s, lo);   // dV^T += dO^T P
     accumulate_t_px<D, TR>(dka, qc, dp, lo);  // dK^T += Q^T dS
   }
