@@ -349,10 +349,10 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
     const DropParams dr) {
   constexpr int NT = 64 * kGroups * KS, TR = 64, CPT = 2 / KS;  // chunks per tile and wave
   // K and V tiles as three bf16 planes each; after the tile loop they hold the second waves'
-  // partial results, then the epilogue's fp32 staging rows
+  // partial results, then the epilogue's fp32 staging rows. With two waves per group there are
+  // two sets (one workgroup has the CU's LDS to itself), see the tile loop.
   constexpr int kPlane = 3 * TR * D;
-  __shared__ __attribute__((aligned(16))) bf16 planes[2 * kPlane];
-  bf16 *skp = planes, *svp = planes + kPlane;
+  __shared__ __attribute__((aligned(16))) bf16 planes[KS * 2 * kPlane];
   constexpr int kPart = (D / 32) * 1024 + 128;  // a partial: O, m and l (floats)
   constexpr int kStage = 32 * (D + kPitchPad);  // a wave's staged rows (floats)
   static_assert(4 * kPlane >= 4 * kGroups * (KS > 1 && kPart > kStage ? kPart : kStage),
@@ -378,15 +378,17 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
   Tile<D, TR, NT> tk, tv;
   tk.load(k + base, 0, S);
   tv.load(v + base, 0, S);
-  for (int t = 0; t < n_tiles; ++t) {
-    __syncthreads();  // the previous tile's reads are done
-    store_x3<D, TR>(tk, skp);
-    store_x3<D, TR>(tv, svp);
-    __syncthreads();
-    if (t + 1 < n_tiles) {  // next tile in flight during this one
+  // Splits the loaded tile t into `to` and loads tile t + 1.
+  auto stage = [&](int t, bf16* to) {
+    store_x3<D, TR>(tk, to);
+    store_x3<D, TR>(tv, to + kPlane);
+    if (t + 1 < n_tiles) {
       tk.load(k + base, (t + 1) * TR, S);
       tv.load(v + base, (t + 1) * TR, S);
     }
+  };
+  auto compute = [&](int t, const bf16* skp) {
+    const bf16* svp = skp + kPlane;
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
       const int c = KS == 1 ? i : sub;
@@ -440,6 +442,31 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
 #pragma unroll
       for (int u = 0; u < 16; ++u) s[u] = DROP ? w[u] * keep_factor(keep, u, dr) : w[u];
       accumulate_t_p<D, TR>(o, svp, 32 * c, s, lane);
+    }
+  };
+  if constexpr (KS == 1) {
+    for (int t = 0; t < n_tiles; ++t) {
+      __syncthreads();  // the previous tile's reads are done
+      stage(t, planes);
+      __syncthreads();
+      compute(t, planes);
+    }
+  } else {
+    // One barrier per tile: tile t is computed from one set while t + 1 is split into the other.
+    // A SIMD holds one wave of each half, and the halves do the two in opposite order: in step,
+    // both would be on the matrix cores and then both on the VALU.
+    bf16 *set0 = planes, *set1 = planes + 2 * kPlane;
+    stage(0, set0);
+    __syncthreads();
+    auto tile = [&](int t, bf16* cur, bf16* next) {
+      if (sub == 1 && t + 1 < n_tiles) stage(t + 1, next);
+      compute(t, cur);
+      if (sub == 0 && t + 1 < n_tiles) stage(t + 1, next);
+      __syncthreads();
+    };
+    for (int t = 0; t < n_tiles; t += 2) {
+      tile(t, set0, set1);
+      if (t + 1 < n_tiles) tile(t + 1, set1, set0);
     }
   }
   __syncthreads();  // every wave is done with the tiles: they hold partials and staging now
