@@ -62,18 +62,18 @@ int device_cus();
 // 32-row chunks of a tile; with two it owns 64, two waves taking one chunk of each tile and
 // merging at the end. Two make the chain of the longest workgroup half as long and its stream
 // twice as expensive per row, so they pay where a grid is so small that it lasts as long as that
-// chain, and cost 5-15% where the CUs are full anyway. Measured, one wave -> two, forward /
-// backward us (BH x S, D = 64): 48 x 1024 17.4 -> 14.0 / 48 -> 38.6, 64 x 1024 18.2 -> 17.9 /
-// 54.0 -> 54.4, 72 x 1024 19.2 -> 19.8 / 56 -> 59; 24 x 2048 29 -> 22.5 / 84 -> 66, 36 x 2048
-// 32.2 -> 32.2 / 96 -> 95; 12 x 4096 53 -> 40 / 157 -> 120; 128 x 512 11.2 -> 11.0 / 32 -> 38;
-// 96 x 384 9.3 -> 8.5 / 24.2 -> 22.5, 128 x 320 8.3 -> 7.8 / 21.7 -> 21.2, hence the line at two
-// 128-row workgroups per CU, one more per head counted. Short sequences (S <= 256, at most two
-// tiles' worth of chain to save) need one 64-row workgroup per CU: 128 x 128 5.5 -> 5.2 /
-// 13.2 -> 11.7, 192 x 128 5.6 -> 5.7 / 13.5 -> 13.8; one tile (S <= 64) has nothing to share. At
-// D = 32, where half the registers leave more workgroups resident, and with dropout, whose
-// generator lengthens the chain, the line lies further out: D = 32 72 x 1024 14.4 -> 12.8 /
-// 37 -> 32, 96 x 1024 14.4 -> 14.6 / 39.3 -> 38.3; dropout 96 x 1024 32 -> 31 / 99 -> 92,
-// 128 x 1024 35.3 -> 37.5 / 110 -> 115, 128 x 512 14.6 -> 14.6 / 41.1 -> 42.7.
+// chain, and cost 5-15% where the CUs are full anyway. Forward, one wave -> two, us (BH x S,
+// D = 64): 48 x 1024 16.8 -> 14.3, 64 x 1024 18.2 -> 16.1, 72 x 1024 18.8 -> 19.1, 96 x 1024
+// 21.5 -> 23.4; 36 x 2048 32.4 -> 29.0, 48 x 2048 35.7 -> 35.9; 12 x 4096 55 -> 39.6, 24 x 4096
+// 64.4 -> 64.3; 96 x 512 11.7 -> 10.5, 100 x 520 11.6 -> 10.5, 128 x 512 11.8 -> 11.8, 192 x 512
+// 16.1 -> 19.2: the line is at 2.4 128-row workgroups per CU, one more per head counted. Short
+// sequences (S <= 256, at most two tiles' worth of chain to save) need one 64-row workgroup per
+// CU: 128 x 128 5.5 -> 5.2, 192 x 128 5.6 -> 5.7, 192 x 256 7.6 -> 8.1; one tile (S <= 64) has
+// nothing to share. At D = 32, where half the registers leave more workgroups resident, and with
+// dropout, whose generator lengthens the chain, the line lies further out: D = 32 72 x 1024
+// 14.4 -> 12.8, 96 x 1024 14.8 -> 14.8; dropout, forward and dQ + dK/dV 96 x 1024 32 / 99 ->
+// 31 / 92, 128 x 1024 35.3 / 110 -> 37.5 / 115, 128 x 512 14.6 / 41.1 -> 14.6 / 42.7. (The backward
+// follows this only where it runs as two launches, see bwd_plan.)
 inline int waves_per_group(int BH, int S, int D, bool drop) {
   if (S <= 64) return 1;
   const long long cus = device_cus(), wgs = (long long)BH * ((S + 127) / 128 + 1);
@@ -85,7 +85,7 @@ inline int waves_per_group(int BH, int S, int D, bool drop) {
   else if (drop && S > 512)
     two = 2 * wgs <= 7 * cus;
   else
-    two = wgs <= 2 * cus;
+    two = 5 * wgs <= 12 * cus;
   return two ? 2 : 1;
 }
 
@@ -99,8 +99,8 @@ hipError_t launch_fwd_bf16(bf16* out, float* lse, const bf16* q, const bf16* k, 
 // Causal flash backward, bf16 in/out. delta [BH,S] fp32 is written (scratch, as the
 // reference's). dq/dk/dv are overwritten. `phases` selects the kernels launched, in order:
 // bit 1 dQ (which also computes and writes delta), bit 2 dK/dV (reads delta); kBwdAll is the
-// whole backward, which may run both in one launch. Bit 0 launches the standalone delta kernel (a separate pass, equal up to
-// fp32 summation order; not part of kBwdAll).
+// whole backward, which may run both in one launch. Bit 0 launches the standalone delta kernel
+// (a separate pass, equal up to fp32 summation order; not part of kBwdAll).
 constexpr int kBwdDelta = 1, kBwdDq = 2, kBwdDkdv = 4, kBwdAll = kBwdDq | kBwdDkdv;
 hipError_t launch_bwd_bf16(bf16* dq, bf16* dk, bf16* dv, float* delta, const bf16* dout,
                            const bf16* out, const float* lse, const bf16* q, const bf16* k,
