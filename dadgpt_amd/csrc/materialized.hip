@@ -39,6 +39,30 @@ __device__ __forceinline__ unsigned wave_row0() {
 
 __device__ __forceinline__ float wave_max(float x) { return lanes::group_max<64>(x); }
 __device__ __forceinline__ float wave_sum(float x) { return lanes::group_sum<64>(x); }
+// The same for several rows side by side, step by step.
+template <int N, typename F>
+__device__ __forceinline__ void each(float (&x)[N], F f) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = f(x[i]);
+}
+template <int N>
+__device__ __forceinline__ void wave_max_of(float (&x)[N]) {
+  each(x, [](float v) { return fmaxf(v, lanes::dpp<lanes::kQuadXor1>(v)); });
+  each(x, [](float v) { return fmaxf(v, lanes::dpp<lanes::kQuadXor2>(v)); });
+  each(x, [](float v) { return fmaxf(v, lanes::dpp<lanes::kHalfMirror>(v)); });
+  each(x, [](float v) { return fmaxf(v, lanes::dpp<lanes::kMirror>(v)); });
+  each(x, [](float v) { return lanes::max_xor16(v); });
+  each(x, [](float v) { return lanes::max_xor32(v); });
+}
+template <int N>
+__device__ __forceinline__ void wave_sum_of(float (&x)[N]) {
+  each(x, [](float v) { return v + lanes::dpp<lanes::kQuadXor1>(v); });
+  each(x, [](float v) { return v + lanes::dpp<lanes::kQuadXor2>(v); });
+  each(x, [](float v) { return v + lanes::dpp<lanes::kHalfMirror>(v); });
+  each(x, [](float v) { return v + lanes::dpp<lanes::kMirror>(v); });
+  each(x, [](float v) { return lanes::sum_xor16(v); });
+  each(x, [](float v) { return lanes::sum_xor32(v); });
+}
 
 // Four floats at any 4-byte address: gfx950 loads and stores 16 bytes at dword alignment in one
 // instruction, so rows of any length and offset move in the same pieces as aligned ones.
@@ -126,11 +150,13 @@ int rows_per_wave(long long rows, int pieces) {
   return n;
 }
 
-// Softmax of rows of at most 256 NP columns, RPW rows per wave, each read once.
-// [BH 192, S 256] (50 MB) causal, in place: 27 us with the looping kernel below (three passes,
-// two exponentials per element), 19 us here (its 75 MB take 13-15; the exponentials' VALU work
-// does not hide completely under them).
-template <int MODE, int NP, int RPW>
+// Softmax of rows of at most 256 NP columns, RPW rows per wave, each read once. WHOLE: the
+// columns are a multiple of four, so no piece crosses a row's end.
+// [BH 192, S 256] (50 MB) causal, in place: 24-27 us with the looping kernel below (three
+// passes, two exponentials per element), 17.7 us read once but reduced row after row (each
+// reduction's twelve dependent steps waited out, every element selected three times), 16.4 us
+// here; its 75 MB take 15 at the rate of a copy.
+template <int MODE, int NP, int RPW, bool WHOLE>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_reg_kernel(
     float* out, const float* in, unsigned rows, int cols, int S, float scale,
     const int* __restrict__ lens, int H) {
@@ -147,38 +173,59 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_reg_kernel(
     for (int n = 0; n < NP; ++n)
       x[i][n] = load_raw(in + (size_t)r * cols, c0 + 256 * n, max(limit[i] - 1, 0), cols);
   }
+  // Masked columns become -inf, which exponentiates to 0; whatever a piece's other columns hold
+  // (past the row's end, or past the last visible piece) does too. The rows' reductions run side
+  // by side: a single one waits out each of its twelve dependent steps.
+  float mx[RPW], sum[RPW];
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) {
+    mx[i] = initial_max(limit[i], cols);
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      const int c = c0 + 256 * n;
+      if constexpr (!WHOLE) x[i][n] = whole_piece(x[i][n], c, cols);
+      if constexpr (MODE != kPlain) x[i][n] *= scale;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[i][n][e] = c + e < limit[i] ? x[i][n][e] : neg_inf();
+        mx[i] = fmaxf(mx[i], x[i][n][e]);
+      }
+    }
+  }
+  wave_max_of(mx);
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) {
+    sum[i] = 0.f;
+#pragma unroll
+    for (int n = 0; n < NP; ++n)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[i] += x[i][n][e] = expf(x[i][n][e] - mx[i]);
+  }
+  wave_sum_of(sum);
 #pragma unroll
   for (int i = 0; i < RPW; ++i) {
     if (r0 + i >= rows) return;
     float* dst = out + (size_t)(r0 + i) * cols;
-    float mx = initial_max(limit[i], cols);
-#pragma unroll
-    for (int n = 0; n < NP; ++n) {
-      x[i][n] = whole_piece(x[i][n], c0 + 256 * n, cols);
-      if constexpr (MODE != kPlain) x[i][n] *= scale;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c0 + 256 * n + e < limit[i]) mx = fmaxf(mx, x[i][n][e]);
-    }
-    mx = wave_max(mx);
-    float sum = 0.f;
-#pragma unroll
-    for (int n = 0; n < NP; ++n)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c0 + 256 * n + e < limit[i]) sum += x[i][n][e] = expf(x[i][n][e] - mx);
-    const float masked = masked_weight(mx);
-    sum = wave_sum(sum) + (limit[i] < cols ? (float)(cols - limit[i]) * masked : 0.f);
-    const float inv = 1.0f / sum;
-    const bool empty = MODE == kLength && limit[i] == 0;  // no keys: a zero row
+    const float masked = masked_weight(mx[i]);
+    if (limit[i] < cols) sum[i] += (float)(cols - limit[i]) * masked;
+    // no keys: a zero row (0 times a finite reciprocal)
+    const float d = MODE == kLength && limit[i] == 0 ? 1.0f : sum[i], inv = 1.0f / d;
 #pragma unroll
     for (int n = 0; n < NP; ++n) {
       const int c = c0 + 256 * n;
-      f32x4 v;
+      f32x4 v = x[i][n];
+      if (masked != 0.f && limit[i] > 0) {  // wave-uniform, see masked_weight
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[e] = empty ? 0.f : divide(c + e < limit[i] ? x[i][n][e] : masked, sum, inv);
-      if (c < cols) store_piece(dst, c, cols, v);
+        for (int e = 0; e < 4; ++e) v[e] = c + e < limit[i] ? v[e] : masked;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = divide(v[e], d, inv);
+      if (c < cols) {
+        if constexpr (WHOLE)
+          *reinterpret_cast<f32x4u*>(dst + c) = v;
+        else
+          store_piece(dst, c, cols, v);
+      }
     }
   }
 }
@@ -472,9 +519,10 @@ hipError_t launch_softmax(float* out, const float* in, long long rows, int cols,
         out, in, (unsigned)rows, cols, S, scale, lens, H);
   else
     with_row_shape(rows, cols, [&](auto np, auto rpw) {
-      softmax_rows_reg_kernel<MODE, np(), rpw()>
-          <<<row_blocks((rows + rpw() - 1) / rpw()), 64 * kRowsPerBlock, 0, stream>>>(
-              out, in, (unsigned)rows, cols, S, scale, lens, H);
+      auto kernel = cols % 4 == 0 ? softmax_rows_reg_kernel<MODE, np(), rpw(), true>
+                                  : softmax_rows_reg_kernel<MODE, np(), rpw(), false>;
+      kernel<<<row_blocks((rows + rpw() - 1) / rpw()), 64 * kRowsPerBlock, 0, stream>>>(
+          out, in, (unsigned)rows, cols, S, scale, lens, H);
     });
   return hipGetLastError();
 }

@@ -79,10 +79,10 @@ def test_causal_rows(gpu, S, BH):
     assert torch.equal(dropped, probs)
 
 
-def test_rows_at_the_mask_value(gpu):
+@pytest.mark.parametrize("S", [70, 72])
+def test_rows_at_the_mask_value(gpu, S):
     """Visible scores at and below the mask's -1e9: the masked columns then carry weight, as in
     the reference's fill-then-softmax."""
-    S = 70
     s = torch.full((1, S, S), -1e9, device="cuda")
     s[0, 5] = -2e9
     s[0, 6] = float("-inf")
@@ -94,6 +94,23 @@ def test_rows_at_the_mask_value(gpu):
     want = torch.zeros(S, device="cuda")
     want[7:] = 1.0 / (S - 7)
     assert torch.allclose(s[0, 6], want, rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("cols", [255, 256, 1025])
+def test_rows_of_special_values(gpu, cols):
+    """A NaN, an infinity or nothing but -inf makes its own row NaN and no other (rows share a
+    wave); a -inf among finite scores weighs nothing. Tolerance as for the plain rows."""
+    rows = 16387
+    x = _normal((rows, cols), 40, 3.0)
+    for r, value in ((1, float("nan")), (6, float("inf")), (16384, float("-inf"))):
+        x[r, cols // 2] = value
+    x[10] = float("-inf")
+    out = torch.empty_like(x)
+    A.softmax(out, x, rows, cols)
+    p = torch.softmax(x.double(), -1)
+    assert torch.equal(out.isnan(), p.isnan())
+    assert (out.double() - p).nan_to_num().abs().max().item() <= 1e-6
+    assert out[16384, cols // 2].item() == 0.0
 
 
 def test_length_rows(gpu):
