@@ -441,14 +441,19 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
 constexpr int kQW = 32;  // queries per wave
 
 // One 32-key chunk (tile keys 32*kb ..) against the wave's 32 queries. Register 8j+e of lane
-// half hi holds tile key 32kb + 16j + 8hi + e. With dropout (DROP), dS = P (dP * f - delta)
-// with f = keep/(1-p) from register 8j+e's uniform in `keep`.
+// half hi holds tile key 32kb + 16j + 8hi + e. dP starts from `ndl`, -delta of the lane's query
+// in every element, so that P dP is dS. VALU and matrix pipe are both ~65% busy here, at a clock
+// of 1.75 GHz: without the 16 subtractions dQ takes 284 us for 295 at [96, 4096, 64], 47.9 for
+// 49.6 at [192, 1024, 64] (with a third tile buffer and loads two tiles ahead: 286 and 48.7; K^T
+// read before the exponentials spills). With dropout (DROP), dS = P (dP * f - delta), f =
+// keep/(1-p) from register 8j+e's uniform in `keep`: dP from zero there, as the 16 registers held
+// across the loop cost that kernel more (96 x 1024: backward 88 -> 92.5).
 template <int D, bool DROP>
 __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
                                          const bf16x8 (&qop)[D / 16],
                                          const bf16x8 (&doop)[D / 16], const bf16* sk,
                                          const bf16* sv, int kb, int qrow_minus_k0, float lse2,
-                                         float dlt, int lane, float scale_log2,
+                                         const f32x16& ndl, int lane, float scale_log2,
                                          const KeepWords16& keep, const DropParams& dr) {
   constexpr int DS = D / 16, DB = D / 32;
   const int l32 = lane & 31, hi = lane >> 5;
@@ -466,7 +471,7 @@ __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
   float pr[16];
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) {
-    dp = mfma32(va[ds], doop[ds], dp);
+    dp = mfma32(va[ds], doop[ds], !DROP && ds == 0 ? ndl : dp);
 #pragma unroll
     for (int i = ds * (16 / DS); i < (ds + 1) * (16 / DS); ++i)
       pr[i] = fast_exp2(fmaf(s[i], scale_log2, -lse2));
@@ -489,9 +494,9 @@ __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
         const int e = 2 * e2 + h;
         const float p = pr[8 * j + e];
         if constexpr (DROP)
-          d[h] = p * fmaf(dp[8 * j + e], keep_factor(keep, 8 * j + e, dr), -dlt);
+          d[h] = p * fmaf(dp[8 * j + e], keep_factor(keep, 8 * j + e, dr), ndl[0]);
         else
-          d[h] = p * (dp[8 * j + e] - dlt);
+          d[h] = p * dp[8 * j + e];
       }
       w[e2] = pack_bf16x2(d[0], d[1]);
     }
@@ -580,6 +585,9 @@ __device__ __forceinline__ void dq_workgroup(const BwdArgs& a, int bh, int qblk,
       dpart += bf16_lo(g[w]) * bf16_lo(o[w]) + bf16_hi(g[w]) * bf16_hi(o[w]);
   }
   const float dlt = sum_halves(dpart);
+  f32x16 ndl;  // what dP starts from
+#pragma unroll
+  for (int i = 0; i < 16; ++i) ndl[i] = -dlt;
   if (WRITE_DELTA && hi == 0 && qrow < S && sub == 0) delta[(size_t)bh * S + qrow] = dlt;
 
   auto tile = [&](int t, const bf16* ck, const bf16* cv, bf16* nk, bf16* nv) {
@@ -596,7 +604,7 @@ __device__ __forceinline__ void dq_workgroup(const BwdArgs& a, int bh, int qblk,
         KeepWords16 keep = {};
         if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qrow, klo, hi);
         // some key after some query: mask
-        dq_chunk<D, DROP>(klo + 31 > q0, dqacc, qop, doop, ck, cv, kb, qrow - k0, lse2, dlt,
+        dq_chunk<D, DROP>(klo + 31 > q0, dqacc, qop, doop, ck, cv, kb, qrow - k0, lse2, ndl,
                           lane, scale_log2, keep, dr);
       }
     }
@@ -741,6 +749,7 @@ hipError_t launch_bwd_bf16(bf16* dq, bf16* dk, bf16* dv, float* delta, const bf1
                            const bf16* v, int BH, int S, int D, float scale,
                            const AttnLayout& layout, hipStream_t stream, int phases,
                            const Dropout* drop) {
+  if (drop != nullptr && drop->p == 0.f) drop = nullptr;  // nothing to draw: the plain kernels
   if (D == 64)
     return launch_bwd_bf16_t<64>(dq, dk, dv, delta, dout, out, lse, q, k, v, BH, S, scale,
                                  layout, stream, phases, drop);
