@@ -637,9 +637,9 @@ __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(cons
 }
 
 // ---------------------------------------------------------------- both in one launch
-// Grid (BH, key blocks + query blocks): dK/dV workgroups first (the longer chains), then the dQ
-// ones. OWN_DELTA: the dK/dV workgroups compute delta of their rows themselves (up to
-// kOwnDeltaMaxS of them) and the dQ workgroups write it; otherwise a pass before has.
+// Grid (BH, blocks, 2): dK/dV workgroups first (z = 0, the longer chains), then the dQ ones.
+// OWN_DELTA: the dK/dV workgroups compute delta of their rows themselves (up to kOwnDeltaMaxS of
+// them) and the dQ workgroups write it; otherwise a pass before has.
 constexpr int kOwnDeltaMaxS = 1024;
 template <int D, bool STRIDED, bool DROP, int KS, bool OWN_DELTA>
 __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocksNoDrop) void bwd_bf16_kernel(
@@ -647,11 +647,12 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
   __shared__ BwdTiles<D> tiles;
   __shared__ BwdStats stats;
   __shared__ float own_delta[OWN_DELTA ? kOwnDeltaMaxS : 1];
-  const int n = gridDim.y / 2, y = blockIdx.y;  // as many key blocks as query blocks
-  if (y < n)
-    dkdv_workgroup<D, STRIDED, DROP, KS, OWN_DELTA>(a, blockIdx.x, y, tiles, stats, own_delta);
+  if (blockIdx.z == 0)
+    dkdv_workgroup<D, STRIDED, DROP, KS, OWN_DELTA>(a, blockIdx.x, blockIdx.y, tiles, stats,
+                                                    own_delta);
   else
-    dq_workgroup<D, STRIDED, DROP, KS, OWN_DELTA>(a, blockIdx.x, 2 * n - 1 - y, tiles);
+    dq_workgroup<D, STRIDED, DROP, KS, OWN_DELTA>(a, blockIdx.x, gridDim.y - 1 - blockIdx.y,
+                                                  tiles);
 }
 
 // How a backward is launched: dQ, then dK/dV (kSeparate); both in one launch with delta
@@ -721,10 +722,10 @@ hipError_t launch_bwd_bf16_t(bf16* dq, bf16* dk, bf16* dv, float* delta, const b
   with_shape(ks, drop != nullptr, !contiguous, [&](auto strided, auto dropped, auto w) {
     if (plan.how == kOneOwnDelta)
       bwd_bf16_kernel<D, strided(), dropped(), w(), true>
-          <<<dim3(BH, 2 * blocks), 64 * kWaves, 0, stream>>>(args);
+          <<<dim3(BH, blocks, 2), 64 * kWaves, 0, stream>>>(args);
     else if (plan.how == kOneAfterDelta)
       bwd_bf16_kernel<D, strided(), dropped(), w(), false>
-          <<<dim3(BH, 2 * blocks), 64 * kWaves, 0, stream>>>(args);
+          <<<dim3(BH, blocks, 2), 64 * kWaves, 0, stream>>>(args);
     if (plan.how != kSeparate) {
       e = hipGetLastError();
       return;

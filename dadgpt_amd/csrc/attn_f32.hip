@@ -18,8 +18,9 @@
 //           three bf16 planes each in the bf16 kernels' swizzled layout, read with
 //           ds_read_b128 (K rows) and ds_read_b64_tr_b16 (V^T);
 //  dK/dV    a wave owns 32 keys (lane l holds key l % 32) and walks the later query chunks:
-//           S = Q K^T and dP = dO V^T with K and V in registers (split once), Q and dO as bf16
-//           planes, P and dS in registers, dV^T += dO^T P and dK^T += Q^T dS (no atomics);
+//           S = Q K^T and dP = dO V^T with K and V split once (in registers; at d_head 64 V's two
+//           lower planes in LDS), Q and dO as bf16 planes, P and dS in registers, dV^T += dO^T P
+//           and dK^T += Q^T dS (no atomics);
 //  dQ       a wave owns 32 queries again: S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T, with
 //           Q and dO split once and K, V as bf16 planes;
 //  delta    rowsum(dO * O), computed by the backward's workgroups or, for long rows, by a pass of
@@ -836,8 +837,8 @@ __device__ __forceinline__ void dq_f32_workgroup(const F32BwdArgs& a, int bh, in
   store_rows_t<D>(dq + base, q0, S, acc, 1.0f, slot, lane);
 }
 
-// The backward is one launch: grid (BH, key blocks + query blocks), dK/dV workgroups first (the
-// longer chains), then the dQ ones, which fill the CUs as those run out. As two launches, each
+// The backward is one launch: grid (BH, blocks, 2), dK/dV workgroups first (z = 0, the longer
+// chains), then the dQ ones, which fill the CUs as those run out. As two launches, each
 // with its own start, end and half-idle last round (B4 H12 S1024 / B1 H24 S1024 / B16 H12 S256,
 // us): 158 -> 143, 140 -> 86, 68 -> 55; where the CUs are full anyway (B16 H12 S1024) 532 -> 527.
 // OWN_DELTA: both kinds compute delta themselves, which saves the small grids a launch (4 x 64:
@@ -849,11 +850,10 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void bwd_f32_ker
     const F32BwdArgs a) {
   __shared__ F32BwdShared<D, KS> sm;
   __shared__ float own_delta[OWN_DELTA ? kOwnDeltaMaxS : 1];
-  const int n = gridDim.y / 2, y = blockIdx.y;  // as many key blocks as query blocks
-  if (y < n)
-    dkdv_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, y, sm, own_delta);
+  if (blockIdx.z == 0)
+    dkdv_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, blockIdx.y, sm, own_delta);
   else
-    dq_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, 2 * n - 1 - y, sm);
+    dq_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, gridDim.y - 1 - blockIdx.y, sm);
 }
 
 // Waves per row group. With one, a workgroup walks its chunks four waves wide, two workgroups
@@ -919,7 +919,7 @@ hipError_t bwd_f32_t(float* dq, float* dk, float* dv, float* delta, const float*
         delta, dout, out, rows);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  const dim3 grid(BH, 2 * ((S + kRows - 1) / kRows));
+  const dim3 grid(BH, (S + kRows - 1) / kRows, 2);
   with_f32_shape(bwd_waves_per_group(BH, S), drop != nullptr, [&](auto drop_c, auto ks) {
     constexpr int threads = 64 * kGroups * ks();
     if (own)
