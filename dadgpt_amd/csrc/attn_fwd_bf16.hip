@@ -163,6 +163,14 @@ __device__ __forceinline__ float fwd_exp(bf16x8 (&pb)[2], const f32x16& s, float
   return ls;
 }
 
+// What a row's exponentials are taken against: its running maximum, or 0 while every score it
+// has seen is -inf (then each P is exp2(-inf) = 0, where -inf - (-inf) would make the row NaN for
+// good; a second wave's first chunk may be such keys alone). A NaN maximum stays NaN: compared on
+// the bits, as this file is built assuming no NaNs.
+__device__ __forceinline__ float finite_max(float m) {
+  return __float_as_uint(m) == __float_as_uint(neg_inf()) ? 0.f : m;
+}
+
 // Online softmax of one chunk's scores (masked ones already -inf) and
 // O^T += V^T[:, chunk] P^T.
 //
@@ -198,17 +206,19 @@ __device__ __forceinline__ void fwd_softmax_pv(f32x16 (&s)[NQB], f32x16 (&oacc)[
       float mx = s[i][0];
 #pragma unroll
       for (int r = 1; r < 15; r += 2) mx = fmaxf(fmaxf(mx, s[i][r]), s[i][r + 1]);
-      // every row of a chunk the wave computes has an unmasked key, so mx is finite
+      // every row of a chunk the wave computes has an unmasked key: mx is -inf only if every
+      // score of the row so far is
       mx = max_halves(fmaxf(mx, s[i][15])) * scale_log2;
       // the two lane halves of a row hold different keys of it, and P V sums both against one
       // maximum: the row moves it if either half needs to
       const float mnew = or_halves(need) ? fmaxf(mrun[i], mx) : mrun[i];
-      const float corr = fast_exp2(mrun[i] - mnew);  // 0 on a row's first chunk
+      const float mref = finite_max(mnew);
+      const float corr = fast_exp2(mrun[i] - mref);  // 0 on a row's first chunk
       mrun[i] = mnew;
       lrun[i] *= corr;
 #pragma unroll
       for (int db = 0; db < DB; ++db) oacc[i][db] *= corr;
-      ls = fwd_exp<DROP>(pb[i], s[i], mnew, scale_log2, keep[i], dr);
+      ls = fwd_exp<DROP>(pb[i], s[i], mref, scale_log2, keep[i], dr);
     }
     lrun[i] += ls;
   }
@@ -357,7 +367,8 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
 
   if constexpr (KS == 2) {
     // (m, l, O) of the group's second wave: rescaled to the larger maximum and added. A wave
-    // that saw no chunk of the row has m = -inf and zeros, which get weight 2^-inf = 0.
+    // that saw no chunk of the row, or only scores of -inf, has m = -inf and zeros, which get
+    // weight 2^-inf = 0.
     AccLds* slot = reinterpret_cast<AccLds*>(&sk[0][0]) + grp * DB;
     float* ml = reinterpret_cast<float*>(&smask[0][0]) + grp * 128;
     if (sub == 1) {
@@ -368,7 +379,8 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
     __syncthreads();
     if (sub == 1) return;
     const float m1 = ml[lane], mn = fmaxf(mrun[0], m1);
-    const float a0 = fast_exp2(mrun[0] - mn), a1 = fast_exp2(m1 - mn);
+    const float mref = finite_max(mn);
+    const float a0 = fast_exp2(mrun[0] - mref), a1 = fast_exp2(m1 - mref);
     mrun[0] = mn;
     lrun[0] = lrun[0] * a0 + ml[64 + lane] * a1;
 #pragma unroll

@@ -113,3 +113,41 @@ def test_bf16_dropout_and_strided_shapes(gpu, BH, S):
     g3 = [torch.empty_like(tokens[0]) for _ in range(3)]
     A.flash_attention_backward_bf16_strided(*g3, delta, tokens[3], o3, l3, *tokens[:3], scale)
     close((o3.reshape(BH, S, D), l3, *[x.reshape(BH, S, D) for x in g3]))
+
+
+# (3 slices: two waves per group; 400 slices: one wave per group, at S = 160 in D = 64 and 32)
+@pytest.mark.parametrize("BH,S,D", [(3, 160, 64), (3, 700, 64), (3, 160, 32), (400, 160, 64),
+                                    (400, 160, 32)])
+@pytest.mark.parametrize("first", [0, 32, 64])
+def test_bf16_chunk_of_minus_infinity(gpu, BH, S, D, first):
+    """Scores that overflow to -inf weigh nothing, in the bf16 forward, also where they fill a
+    whole 32-key chunk: the first of the row, the first that a group's second wave sees, or a
+    later one. Rows that see no other key (those up to first + 31, for the first chunk) are left
+    out: they have no defined softmax."""
+    print(f"[case] -inf scores of keys {first}..{first + 31} BH={BH} S={S} D={D}", flush=True)
+    q, k, v, _ = _inputs(BH, S, D, torch.bfloat16, 3 * S + first)
+    # one column decides: 2^60 x -2^90 is far below fp32's range, 2^60 x 0 adds nothing
+    q[..., 0], k[..., 0] = 2.0 ** 60, 0.0
+    k[:, first:first + 32, 0] = -(2.0 ** 90)
+    scale = A.default_scale(D)
+    runs = [A.attention_forward(q, k, v, scale)]
+    out, lse = torch.empty_like(q), torch.empty((BH, S), device="cuda")
+    A.flash_attention_forward_bf16_dropout(out, lse, q, k, v, BH, S, D, scale, 0.1, 5)
+    x = [t.view(1, BH, S, D).transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v)]
+    o3, l3 = torch.empty_like(x[0]), torch.empty_like(lse)
+    A.flash_attention_forward_bf16_strided(o3, l3, *x, scale)
+    runs.append((o3.reshape(BH, S, D), l3))
+    rows = slice(first + 32 if first == 0 else 0, S)
+    hidden = torch.ones((S, S), dtype=torch.bool, device="cuda").triu(1)
+    hidden[:, first:first + 32] = True
+    heads = [0, BH // 2, BH - 1]
+    q6, k6, v6 = (t[heads].double() for t in (q, k, v))
+    s = torch.bmm(q6, k6.transpose(1, 2).contiguous()) * scale
+    s = s.masked_fill(hidden, float("-inf"))[:, rows]
+    want_lse, want = torch.logsumexp(s, -1), torch.bmm(torch.softmax(s, -1), v6)
+    for o, l in runs:
+        assert torch.isfinite(o[:, rows]).all().item() and torch.isfinite(l[:, rows]).all().item()
+        assert (o[heads][:, rows].double() - want).abs().max().item() <= BF16_TOLS[0]
+        assert (l[heads][:, rows].double() - want_lse).abs().max().item() <= BF16_TOLS[1]
+    assert torch.isfinite(out[:, rows]).all().item()
+    assert (lse[heads][:, rows].double() - want_lse).abs().max().item() <= BF16_TOLS[1]
