@@ -697,9 +697,19 @@ hipError_t launch_bwd_bf16_t(bf16* dq, bf16* dk, bf16* dv, float* delta, const b
   hipError_t e = hipSuccess;
   const bool contiguous = is_contiguous(L, S, D);
   const DropParams dr = drop_params(drop);  // dropout: contiguous layout only (caller checks)
-  const BwdPlan plan = phases == kBwdAll
-                           ? bwd_plan(BH, S, D, drop != nullptr)
-                           : BwdPlan{kSeparate, waves_per_group(BH, S, D, drop != nullptr)};
+  auto span = [&](const bf16* p, int t) {  // tensor t's extent
+    const HeadStrides& h = L.t[t];
+    const size_t batches = BH / L.n_heads, heads = L.n_heads;
+    return Span{p, 2 * ((batches - 1) * h.batch + (heads - 1) * h.head + (size_t)(S - 1) * h.row + D)};
+  };
+  // The phase calls, and a backward in place (dk = k, dv = v, or any gradient = out), run dQ first,
+  // then dK/dV.
+  const bool separate =
+      phases != kBwdAll || in_place({span(dq, kTDQ), span(dk, kTDK), span(dv, kTDV)},
+                                    {span(q, kTQ), span(k, kTK), span(v, kTV), span(dout, kTDO),
+                                     span(out, kTO)});
+  const BwdPlan plan = separate ? BwdPlan{kSeparate, waves_per_group(BH, S, D, drop != nullptr)}
+                                : bwd_plan(BH, S, D, drop != nullptr);
   if ((phases & kBwdDelta) || plan.how == kOneAfterDelta) {
     const long long rows = (long long)BH * S;
     const int row_blocks = (S + 31) / 32;

@@ -542,6 +542,7 @@ struct F32BwdArgs {
   int S;
   float scale;
   DropParams dr;
+  int first;  // what the workgroups of grid z = 0 compute: 0 dK/dV, 1 dQ
 };
 // LDS of a workgroup: the tiles, and per query row of a dK/dV tile lse and delta * scale.
 template <int D, int KS>
@@ -843,14 +844,15 @@ __device__ __forceinline__ void dq_f32_workgroup(const F32BwdArgs& a, int bh, in
 // us): 158 -> 143, 140 -> 86, 68 -> 55; where the CUs are full anyway (B16 H12 S1024) 532 -> 527.
 // OWN_DELTA: both kinds compute delta themselves, which saves the small grids a launch (4 x 64:
 // 10.0 -> 8.3 us); past kOwnDeltaMaxS rows, where dK/dV would read O and dO once per key block
-// more, a pass before does it (96 x 1024: 268 against 263.5 us).
+// more, a pass before does it (96 x 1024: 268 against 263.5 us). A backward in place (dq = q or
+// dout, or any gradient = out) runs as the delta pass, dK/dV and dQ, one after the other.
 constexpr int kOwnDeltaMaxS = 512;
 template <int D, bool DROP, int KS, bool OWN_DELTA>
 __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void bwd_f32_kernel(
     const F32BwdArgs a) {
   __shared__ F32BwdShared<D, KS> sm;
   __shared__ float own_delta[OWN_DELTA ? kOwnDeltaMaxS : 1];
-  if (blockIdx.z == 0)
+  if (a.first + blockIdx.z == 0)
     dkdv_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, blockIdx.y, sm, own_delta);
   else
     dq_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, gridDim.y - 1 - blockIdx.y, sm);
@@ -910,8 +912,11 @@ hipError_t bwd_f32_t(float* dq, float* dk, float* dv, float* delta, const float*
                      const float* out, const float* lse, const float* q, const float* k,
                      const float* v, int BH, int S, float scale, hipStream_t stream,
                      const Dropout* drop) {
-  const F32BwdArgs args{dq, dk, dv, delta, q, k, v, dout, out, lse, S, scale, drop_params(drop)};
-  const bool own = S <= kOwnDeltaMaxS;
+  F32BwdArgs args{dq, dk, dv, delta, q, k, v, dout, out, lse, S, scale, drop_params(drop), 0};
+  auto span = [&](const float* p) { return Span{p, (size_t)BH * S * D * sizeof(float)}; };
+  const bool separate = in_place({span(dq), span(dk), span(dv)},
+                                 {span(q), span(k), span(v), span(dout), span(out)});
+  const bool own = S <= kOwnDeltaMaxS && !separate;
   hipError_t e = hipSuccess;
   if (!own) {
     const long long rows = (long long)BH * S, blocks = (rows * (D / 4) + 255) / 256;
@@ -919,13 +924,17 @@ hipError_t bwd_f32_t(float* dq, float* dk, float* dv, float* delta, const float*
         delta, dout, out, rows);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  const dim3 grid(BH, (S + kRows - 1) / kRows, 2);
+  const dim3 grid(BH, (S + kRows - 1) / kRows, separate ? 1 : 2);
   with_f32_shape(bwd_waves_per_group(BH, S), drop != nullptr, [&](auto drop_c, auto ks) {
     constexpr int threads = 64 * kGroups * ks();
     if (own)
       bwd_f32_kernel<D, drop_c(), ks(), true><<<grid, threads, 0, stream>>>(args);
     else
       bwd_f32_kernel<D, drop_c(), ks(), false><<<grid, threads, 0, stream>>>(args);
+    e = hipGetLastError();
+    if (!separate || e != hipSuccess) return;
+    args.first = 1;
+    bwd_f32_kernel<D, drop_c(), ks(), false><<<grid, threads, 0, stream>>>(args);
     e = hipGetLastError();
   });
   return e;

@@ -7,6 +7,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <initializer_list>
+
 namespace dadgpt {
 
 typedef __bf16 bf16;
@@ -44,6 +46,26 @@ inline bool is_contiguous(const AttnLayout& L, int S, int D) {
       return false;
     }
   return true;
+}
+
+// Whether two buffers share memory (their whole extents: interleaved rows count).
+struct Span {
+  const void* p;
+  size_t bytes;
+};
+inline bool overlap(const Span& a, const Span& b) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a.p), y = reinterpret_cast<uintptr_t>(b.p);
+  return x < y + b.bytes && y < x + a.bytes;
+}
+// Whether any of a backward's gradients shares memory with what it reads. Each workgroup reads
+// its own rows of some inputs (dK/dV of K and V, dQ of Q, dO and O) before it writes theirs, so
+// a gradient may take such an input's place, but only while the kernels run one after the other:
+// in one launch the other kind's workgroups still read it.
+inline bool in_place(std::initializer_list<Span> gradients, std::initializer_list<Span> inputs) {
+  for (const Span& g : gradients)
+    for (const Span& x : inputs)
+      if (overlap(g, x)) return true;
+  return false;
 }
 
 // Attention-probability dropout of a call: rate p in [0, 1) and the generator's seed (the

@@ -15,6 +15,10 @@
  *    (cuda/attention.cu:71).
  *  - bf16 tensors are passed as uint16_t* holding IEEE bfloat16 bit patterns.
  *  - Outputs are overwritten, never accumulated (cuda/gpu_ops.cuh:118).
+ *  - Outputs must not overlap each other or the inputs, except where an entry point says so,
+ *    and that a flash backward may write a gradient over an input that only the workgroup of
+ *    those rows reads: bf16 dk = k, dv = v, and one of dq, dk, dv = out; fp32 dq = q or dq =
+ *    dout, and one of dq, dk, dv = out. Its kernels then run one after the other.
  *  - Arguments are validated on the host before any HIP call; a failing call returns a
  *    nonzero dadgpt_status and dadgpt_last_error() describes it (thread-local). Launch errors
  *    (hipGetLastError) map to DADGPT_ERR_HIP; asynchronous faults surface at the caller's

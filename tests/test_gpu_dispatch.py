@@ -151,3 +151,56 @@ def test_bf16_chunk_of_minus_infinity(gpu, BH, S, D, first):
         assert (l[heads][:, rows].double() - want_lse).abs().max().item() <= BF16_TOLS[1]
     assert torch.isfinite(out[:, rows]).all().item()
     assert (lse[heads][:, rows].double() - want_lse).abs().max().item() <= BF16_TOLS[1]
+
+
+@pytest.mark.parametrize("BH,S,D", [(4, 70, 64), (24, 300, 32), (24, 1024, 64), (3, 1030, 64),
+                                    (160, 520, 64)])
+def test_bf16_backward_in_place(gpu, BH, S, D):
+    """Gradients that take the place of an input which only their own workgroup reads (dk = k,
+    dv = v, dq = out, and dk or dv = out): dQ and dK/dV then run one after the other, as the phase
+    calls do, bit for bit; contiguous and token-major."""
+    print(f"[case] bf16 backward in place BH={BH} S={S} D={D}", flush=True)
+    q, k, v, dout = _inputs(BH, S, D, torch.bfloat16, S)
+    scale = A.default_scale(D)
+    out, lse = A.attention_forward(q, k, v, scale)
+    delta = torch.empty_like(lse)
+    want = [torch.empty_like(q) for _ in range(3)]
+    for phase in (1, 2):
+        A.flash_attention_backward_bf16_phase(phase, *want, delta, dout, out, lse, q, k, v, BH, S,
+                                              D, scale)
+    for places in (("out", "k", "v"), ("q2", "out", "v"), ("q2", "k", "out"), ("q2", "k2", "v")):
+        t = {"q": q.clone(), "k": k.clone(), "v": v.clone(), "out": out.clone(),
+             "q2": torch.empty_like(q), "k2": torch.empty_like(q)}
+        A.flash_attention_backward_bf16(t[places[0]], t[places[1]], t[places[2]], delta, dout,
+                                        t["out"], lse, t["q"], t["k"], t["v"], BH, S, D, scale)
+        for x, y in zip(places, want):
+            assert torch.equal(t[x], y), places
+    tok = {n: x.view(1, BH, S, D).transpose(1, 2).contiguous().transpose(1, 2)
+           for n, x in (("q", q), ("k", k), ("v", v), ("out", out), ("dout", dout))}
+    A.flash_attention_backward_bf16_strided(tok["out"], tok["k"], tok["v"], delta, tok["dout"],
+                                            tok["out"], lse, tok["q"], tok["k"], tok["v"], scale)
+    for x, y in zip(("out", "k", "v"), want):
+        assert torch.equal(tok[x].reshape(BH, S, D), y), x
+
+
+@pytest.mark.parametrize("BH,S,D", [(4, 70, 64), (24, 300, 32), (24, 600, 64), (160, 300, 64)])
+@pytest.mark.parametrize("p", [0.0, 0.2])
+def test_f32_backward_in_place(gpu, BH, S, D, p):
+    """As above in fp32, where the delta pass, dK/dV and dQ run in this order: dq = q, dq = dout,
+    and any gradient = out. Up to 512 rows delta is otherwise summed in another order, so the
+    gradients agree to the fp32 bound."""
+    print(f"[case] fp32 backward in place BH={BH} S={S} D={D} p={p}", flush=True)
+    q, k, v, dout = _inputs(BH, S, D, torch.float32, S)
+    shape = (BH, S, D, A.default_scale(D), p, 11)
+    out, lse = torch.empty_like(q), torch.empty((BH, S), device="cuda")
+    A.flash_attention_forward_dropout(out, lse, q, k, v, *shape)
+    delta = torch.empty_like(lse)
+    want = [torch.empty_like(q) for _ in range(3)]
+    A.flash_attention_backward_dropout(*want, delta, dout, out, lse, q, k, v, *shape)
+    for places in (("q", "out", "v2"), ("dout", "k2", "out"), ("out", "k2", "v2")):
+        t = {"q": q.clone(), "dout": dout.clone(), "out": out.clone(),
+             "k2": torch.empty_like(q), "v2": torch.empty_like(q)}
+        A.flash_attention_backward_dropout(t[places[0]], t[places[1]], t[places[2]], delta,
+                                           t["dout"], t["out"], lse, t["q"], k, v, *shape)
+        for x, y in zip(places, want):
+            assert (t[x] - y).abs().max().item() <= 1e-5, places
