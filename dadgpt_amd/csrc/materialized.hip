@@ -93,6 +93,13 @@ __device__ __forceinline__ f32x4 load_piece(const float* row, int c, int cols) {
     if (c + e < cols) v[e] = row[c + e];
   return v;
 }
+// load_piece and store_piece of rows without a crossing piece (WHOLE: the columns are a multiple
+// of four), or of any row.
+template <bool WHOLE>
+__device__ __forceinline__ f32x4 load_cols(const float* row, int c, int cols) {
+  if constexpr (WHOLE) return *reinterpret_cast<const f32x4u*>(row + c);
+  return load_piece(row, c, cols);
+}
 __device__ __forceinline__ void store_piece(float* row, int c, int cols, const f32x4& v) {
   if (c + 4 <= cols) {
     *reinterpret_cast<f32x4u*>(row + c) = v;
@@ -101,6 +108,14 @@ __device__ __forceinline__ void store_piece(float* row, int c, int cols, const f
 #pragma unroll
   for (int e = 0; e < 3; ++e)
     if (c + e < cols) row[c + e] = v[e];
+}
+
+template <bool WHOLE>
+__device__ __forceinline__ void store_cols(float* row, int c, int cols, const f32x4& v) {
+  if constexpr (WHOLE)
+    *reinterpret_cast<f32x4u*>(row + c) = v;
+  else
+    store_piece(row, c, cols, v);
 }
 
 // What a softmax row sees of its input: the raw value (kPlain), scale then causal mask
@@ -220,12 +235,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_reg_kernel(
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = divide(v[e], d, inv);
-      if (c < cols) {
-        if constexpr (WHOLE)
-          *reinterpret_cast<f32x4u*>(dst + c) = v;
-        else
-          store_piece(dst, c, cols, v);
-      }
+      if (c < cols) store_cols<WHOLE>(dst, c, cols, v);
     }
   }
 }
@@ -369,27 +379,35 @@ struct Group8 {
   float v[8];
   __device__ __forceinline__ float& operator[](int e) { return v[e]; }
 };
+// WHOLE: the columns are a multiple of eight, so every group is whole.
+template <bool WHOLE>
 __device__ __forceinline__ Group8 load_group(const float* row, int c, int cols) {
-  const f32x4 a = load_piece(row, c, cols), b = load_piece(row, c + 4, cols);
+  f32x4 a, b;
+  if constexpr (WHOLE)
+    a = load_cols<true>(row, c, cols), b = load_cols<true>(row, c + 4, cols);
+  else
+    a = load_piece(row, c, cols), b = load_piece(row, c + 4, cols);
   return Group8{{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}};
 }
+template <bool WHOLE>
 __device__ __forceinline__ void store_group(float* row, int c, int cols, Group8& g) {
-  store_piece(row, c, cols, f32x4{g[0], g[1], g[2], g[3]});
-  if (c + 4 < cols) store_piece(row, c + 4, cols, f32x4{g[4], g[5], g[6], g[7]});
+  store_cols<WHOLE>(row, c, cols, f32x4{g[0], g[1], g[2], g[3]});
+  if (WHOLE || c + 4 < cols) store_cols<WHOLE>(row, c + 4, cols, f32x4{g[4], g[5], g[6], g[7]});
 }
 
 // out = p * keep / (1 - p_drop) (the reference's gpu_dropout_forward, cuda/gpu_ops.cu:712-733,
 // with this mask). out may be p.
+template <bool WHOLE>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void dropout_rows_kernel(
     float* out, const float* p, unsigned rows, int cols, DropParams dr) {
   const unsigned r = wave_row0();
   if (r >= rows) return;
   for (int c = 8 * (threadIdx.x & 63); c < cols; c += 512) {
-    Group8 g = load_group(p + (size_t)r * cols, c, cols);
+    Group8 g = load_group<WHOLE>(p + (size_t)r * cols, c, cols);
     const uint32_t bits = keep8(dr, (uint64_t)r, (uint32_t)c >> 3);
 #pragma unroll
     for (int e = 0; e < 8; ++e) g[e] *= keep_factor(bits, e, dr.scale);
-    store_group(out + (size_t)r * cols, c, cols, g);
+    store_group<WHOLE>(out + (size_t)r * cols, c, cols, g);
   }
 }
 
@@ -398,7 +416,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void dropout_rows_kernel(
 // against the undropped P, zero past the causal diagonal, times scale. ds may be dpd. NG > 0:
 // rows of at most 512 NG columns, read and their keep bits generated once; NG = 0: any length,
 // both done again for the second pass.
-template <int NG>
+template <int NG, bool WHOLE>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void attn_probs_backward_dropout_kernel(
     float* ds, const float* dpd, const float* __restrict__ p, unsigned rows, int S,
     float scale, DropParams dr) {
@@ -408,7 +426,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void attn_probs_backward_dropou
   const float *gr = dpd + (size_t)r * S, *pr = p + (size_t)r * S;
   const int limit = (int)(r % (unsigned)S) + 1;
   auto undrop = [&](int c) {  // dP of the undropped probabilities
-    Group8 g = load_group(gr, c, S);
+    Group8 g = load_group<WHOLE>(gr, c, S);
     const uint32_t bits = keep8(dr, (uint64_t)r, (uint32_t)c >> 3);
 #pragma unroll
     for (int e = 0; e < 8; ++e) g[e] *= keep_factor(bits, e, dr.scale);
@@ -422,7 +440,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void attn_probs_backward_dropou
   auto finish = [&](int c, Group8& g, Group8& q, float dot) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) g[e] = c + e < limit ? q[e] * (g[e] - dot) * scale : 0.f;
-    store_group(ds + (size_t)r * S, c, S, g);
+    store_group<WHOLE>(ds + (size_t)r * S, c, S, g);
   };
   float dot = 0.f;
   if constexpr (NG > 0) {
@@ -430,7 +448,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void attn_probs_backward_dropou
 #pragma unroll
     for (int n = 0; n < NG; ++n)
       if (c0 + 512 * n < S) {
-        q[n] = load_group(pr, c0 + 512 * n, S);
+        q[n] = load_group<WHOLE>(pr, c0 + 512 * n, S);
         g[n] = undrop(c0 + 512 * n);
         dot = row_dot(g[n], q[n], dot);
       }
@@ -440,12 +458,12 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void attn_probs_backward_dropou
       if (c0 + 512 * n < S) finish(c0 + 512 * n, g[n], q[n], dot);
   } else {
     for (int c = c0; c < S; c += 512) {
-      Group8 g = undrop(c), q = load_group(pr, c, S);
+      Group8 g = undrop(c), q = load_group<WHOLE>(pr, c, S);
       dot = row_dot(g, q, dot);
     }
     dot = wave_sum(dot);
     for (int c = c0; c < S; c += 512) {
-      Group8 g = undrop(c), q = load_group(pr, c, S);
+      Group8 g = undrop(c), q = load_group<WHOLE>(pr, c, S);
       finish(c, g, q, dot);
     }
   }
@@ -585,7 +603,8 @@ hipError_t launch_attention_dropout(float* out, const float* p, int BH, int S,
                                    const Dropout& drop, hipStream_t stream) {
   const long long rows = (long long)BH * S;
   const DropParams dr = drop_params(&drop);
-  dropout_rows_kernel<<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(out, p, (unsigned)rows, S, dr);
+  auto kernel = S % 8 == 0 ? dropout_rows_kernel<true> : dropout_rows_kernel<false>;
+  kernel<<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(out, p, (unsigned)rows, S, dr);
   return hipGetLastError();
 }
 
@@ -594,15 +613,17 @@ hipError_t launch_attention_probs_backward_dropout(float* ds, const float* dpd, 
                                                    const Dropout& drop, hipStream_t stream) {
   const long long rows = (long long)BH * S;
   const DropParams dr = drop_params(&drop);
-  if (S <= 512)
-    attn_probs_backward_dropout_kernel<1><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-        ds, dpd, p, (unsigned)rows, S, scale, dr);
-  else if (S <= 1024)
-    attn_probs_backward_dropout_kernel<2><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-        ds, dpd, p, (unsigned)rows, S, scale, dr);
+  auto run = [&](auto whole) {
+    auto kernel = S <= 512    ? attn_probs_backward_dropout_kernel<1, whole()>
+                  : S <= 1024 ? attn_probs_backward_dropout_kernel<2, whole()>
+                              : attn_probs_backward_dropout_kernel<0, whole()>;
+    kernel<<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(ds, dpd, p, (unsigned)rows, S,
+                                                                scale, dr);
+  };
+  if (S % 8 == 0)
+    run(std::true_type{});
   else
-    attn_probs_backward_dropout_kernel<0><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
-        ds, dpd, p, (unsigned)rows, S, scale, dr);
+    run(std::false_type{});
   return hipGetLastError();
 }
 
