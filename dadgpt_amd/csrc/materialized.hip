@@ -241,7 +241,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_reg_kernel(
 }
 
 // Softmax of rows of any length: one row per wave, read again for each reduction.
-template <int MODE>
+template <int MODE, bool WHOLE>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_kernel(
     float* out, const float* in, unsigned rows, int cols, int S,
     float scale, const int* __restrict__ lens, int H) {
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_kernel(
   const int limit = row_limit<MODE>(r, cols, S, lens, H);
   auto visible = [&](auto f) {  // f(piece of scaled values, its first column)
     for (int c = c0; c < limit; c += 256) {
-      f32x4 v = load_piece(src, c, cols);
+      f32x4 v = load_cols<WHOLE>(src, c, cols);
       if constexpr (MODE != kPlain) v *= scale;
       f(v, c);
     }
@@ -278,12 +278,12 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_kernel(
   // in == out is allowed: each lane writes exactly the columns it reads, after reading them
   for (int c = c0; c < cols; c += 256) {
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (c < limit) v = load_piece(src, c, cols);
+    if (c < limit) v = load_cols<WHOLE>(src, c, cols);
     if constexpr (MODE != kPlain) v *= scale;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       v[e] = empty ? 0.f : divide(c + e < limit ? expf(v[e] - mx) : masked, sum, inv);
-    store_piece(dst, c, cols, v);
+    store_cols<WHOLE>(dst, c, cols, v);
   }
 }
 
@@ -291,10 +291,11 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_kernel(
 // reference's operator). Otherwise the attention form: din = g, zero past the causal
 // diagonal, times scale (din may be dout). The sum runs over whole rows, whatever p holds past
 // the diagonal. REG: rows of at most 256 NP columns, RPW rows per wave, each read once;
-// otherwise (NP = RPW = 1) any length, the row read twice.
+// otherwise (NP = RPW = 1) any length, the row read twice. WHOLE (read by the loop only): the
+// columns are a multiple of four.
 // [BH 192, S 256], 3 x 50 MB: 36 us with 4-byte loads in two passes, 24.5 us here
 // (6.1 TB/s).
-template <bool ACCUMULATE, bool REG, int NP, int RPW>
+template <bool ACCUMULATE, bool REG, int NP, int RPW, bool WHOLE>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_backward_rows_kernel(
     float* din, const float* dout, const float* __restrict__ p, unsigned rows, int cols, int S,
     float scale) {
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_backward_rows_kern
     const int limit = ACCUMULATE ? cols : (int)(r % (unsigned)S) + 1;
     float* d = din + (size_t)r * cols;
     f32x4 v;
-    if constexpr (ACCUMULATE) v = load_piece(d, c, cols);
+    if constexpr (ACCUMULATE) v = load_cols<WHOLE>(d, c, cols);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float t = pr[e] * (g[e] - dot);
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_backward_rows_kern
       else
         v[e] = c + e < limit ? t * scale : 0.0f;
     }
-    store_piece(d, c, cols, v);
+    store_cols<WHOLE>(d, c, cols, v);
   };
   if constexpr (REG) {
     f32x4 g[RPW][NP], pr[RPW][NP];
@@ -351,10 +352,10 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_backward_rows_kern
     const float *gr = dout + (size_t)r0 * cols, *prow = p + (size_t)r0 * cols;
     float dot = 0.f;
     for (int c = c0; c < cols; c += 256)
-      dot = row_dot(load_piece(gr, c, cols), load_piece(prow, c, cols), dot);
+      dot = row_dot(load_cols<WHOLE>(gr, c, cols), load_cols<WHOLE>(prow, c, cols), dot);
     dot = wave_sum(dot);
     for (int c = c0; c < cols; c += 256)
-      finish(r0, c, load_piece(gr, c, cols), load_piece(prow, c, cols), dot);
+      finish(r0, c, load_cols<WHOLE>(gr, c, cols), load_cols<WHOLE>(prow, c, cols), dot);
   }
 }
 
@@ -532,15 +533,18 @@ void with_row_shape(long long rows, int cols, F f) {
 template <int MODE>
 hipError_t launch_softmax(float* out, const float* in, long long rows, int cols, int S,
                           float scale, const int* lens, int H, hipStream_t stream) {
-  if (cols < 4 || cols > 256 * kMaxPieces)
-    softmax_rows_kernel<MODE><<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(
+  auto run = [&](auto kernel, int rpw) {
+    kernel<<<row_blocks((rows + rpw - 1) / rpw), 64 * kRowsPerBlock, 0, stream>>>(
         out, in, (unsigned)rows, cols, S, scale, lens, H);
+  };
+  const bool whole = cols % 4 == 0;
+  if (cols < 4 || cols > 256 * kMaxPieces)
+    run(whole ? softmax_rows_kernel<MODE, true> : softmax_rows_kernel<MODE, false>, 1);
   else
     with_row_shape(rows, cols, [&](auto np, auto rpw) {
-      auto kernel = cols % 4 == 0 ? softmax_rows_reg_kernel<MODE, np(), rpw(), true>
-                                  : softmax_rows_reg_kernel<MODE, np(), rpw(), false>;
-      kernel<<<row_blocks((rows + rpw() - 1) / rpw()), 64 * kRowsPerBlock, 0, stream>>>(
-          out, in, (unsigned)rows, cols, S, scale, lens, H);
+      run(whole ? softmax_rows_reg_kernel<MODE, np(), rpw(), true>
+                : softmax_rows_reg_kernel<MODE, np(), rpw(), false>,
+          rpw());
     });
   return hipGetLastError();
 }
@@ -548,14 +552,17 @@ hipError_t launch_softmax(float* out, const float* in, long long rows, int cols,
 template <bool ACCUMULATE>
 hipError_t launch_softmax_backward(float* din, const float* dout, const float* p, long long rows,
                                    int cols, int S, float scale, hipStream_t stream) {
+  auto run = [&](auto kernel, int rpw) {
+    kernel<<<row_blocks((rows + rpw - 1) / rpw), 64 * kRowsPerBlock, 0, stream>>>(
+        din, dout, p, (unsigned)rows, cols, S, scale);
+  };
   if (cols < 4 || cols > 256 * kMaxPieces)
-    softmax_backward_rows_kernel<ACCUMULATE, false, 1, 1>
-        <<<row_blocks(rows), 64 * kRowsPerBlock, 0, stream>>>(din, dout, p, (unsigned)rows, cols, S, scale);
+    run(cols % 4 == 0 ? softmax_backward_rows_kernel<ACCUMULATE, false, 1, 1, true>
+                      : softmax_backward_rows_kernel<ACCUMULATE, false, 1, 1, false>,
+        1);
   else
     with_row_shape(rows, cols, [&](auto np, auto rpw) {
-      softmax_backward_rows_kernel<ACCUMULATE, true, np(), rpw()>
-          <<<row_blocks((rows + rpw() - 1) / rpw()), 64 * kRowsPerBlock, 0, stream>>>(
-              din, dout, p, (unsigned)rows, cols, S, scale);
+      run(softmax_backward_rows_kernel<ACCUMULATE, true, np(), rpw(), false>, rpw());
     });
   return hipGetLastError();
 }
