@@ -1,6 +1,6 @@
-"""The row kernels of the materialized path at the edges of their shapes: rows that end inside
-a 16-byte piece, one row and several per wave, register rows (4 to 1,024 columns) and looped ones,
-against float64."""
+"""The row kernels of the materialized path at the edges of their shapes: rows of one column a lane
+(up to 64) and of 16-byte pieces, rows that end inside a piece, one row and several per wave,
+register rows (up to 1,024 columns) and looped ones, against float64."""
 import numpy as np
 import pytest
 import torch
@@ -9,11 +9,11 @@ from dadgpt_amd import attention as A
 
 pytestmark = pytest.mark.gpu
 
-# (columns, rows): 16-byte remainders 0-3, both sides of 256, 512 and 1,024 columns, and row
+# (columns, rows): 16-byte remainders 0-3, both sides of 64, 256, 512 and 1,024 columns, and row
 # counts that give one, two and four rows per wave with a last wave that is not full.
 SHAPES = [(1, 5), (3, 4099), (4, 9), (5, 16387), (66, 8193), (255, 16389), (256, 16384),
           (257, 8195), (511, 8193), (512, 4097), (513, 33), (1021, 7), (1024, 5), (1025, 6),
-          (2047, 3)]
+          (2047, 3), (2048, 3), (2, 8193), (31, 4097), (63, 16387), (64, 33), (65, 16385)]
 
 
 def _normal(shape, seed, scale=1.0):
@@ -44,7 +44,7 @@ def test_plain_rows(gpu, cols, rows):
 
 @pytest.mark.parametrize("S,BH", [(1, 3), (3, 5), (4, 2), (63, 70), (64, 260), (130, 127),
                                   (256, 65), (257, 32), (509, 17), (512, 9), (515, 2), (1023, 1),
-                                  (1030, 1)])
+                                  (1030, 1), (31, 260), (65, 127), (1032, 1)])
 def test_causal_rows(gpu, S, BH):
     """attention_probs and attention_probs_backward, without and with dropout (p = 0, whose
     factors are exactly 1, must give the plain result's values). What lies past the diagonal of
@@ -79,7 +79,7 @@ def test_causal_rows(gpu, S, BH):
     assert torch.equal(dropped, probs)
 
 
-@pytest.mark.parametrize("S", [70, 72])
+@pytest.mark.parametrize("S", [50, 70, 72, 1100, 1101])
 def test_rows_at_the_mask_value(gpu, S):
     """Visible scores at and below the mask's -1e9: the masked columns then carry weight, as in
     the reference's fill-then-softmax."""
@@ -96,7 +96,7 @@ def test_rows_at_the_mask_value(gpu, S):
     assert torch.allclose(s[0, 6], want, rtol=1e-6, atol=0)
 
 
-@pytest.mark.parametrize("cols", [255, 256, 1025])
+@pytest.mark.parametrize("cols", [33, 64, 255, 256, 1025, 1028])
 def test_rows_of_special_values(gpu, cols):
     """A NaN, an infinity or nothing but -inf makes its own row NaN and no other (rows share a
     wave); a -inf among finite scores weighs nothing. Tolerance as for the plain rows."""
@@ -113,12 +113,14 @@ def test_rows_of_special_values(gpu, cols):
     assert out[16384, cols // 2].item() == 0.0
 
 
-def test_length_rows(gpu):
-    """decode_probs over rows of 1,022 columns: only the first lens keys, zero past them, a zero
+@pytest.mark.parametrize("L", [1022, 3, 33, 64, 65, 1300, 1301])
+def test_length_rows(gpu, L):
+    """decode_probs over rows of `L` columns: only the first lens keys, zero past them, a zero
     row for an empty cache."""
-    n, H, L = 6, 700, 1022
+    n, H = 6, 700
     s = _normal((n * H, L), 30, 4.0)
-    lens = torch.tensor([1, 0, 513, 1022, 4, 257], dtype=torch.int32, device="cuda")
+    lens = torch.tensor([1, 0, L // 2 + 1, L, min(4, L), L // 4 + 1], dtype=torch.int32,
+                        device="cuda")
     keep = torch.arange(L, device="cuda") < lens.repeat_interleave(H).unsqueeze(1)
     probs = s.masked_fill(~keep, float("nan"))
     A.decode_probs(probs, lens, n, H, L, 0.5)
