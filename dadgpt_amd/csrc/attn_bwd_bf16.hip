@@ -441,14 +441,15 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
 constexpr int kQW = 32;  // queries per wave
 
 // One 32-key chunk (tile keys 32*kb ..) against the wave's 32 queries. Register 8j+e of lane
-// half hi holds tile key 32kb + 16j + 8hi + e. dP starts from `ndl`, -delta of the lane's query
-// in every element, so that P dP is dS. VALU and matrix pipe are both ~65% busy here, at a clock
-// of 1.75 GHz: without the 16 subtractions dQ takes 284 us for 295 at [96, 4096, 64], 47.9 for
-// 49.6 at [192, 1024, 64] (with a third tile buffer and loads two tiles ahead: 286 and 48.7; K^T
-// read before the exponentials spills). With dropout (DROP), dS = P (dP * f - delta), f =
-// keep/(1-p) from register 8j+e's uniform in `keep`: dP from zero there, as the 16 registers held
-// across the loop cost that kernel more (96 x 1024: backward 88 -> 92.5).
-template <int D, bool DROP>
+// half hi holds tile key 32kb + 16j + 8hi + e. FROM_DELTA: dP starts from `ndl`, -delta of the
+// lane's query in every element, so that P dP is dS; otherwise -delta (ndl[0]) is added after.
+// VALU and matrix pipe are both busy here: without the 16 subtractions dQ takes 284 us for 295 at
+// [96, 4096, 64], 47.9 for 49.6 at [192, 1024, 64] (with a third tile buffer and loads two tiles
+// ahead: 286 and 48.7; K^T read before the exponentials spills). The 16 registers held across the
+// loop must not cost a wave per SIMD, though (see dq_bf16_kernel). With dropout (DROP), dS =
+// P (dP * f - delta), f = keep/(1-p) from register 8j+e's uniform in `keep`: dP from zero, as
+// those registers cost that kernel more too (96 x 1024: backward 88 -> 92.5).
+template <int D, bool DROP, bool FROM_DELTA>
 __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
                                          const bf16x8 (&qop)[D / 16],
                                          const bf16x8 (&doop)[D / 16], const bf16* sk,
@@ -471,7 +472,7 @@ __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
   float pr[16];
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) {
-    dp = mfma32(va[ds], doop[ds], !DROP && ds == 0 ? ndl : dp);
+    dp = mfma32(va[ds], doop[ds], FROM_DELTA && ds == 0 ? ndl : dp);
 #pragma unroll
     for (int i = ds * (16 / DS); i < (ds + 1) * (16 / DS); ++i)
       pr[i] = fast_exp2(fmaf(s[i], scale_log2, -lse2));
@@ -496,7 +497,7 @@ __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
         if constexpr (DROP)
           d[h] = p * fmaf(dp[8 * j + e], keep_factor(keep, 8 * j + e, dr), ndl[0]);
         else
-          d[h] = p * dp[8 * j + e];
+          d[h] = p * (FROM_DELTA ? dp[8 * j + e] : dp[8 * j + e] + ndl[0]);
       }
       w[e2] = pack_bf16x2(d[0], d[1]);
     }
@@ -513,7 +514,7 @@ __device__ __forceinline__ void dq_chunk(bool diag, f32x16 (&dqacc)[D / 32],
 // dQ for one query block per wave; the kernel also computes delta = rowsum(dO * O) of its
 // rows (from the dO operands it holds and one load of O) and writes it for the dK/dV kernel,
 // so the backward needs no separate delta pass.
-template <int D, bool STRIDED, bool DROP, int KS, bool WRITE_DELTA>
+template <int D, bool STRIDED, bool DROP, int KS, bool WRITE_DELTA, bool FROM_DELTA>
 __device__ __forceinline__ void dq_workgroup(const BwdArgs& a, int bh, int qblk,
                                              BwdTiles<D>& tiles) {
   constexpr int kGroups = kWaves / KS, QB = kQW * kGroups;  // query groups, queries
@@ -585,7 +586,7 @@ __device__ __forceinline__ void dq_workgroup(const BwdArgs& a, int bh, int qblk,
       dpart += bf16_lo(g[w]) * bf16_lo(o[w]) + bf16_hi(g[w]) * bf16_hi(o[w]);
   }
   const float dlt = sum_halves(dpart);
-  f32x16 ndl;  // what dP starts from
+  f32x16 ndl;  // -delta (what dP starts from)
 #pragma unroll
   for (int i = 0; i < 16; ++i) ndl[i] = -dlt;
   if (WRITE_DELTA && hi == 0 && qrow < S && sub == 0) delta[(size_t)bh * S + qrow] = dlt;
@@ -604,7 +605,7 @@ __device__ __forceinline__ void dq_workgroup(const BwdArgs& a, int bh, int qblk,
         KeepWords16 keep = {};
         if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qrow, klo, hi);
         // some key after some query: mask
-        dq_chunk<D, DROP>(klo + 31 > q0, dqacc, qop, doop, ck, cv, kb, qrow - k0, lse2, ndl,
+        dq_chunk<D, DROP, FROM_DELTA>(klo + 31 > q0, dqacc, qop, doop, ck, cv, kb, qrow - k0, lse2, ndl,
                           lane, scale_log2, keep, dr);
       }
     }
@@ -633,7 +634,12 @@ template <int D, bool STRIDED, bool DROP, int KS>
 __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(const BwdArgs a) {
   __shared__ BwdTiles<D> tiles;
   // longest (latest) query blocks dispatch first
-  dq_workgroup<D, STRIDED, DROP, KS, true>(a, blockIdx.x, gridDim.y - 1 - blockIdx.y, tiles);
+  // At d_head 32 with one wave per group, dP from zero keeps the kernel at 120 registers, four
+  // waves per SIMD; from -delta it takes 138 and three: 320 x 384 backward 24.8 -> 26.8 us,
+  // 640 x 300 35.1 -> 37.5. (In one launch the dK/dV workgroups set the registers anyway.)
+  constexpr bool kFromDelta = !DROP && (D == 64 || KS == 2);
+  dq_workgroup<D, STRIDED, DROP, KS, true, kFromDelta>(a, blockIdx.x,
+                                                       gridDim.y - 1 - blockIdx.y, tiles);
 }
 
 // ---------------------------------------------------------------- both in one launch
@@ -651,8 +657,8 @@ __global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocks
     dkdv_workgroup<D, STRIDED, DROP, KS, OWN_DELTA>(a, blockIdx.x, blockIdx.y, tiles, stats,
                                                     own_delta);
   else
-    dq_workgroup<D, STRIDED, DROP, KS, OWN_DELTA>(a, blockIdx.x, gridDim.y - 1 - blockIdx.y,
-                                                  tiles);
+    dq_workgroup<D, STRIDED, DROP, KS, OWN_DELTA, !DROP>(a, blockIdx.x,
+                                                         gridDim.y - 1 - blockIdx.y, tiles);
 }
 
 // How a backward is launched: dQ, then dK/dV (kSeparate); both in one launch with delta
