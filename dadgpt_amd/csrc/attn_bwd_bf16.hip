@@ -670,25 +670,45 @@ struct BwdPlan {
 };
 
 // One launch saves a kernel's start and end (~4 us) and lets the dQ workgroups fill the CUs that
-// the dK/dV ones leave idle at the end of their chains. It pays up to about four 128-row
-// workgroups of each kind per CU (one more per head counted), and whatever the batch for S <=
-// 256; beyond, the CUs are full and recomputing delta costs more. Separate -> one launch, us
-// (BH x S, D = 64): 128 x 128 11.5 -> 7.8, 192 x 256 20.0 -> 15.4, 24 x 1024 32.8 -> 24.5,
-// 96 x 1024 67 -> 60, 128 x 1024 83 -> 80, 24 x 4096 211 -> 192, 12 x 4096 127 -> 102, 768 x 256
-// 62 -> 60.5; on the other side 256 x 512 55.7 -> 56.7, 192 x 1024 115 -> 122. With dropout, whose
-// kernel holds two workgroups per CU where dQ alone holds three, the line for long rows is
-// nearer: 24 x 1024 44 -> 33, 40 x 1024 46 -> 44, 64 x 1024 67 -> 68, 96 x 1024 98 -> 107. Up to
-// 1,024 rows the dK/dV workgroups compute delta themselves (96 x 1024: 59 against 61 us with the
-// pass).
+// the dK/dV ones leave idle at the end of their chains; where the CUs are full anyway, delta
+// summed twice and the two kinds' mixture cost more than that. Separate -> one launch, us (BH x S,
+// D = 64): 128 x 128 11.5 -> 7.8, 192 x 256 20.0 -> 15.4, 24 x 1024 32.8 -> 24.5, 96 x 1024 67 ->
+// 60, 128 x 1024 83 -> 80, 24 x 4096 211 -> 192. In 128-row workgroups of each kind per CU the
+// line lies,
+//  - up to two row blocks, at 5 (448 x 256 36.9 -> 33.2, 960 x 256 token-major 77.1 -> 80.9, 1536
+//    x 256 114 -> 125; dropout 576 x 256 59.6 -> 59.4, 768 x 256 77.1 -> 81.2), for single blocks
+//    without dropout at 13 (2500 x 128 token-major 82.2 -> 85.6); at D = 32, whose kernels hold
+//    more workgroups, at 8 (640 x 256 26.6 -> 24.4, 960 x 256 token-major 62.5 -> 64.9), with
+//    dropout none;
+//  - then at 4.5, one more per head counted (160 x 900 82.5 -> 81.1, dropout 96 x 1024 86.9 -> 85.6,
+//    128 x 600 56.6 -> 52.0; 192 x 1024 115 -> 122, dropout 256 x 400 58.7 -> 62.9), and at 3 where
+//    delta takes a pass of its own (64 x 1500 79.3 -> 77.4; 72 x 1500 86.5 -> 90.1);
+//  - with dropout at D = 32 over 512 rows, where two waves per group gain more apart, at 1.5 (64 x
+//    1024 44.7 -> 46.6, 48 x 1200 49.1 -> 53.3).
+// Apart, too, where the heads fill seven eighths of the CUs or more in one round: each CU then has
+// one workgroup of every block, and both kernels end together (256 x 384 31.1 -> 33.1, token-major
+// 32.3 -> 35.9). The line must not tell the layouts apart: a strided call gives the contiguous
+// one's bits. Up to 1,024 rows the dK/dV workgroups compute delta themselves (96 x 1024: 59
+// against 61 us with the pass).
 // Two waves per row group then pay only while the grid, twice as large now, still fits on the
 // CUs, or for long chains up to twice that (one wave -> two): 64 x 256 10.8 -> 10.4, 24 x 1024
 // 30.4 -> 24.5, 96 x 512 21.4 -> 24.4, 64 x 800 31.2 -> 33.2, 24 x 2048 61 -> 57; 128 x 128
 // 7.7 -> 8.0.
+bool bwd_in_one_launch(int BH, int S, int D, bool drop) {
+  const long long cus = device_cus(), wgs = (long long)BH * ((S + 127) / 128);
+  const bool full_round = 8LL * BH >= 7 * cus && BH <= cus;
+  if (D == 64 && !drop && full_round && S >= 224 && S <= kOwnDeltaMaxS) return false;
+  if (S <= 256) {
+    if (D == 32) return drop || wgs <= (S <= 128 ? 13 : 8) * cus;
+    return wgs <= (S <= 128 && !drop ? 13 : 5) * cus;
+  }
+  if (drop && D == 32 && S > 512) return 2 * (wgs + BH) <= 3 * cus;
+  if (!drop && S > kOwnDeltaMaxS) return wgs <= 3 * cus;
+  return 2 * (wgs + BH) <= 9 * cus;
+}
 BwdPlan bwd_plan(int BH, int S, int D, bool drop) {
-  const long long cus = device_cus(), rows64 = (long long)BH * ((S + 63) / 64),
-                  wgs = (long long)BH * ((S + 127) / 128 + 1);
-  const bool one = drop && S > 512 ? 2 * wgs <= 3 * cus : S <= 256 || 2 * wgs <= 9 * cus;
-  if (!one) return {kSeparate, waves_per_group(BH, S, D, drop)};
+  if (!bwd_in_one_launch(BH, S, D, drop)) return {kSeparate, waves_per_group(BH, S, D, drop)};
+  const long long cus = device_cus(), rows64 = (long long)BH * ((S + 63) / 64);
   const bool two = S > 64 && (S <= 128    ? 2 * rows64 <= cus
                               : S < 1024 ? 2 * rows64 <= 3 * cus
                                          : rows64 <= 3 * cus);
