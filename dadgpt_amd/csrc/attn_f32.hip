@@ -148,21 +148,24 @@ struct X3 {
 
 // pack_bf16x2 for a word whose halves are taken apart again: opaque, because the compiler would
 // otherwise convert the low half a second time instead of shifting it out of the word (48 of
-// dK/dV's 576 VALU instructions per chunk).
+// dK/dV's 576 VALU instructions per chunk). ONCE = false leaves the compiler the second
+// conversion, which does not wait for the first: shorter for a wave that has its SIMD to itself.
+template <bool ONCE = true>
 __device__ __forceinline__ uint32_t pack_once(float lo, float hi) {
   uint32_t w = pack_bf16x2(lo, hi);
-  asm("" : "+v"(w));
+  if constexpr (ONCE) asm("" : "+v"(w));
   return w;
 }
 
+template <bool ONCE = true>
 __device__ __forceinline__ X3 split3(const float (&x)[8]) {
   u32x4 w[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float a0 = x[2 * i], a1 = x[2 * i + 1];
-    const uint32_t p = pack_once(a0, a1);
+    const uint32_t p = pack_once<ONCE>(a0, a1);
     const float b0 = a0 - bf16_lo(p), b1 = a1 - bf16_hi(p);  // exact
-    const uint32_t q = pack_once(b0, b1);
+    const uint32_t q = pack_once<ONCE>(b0, b1);
     const float c0 = b0 - bf16_lo(q), c1 = b1 - bf16_hi(q);  // exact
     w[0][i] = p;
     w[1][i] = q;
@@ -211,7 +214,7 @@ __device__ __forceinline__ void store_x3(const T& t, bf16* planes) {
 
 // The B operand of a score product from a global row: lane half h supplies columns
 // 16 ds + 8 h + 0..7 of `row`, split into three bf16 planes.
-template <int D>
+template <int D, bool ONCE = true>
 __device__ __forceinline__ void load_split_row(X3 (&x)[D / 16], const float* row, int h) {
 #pragma unroll
   for (int ds = 0; ds < D / 16; ++ds) {
@@ -220,7 +223,7 @@ __device__ __forceinline__ void load_split_row(X3 (&x)[D / 16], const float* row
     const f32x4 v1 = *reinterpret_cast<const f32x4*>(row + 16 * ds + 8 * h + 4);
 #pragma unroll
     for (int e = 0; e < 4; ++e) a[e] = v0[e], a[4 + e] = v1[e];
-    x[ds] = split3(a);
+    x[ds] = split3<ONCE>(a);
   }
 }
 
@@ -240,7 +243,7 @@ __device__ __forceinline__ f32x16 score_tile_p(const bf16* planes, int chunk_row
   return acc;
 }
 
-template <int D, int TR>
+template <int D, int TR, bool ONCE = true>
 __device__ __forceinline__ void accumulate_t_p(f32x16 (&acc)[D / 32], const bf16* planes,
                                                int chunk_row0, const f32x16& p, int lane) {
 #pragma unroll
@@ -248,7 +251,7 @@ __device__ __forceinline__ void accumulate_t_p(f32x16 (&acc)[D / 32], const bf16
     float x[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = p[8 * j + e];
-    const X3 pb = split3(x);
+    const X3 pb = split3<ONCE>(x);
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) {
       X3 a;
@@ -369,8 +372,12 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
   const int last = min(S, (blk + 1) * kRows) - 1;  // the workgroup's last query
   const int n_tiles = last / TR + 1;
 
+  // Conversions of the weights once only with two waves per group: with one, the last workgroups
+  // run a wave per SIMD (192 x 400 48.6 -> 54.4 us, 256 x 384 42.8 -> 47.0 with it, for 161.5 ->
+  // 160.3 at 192 x 1024; with two, 48 x 1024 48.5 -> 47.8).
+  constexpr bool kOnce = KS == 2;
   X3 qb[D / 16];  // the lane's query row, split
-  load_split_row<D>(qb, q + base + (size_t)min(qi, S - 1) * D, h);
+  load_split_row<D, kOnce>(qb, q + base + (size_t)min(qi, S - 1) * D, h);
   f32x16 o[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) o[db] = zero16();
@@ -442,7 +449,7 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
       if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qi, key0, h);
 #pragma unroll
       for (int u = 0; u < 16; ++u) s[u] = DROP ? w[u] * keep_factor(keep, u, dr) : w[u];
-      accumulate_t_p<D, TR>(o, svp, 32 * c, s, lane);
+      accumulate_t_p<D, TR, kOnce>(o, svp, 32 * c, s, lane);
     }
   };
   if constexpr (KS == 1) {
