@@ -54,7 +54,8 @@ def _check(BH, S, D, dtype, tols):
 F32_SHAPES = [(3, 96, 64), (3, 97, 64), (2, 129, 64), (5, 160, 32), (1, 500, 64), (64, 1000, 64),
               (65, 1000, 64), (128, 385, 32), (129, 390, 32), (512, 100, 64), (513, 100, 32),
               (64, 40, 64), (65, 33, 64), (32, 1000, 64), (33, 1000, 32), (3, 512, 64),
-              (3, 513, 64), (86, 300, 64), (85, 300, 64), (76, 600, 32), (77, 600, 64)]
+              (3, 513, 64), (86, 300, 64), (85, 300, 64), (76, 600, 32), (77, 600, 64),
+              (24, 600, 32)]
 
 
 @pytest.mark.parametrize("BH,S,D", F32_SHAPES)
@@ -86,28 +87,23 @@ def test_bf16_shapes(gpu, BH, S, D):
     _check(BH, S, D, torch.bfloat16, BF16_TOLS)
 
 
-@pytest.mark.parametrize("BH,S", [(2, 70), (5, 300), (99, 520), (150, 520), (3, 1030), (30, 600), (100, 257), (60, 700)])
-def test_bf16_dropout_and_strided_shapes(gpu, BH, S):
-    """The dropout instantiations at p = 0 give the plain results, and the strided ones the
-    contiguous ones', on both sides of the lines that differ between them: to the rounding of
-    another summation order, 2^-8 of the values' scale (outputs and gradients below 8)."""
-    print(f"[case] dropout / strided BH={BH} S={S}", flush=True)
-    D, tol = 64, 8 * 2.0 ** -8
+@pytest.mark.parametrize("BH,S,D", [(2, 70, 64), (5, 300, 64), (99, 520, 64), (150, 520, 64),
+                                    (3, 1030, 64), (30, 600, 64), (100, 257, 64), (60, 700, 64),
+                                    (60, 1100, 64), (60, 1100, 32), (3, 1030, 32), (300, 150, 32),
+                                    (200, 600, 32)])
+def test_bf16_strided_shapes(gpu, BH, S, D):
+    """The strided instantiations give the contiguous ones' bits on both sides of the lines, and a
+    dropout rate of zero, which runs the plain kernels, too."""
+    print(f"[case] strided BH={BH} S={S} D={D}", flush=True)
     q, k, v, dout = _inputs(BH, S, D, torch.bfloat16, S)
     scale = A.default_scale(D)
     out, lse = A.attention_forward(q, k, v, scale)
     want = (out, lse) + A.attention_backward(dout, out, lse, q, k, v, scale)[:3]
-
-    def close(got):
-        for x, y in zip(got, want):
-            assert (x.float() - y.float()).abs().max().item() <= tol
-
     o2, l2, delta = torch.empty_like(out), torch.empty_like(lse), torch.empty_like(lse)
     A.flash_attention_forward_bf16_dropout(o2, l2, q, k, v, BH, S, D, scale, 0.0, 5)
     grads = [torch.empty_like(q) for _ in range(3)]
     A.flash_attention_backward_bf16_dropout(*grads, delta, dout, o2, l2, q, k, v, BH, S, D, scale,
                                             0.0, 5)
-    close((o2, l2, *grads))
     tokens = [x.view(1, BH, S, D).transpose(1, 2).contiguous().transpose(1, 2)
               for x in (q, k, v, dout)]
     o3 = torch.empty_like(tokens[0])
@@ -115,7 +111,10 @@ def test_bf16_dropout_and_strided_shapes(gpu, BH, S):
     A.flash_attention_forward_bf16_strided(o3, l3, *tokens[:3], scale)
     g3 = [torch.empty_like(tokens[0]) for _ in range(3)]
     A.flash_attention_backward_bf16_strided(*g3, delta, tokens[3], o3, l3, *tokens[:3], scale)
-    close((o3.reshape(BH, S, D), l3, *[x.reshape(BH, S, D) for x in g3]))
+    for got in ((o2, l2, *grads),
+                (o3.reshape(BH, S, D), l3, *[x.reshape(BH, S, D) for x in g3])):
+        for x, y in zip(got, want):
+            assert torch.equal(x, y)
 
 
 # (3 slices: two waves per group; 400 slices: one wave per group, at S = 160 in D = 64 and 32)
@@ -184,6 +183,14 @@ def test_bf16_backward_in_place(gpu, BH, S, D):
                                             tok["out"], lse, tok["q"], tok["k"], tok["v"], scale)
     for x, y in zip(("out", "k", "v"), want):
         assert torch.equal(tok[x].reshape(BH, S, D), y), x
+    # with dropout (p = 0.1) against the call with buffers of its own, to the rounding of another
+    # summation order: 2^-8 of values below 8
+    shape = (BH, S, D, scale, 0.1, 5)
+    A.flash_attention_forward_bf16_dropout(out, lse, q, k, v, *shape)
+    A.flash_attention_backward_bf16_dropout(*want, delta, dout, out, lse, q, k, v, *shape)
+    A.flash_attention_backward_bf16_dropout(out, k, v, delta, dout, out, lse, q, k, v, *shape)
+    for x, y in zip((out, k, v), want):
+        assert (x.float() - y.float()).abs().max().item() <= 8 * 2.0 ** -8
 
 
 @pytest.mark.parametrize("BH,S,D", [(4, 70, 64), (24, 300, 32), (24, 600, 64), (160, 300, 64)])

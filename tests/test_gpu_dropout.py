@@ -101,9 +101,7 @@ def test_dropout_random_shapes(gpu, BH, S, D, p):
 
 
 def test_dropout_rate_zero_equals_plain(gpu):
-    """p = 0 keeps every probability with factor 1: the forward and dQ are bit for bit the
-    plain kernels' (dK/dV folds delta in after its products instead of before: within
-    rounding)."""
+    """p = 0 drops nothing: the call runs the plain kernels and gives their bits."""
     BH, S, D = 3, 300, 64
     case(f"bf16 dropout p=0 vs plain BH={BH} S={S} D={D}")
     qn, kn, vn, gn = synth.attn_inputs(BH, S, D, seed=611, with_dout=True, bf16=True)
@@ -114,7 +112,39 @@ def test_dropout_rate_zero_equals_plain(gpu):
     torch.cuda.synchronize()
     assert torch.equal(out, o2) and torch.equal(lse, l2)
     assert torch.equal(dq, dq2) and torch.equal(delta, d2)
-    assert max_abs(host(dk), host(dk2)) <= 1e-2 and max_abs(host(dv), host(dv2)) <= 1e-2
+    assert torch.equal(dk, dk2) and torch.equal(dv, dv2)
+
+
+# Where the bf16 dropout kernels change course, on 256 CUs: the backward in one launch with two
+# waves per row group and one, with its own delta and after a delta pass, and in two launches;
+# at d_head 32 also two launches with two waves. (Last slice: large mask row counters.)
+PLAN_SHAPES = [(24, 1024, 64), (96, 600, 64), (150, 520, 64), (256, 100, 64), (3, 1030, 64),
+               (60, 1100, 64), (24, 2048, 64), (200, 600, 64), (96, 1024, 64), (128, 512, 64),
+               (600, 200, 32), (100, 600, 32), (200, 600, 32), (3, 1030, 32)]
+
+
+@pytest.mark.parametrize("BH,S,D", PLAN_SHAPES)
+def test_dropout_of_every_plan(gpu, BH, S, D):
+    """The bf16 kernels at p = 0.1 against the oracle's first and last slices (long rows: the last,
+    its backward takes seconds); the calls repeat exactly, every output is finite, and lse is the
+    undropped one."""
+    p, seed = 0.1, 0x0DAD_0000_0000 + 7 * S + BH
+    case(f"bf16 dropout plan BH={BH} S={S} D={D}")
+    scale = float(np.float32(1.0 / math.sqrt(D)))
+    gen = torch.Generator(device="cuda").manual_seed(S + BH)
+    q, k, v, g = (torch.randn((BH, S, D), generator=gen, device="cuda").to(torch.bfloat16)
+                  for _ in range(4))
+    got = run(q, k, v, g, scale, p, seed)
+    for x, y in zip(got, run(q, k, v, g, scale, p, seed)):
+        assert torch.equal(x, y) and bool(torch.isfinite(x).all())
+    assert (got[1] - A.attention_forward(q, k, v, scale)[1]).abs().max().item() <= TOL_LSE
+    qn, kn, vn, gn = host(q), host(k), host(v), host(g)
+    for bh in (0, BH - 1) if S <= 1100 else (BH - 1,):
+        o_ref = oracle.attn_fwd_dropout_slices(qn, kn, vn, scale, p, seed, bh, bh + 1)
+        within_scaled(host(got[0][bh]), o_ref[0], TOL_O, p, f"out[{bh}]")
+        refs = oracle.attn_bwd_dropout_slices(gn, qn, kn, vn, scale, p, seed, bh, bh + 1)
+        for x, ref, nm in zip(got[2:5], refs, ("dq", "dk", "dv")):
+            within_scaled(host(x[bh]), ref[0], TOL_GRAD, p, f"{nm}[{bh}]")
 
 
 def test_dropout_seed_changes_mask_and_is_deterministic(gpu):
@@ -188,6 +218,33 @@ def test_dropout_f32_matches_oracle(gpu, BH, S, D, p):
     refs = oracle.attn_bwd_dropout(gn, qn, kn, vn, scale, p, seed, out=o_ref)
     for got, ref, nm in zip((dq, dk, dv, delta), refs, ("dq", "dk", "dv", "delta")):
         assert max_abs(host(got), ref) <= TOL_F32, nm
+
+
+# One and two waves per row group (256 workgroups of 128 rows; 64 up to 96 rows), delta summed by
+# the backward and, past 512 rows, by its own pass.
+F32_PLAN_SHAPES = [(3, 512, 64), (3, 513, 64), (33, 1000, 64), (24, 1000, 32), (129, 390, 64),
+                   (65, 96, 32), (64, 90, 64), (160, 300, 32), (60, 600, 64), (60, 600, 32)]
+
+
+@pytest.mark.parametrize("BH,S,D", F32_PLAN_SHAPES)
+def test_dropout_f32_of_every_plan(gpu, BH, S, D):
+    """The fp32 kernels at p = 0.2 against the oracle's first and last slices, at 1e-5 of the
+    values' magnitude (kept values carry 1 / (1 - p))."""
+    p, seed = 0.2, 0x0DAD_0000_0000 + 9 * S + BH
+    case(f"fp32 dropout plan BH={BH} S={S} D={D}")
+    scale = float(np.float32(1.0 / math.sqrt(D)))
+    gen = torch.Generator(device="cuda").manual_seed(S + BH)
+    q, k, v, g = (torch.randn((BH, S, D), generator=gen, device="cuda") for _ in range(4))
+    got = run_f32(q, k, v, g, scale, p, seed)
+    for x, y in zip(got, run_f32(q, k, v, g, scale, p, seed)):
+        assert torch.equal(x, y) and bool(torch.isfinite(x).all())
+    qn, kn, vn, gn = host(q), host(k), host(v), host(g)
+    for bh in (0, BH - 1):
+        o_ref = oracle.attn_fwd_dropout_slices(qn, kn, vn, scale, p, seed, bh, bh + 1)
+        refs = oracle.attn_bwd_dropout_slices(gn, qn, kn, vn, scale, p, seed, bh, bh + 1)
+        for x, ref, nm in zip((got[0], *got[2:5]), (o_ref, *refs), ("out", "dq", "dk", "dv")):
+            bound = TOL_F32 * max(1.0, float(np.abs(ref).max())) / (1.0 - p)
+            assert max_abs(host(x[bh]), ref[0]) <= bound, (nm, bh)
 
 
 def test_dropout_f32_rate_zero_equals_plain(gpu):
