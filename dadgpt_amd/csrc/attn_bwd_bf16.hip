@@ -46,8 +46,9 @@ constexpr int kWaves = 4;
 #ifndef DADGPT_DQ_MINB
 #define DADGPT_DQ_MINB 3
 #endif
-constexpr int kDkdvMinBlocks = DADGPT_DKDV_MINB;
-constexpr int kDkdvMinBlocksNoDrop = DADGPT_DKDV_MINB_NODROP;
+constexpr int dkdv_wgs_per_cu(bool drop) {
+  return drop ? DADGPT_DKDV_MINB : DADGPT_DKDV_MINB_NODROP;
+}
 constexpr int kDqMinBlocks = DADGPT_DQ_MINB;
 
 // ---------------------------------------------------------------- delta
@@ -112,7 +113,9 @@ constexpr int kKW = 32;  // keys per wave
 // dS = P (dP f - delta), so dp starts from zero and -delta is read separately.
 // XA: operand addresses from `lo` (LaneLds, tiles.hpp), XORed once per phase, instead of
 // computed per read: what brings dK/dV (all but the dropout instantiation) to 168 VGPRs,
-// three workgroups per CU, without spilling in the loop.
+// three workgroups per CU, without spilling in the loop. (The strided kernel of one launch with
+// its own delta and one wave per group keeps two registers in scratch and reloads them as it
+// issues a tile.)
 template <int D, bool DROP, bool XA>
 __device__ __forceinline__ void dkdv_block(bool mask, f32x16 (&dkacc)[D / 32],
                                            f32x16 (&dvacc)[D / 32], const bf16x8 (&kop)[D / 16],
@@ -429,7 +432,7 @@ __device__ __forceinline__ void dkdv_workgroup(const BwdArgs& a, int bh, int kbl
 }
 
 template <int D, bool STRIDED, bool DROP, int KS>
-__global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocksNoDrop) void dkdv_bf16_kernel(
+__global__ __launch_bounds__(64 * kWaves, dkdv_wgs_per_cu(DROP)) void dkdv_bf16_kernel(
     const BwdArgs a) {
   __shared__ BwdTiles<D> tiles;
   __shared__ BwdStats stats;
@@ -605,8 +608,8 @@ __device__ __forceinline__ void dq_workgroup(const BwdArgs& a, int bh, int qblk,
         KeepWords16 keep = {};
         if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qrow, klo, hi);
         // some key after some query: mask
-        dq_chunk<D, DROP, FROM_DELTA>(klo + 31 > q0, dqacc, qop, doop, ck, cv, kb, qrow - k0, lse2, ndl,
-                          lane, scale_log2, keep, dr);
+        dq_chunk<D, DROP, FROM_DELTA>(klo + 31 > q0, dqacc, qop, doop, ck, cv, kb, qrow - k0,
+                                      lse2, ndl, lane, scale_log2, keep, dr);
       }
     }
     wait_vm_lds<0>();
@@ -648,7 +651,7 @@ __global__ __launch_bounds__(64 * kWaves, kDqMinBlocks) void dq_bf16_kernel(cons
 // them) and the dQ workgroups write it; otherwise a pass before has.
 constexpr int kOwnDeltaMaxS = 1024;
 template <int D, bool STRIDED, bool DROP, int KS, bool OWN_DELTA>
-__global__ __launch_bounds__(64 * kWaves, DROP ? kDkdvMinBlocks : kDkdvMinBlocksNoDrop) void bwd_bf16_kernel(
+__global__ __launch_bounds__(64 * kWaves, dkdv_wgs_per_cu(DROP)) void bwd_bf16_kernel(
     const BwdArgs a) {
   __shared__ BwdTiles<D> tiles;
   __shared__ BwdStats stats;
@@ -680,9 +683,9 @@ struct BwdPlan {
 //    without dropout at 13 (2500 x 128 token-major 82.2 -> 85.6); at D = 32, whose kernels hold
 //    more workgroups, at 8 (640 x 256 26.6 -> 24.4, 960 x 256 token-major 62.5 -> 64.9), with
 //    dropout none;
-//  - then at 4.5, one more per head counted (160 x 900 82.5 -> 81.1, dropout 96 x 1024 86.9 -> 85.6,
-//    128 x 600 56.6 -> 52.0; 192 x 1024 115 -> 122, dropout 256 x 400 58.7 -> 62.9), and at 3 where
-//    delta takes a pass of its own (64 x 1500 79.3 -> 77.4; 72 x 1500 86.5 -> 90.1);
+//  - then at 4.5, one more per head counted (160 x 900 82.5 -> 81.1, dropout 96 x 1024 86.9 ->
+//    85.6, 128 x 600 56.6 -> 52.0; 192 x 1024 115 -> 122, dropout 256 x 400 58.7 -> 62.9), and at
+//    3 where delta takes a pass of its own (64 x 1500 79.3 -> 77.4; 72 x 1500 86.5 -> 90.1);
 //  - with dropout at D = 32 over 512 rows, where two waves per group gain more apart, at 1.5 (64 x
 //    1024 44.7 -> 46.6, 48 x 1200 49.1 -> 53.3).
 // Apart, too, where the heads fill seven eighths of the CUs or more in one round: each CU then has
@@ -725,8 +728,8 @@ hipError_t launch_bwd_bf16_t(bf16* dq, bf16* dk, bf16* dv, float* delta, const b
   const DropParams dr = drop_params(drop);  // dropout: contiguous layout only (caller checks)
   auto span = [&](const bf16* p, int t) {  // tensor t's extent
     const HeadStrides& h = L.t[t];
-    const size_t batches = BH / L.n_heads, heads = L.n_heads;
-    return Span{p, 2 * ((batches - 1) * h.batch + (heads - 1) * h.head + (size_t)(S - 1) * h.row + D)};
+    const size_t batches = BH / L.n_heads, heads = L.n_heads, rows = S;
+    return Span{p, 2 * ((batches - 1) * h.batch + (heads - 1) * h.head + (rows - 1) * h.row + D)};
   };
   // The phase calls, and a backward in place (dk = k, dv = v, or any gradient = out), run dQ first,
   // then dK/dV.

@@ -264,7 +264,9 @@ __device__ __forceinline__ void accumulate_t_p(f32x16 (&acc)[D / 32], const bf16
 }
 
 // score_tile_p and accumulate_t_p at the start of `planes`, with the addresses from
-// LaneLds (tiles.hpp): the dK/dV kernel's register relief (no spills at D = 64).
+// LaneLds (tiles.hpp): the dK/dV kernel's register relief. At D = 64 the kernel uses all 256: the
+// one-wave instances without dropout and the two-wave ones with it keep one or two registers in
+// scratch, the others none.
 template <int D, int TR>
 __device__ __forceinline__ f32x16 score_tile_px(const bf16* planes, const X3 (&b)[D / 16],
                                                 const LaneLds& lo) {
@@ -478,7 +480,8 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
     }
   }
   __syncthreads();  // every wave is done with the tiles: they hold partials and staging now
-  float* slot = reinterpret_cast<float*>(planes) + grp * (KS > 1 && kPart > kStage ? kPart : kStage);
+  constexpr int kSlot = KS > 1 && kPart > kStage ? kPart : kStage;
+  float* slot = reinterpret_cast<float*>(planes) + grp * kSlot;
   if constexpr (KS == 2) {
     // (m, l, O) of the group's second wave: rescaled to the larger maximum and added. A wave
     // that saw no chunk has m = -inf and zeros, which get weight 0.

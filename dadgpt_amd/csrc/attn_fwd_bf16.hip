@@ -397,7 +397,8 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
     // the tiles are free after the last barrier: each wave stages its rows in its quarter of sk
     if (q0 + 32 * i < S)
       store_rows_staged<D>(sl.row(out, kTO, q0 + 32 * i), sl.pitch(kTO), S - q0 - 32 * i,
-                           oacc[i], inv, &sk[0][0] + (KS == 1 ? wave : grp * 2) * 32 * D * kNQB + i * 32 * D, lane);
+                           oacc[i], inv,
+                           &sk[0][0] + ((KS == 1 ? wave : grp * 2) * kNQB + i) * 32 * D, lane);
     if (qrow < S && hi == 0) lse[(size_t)bh * S + qrow] = (mrun[i] + __log2f(l)) * kLn2;
   }
 }
@@ -424,7 +425,8 @@ hipError_t launch_fwd_bf16_t(bf16* out, float* lse, const bf16* q, const bf16* k
         out, lse, q, k, v, S, c, scale < 0.f, snake, L, dr);
   };
   // dropout: contiguous layout only (checked by the caller)
-  with_shape(waves_per_group(BH, S, D, drop != nullptr), drop != nullptr, !is_contiguous(L, S, D), launch);
+  with_shape(waves_per_group(BH, S, D, drop != nullptr), drop != nullptr,
+             !is_contiguous(L, S, D), launch);
   return hipGetLastError();
 }
 

@@ -147,9 +147,10 @@ __device__ __forceinline__ float masked_weight(float mx) {
   return expf(kMaskValue - mx);
 }
 
-// x / sum as q = x inv, corrected once by its exact remainder (inv = 1 / sum): the quotient
-// IEEE division gives, in three operations per element. sum >= 1 or the row is degenerate (0 or
-// NaN, which stays NaN).
+// x / sum as q = x inv, corrected once by its remainder (Markstein's division by a reciprocal;
+// inv = 1 / sum): the quotient IEEE division gives wherever it and the remainder are normal, and
+// within a unit in the last place of it below, in three operations per element. sum >= 1 or the
+// row is degenerate (0 or NaN, which stays NaN).
 __device__ __forceinline__ float divide(float x, float sum, float inv) {
   const float q = x * inv;
   return fmaf(fmaf(-q, sum, x), inv, q);
@@ -242,7 +243,8 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_reg_kernel(
 
 // Softmax of rows of at most kNarrow columns, one column a lane, RPW rows per wave: a 16-byte
 // piece would leave most lanes without columns and cost every lane four exponentials. Bound: the
-// instructions per row. 49,152 rows of 3 / 17 / 64 columns: 21.0 / 14.7 / 15.0 us in pieces, 7.4 / 7.6 / 8.7 us here.
+// instructions per row. 49,152 rows of 3 / 17 / 64 columns: 21.0 / 14.7 / 15.0 us in pieces,
+// 7.4 / 7.6 / 8.7 us here.
 constexpr int kNarrow = 64;
 template <int MODE, int RPW>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void softmax_rows_narrow_kernel(
