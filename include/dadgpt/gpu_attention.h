@@ -19,6 +19,9 @@
  *    and that a flash backward may write a gradient over an input that only the workgroup of
  *    those rows reads: bf16 dk = k, dv = v, and one of dq, dk, dv = out; fp32 dq = q or dq =
  *    dout, and one of dq, dk, dv = out. Its kernels then run one after the other.
+ *  - A call repeats bit for bit, and the strided and token-major calls give the contiguous
+ *    ones' bits. The order of the sums follows from the shape and the number of compute units,
+ *    though: the same (b, h) slice may differ in its last bits between calls of another BH or S.
  *  - Arguments are validated on the host before any HIP call; a failing call returns a
  *    nonzero dadgpt_status and dadgpt_last_error() describes it (thread-local). Launch errors
  *    (hipGetLastError) map to DADGPT_ERR_HIP; asynchronous faults surface at the caller's
@@ -133,8 +136,10 @@ int dadgpt_flash_attention_backward_dropout(float* dq, float* dk, float* dv, flo
 
 /* One kernel of dadgpt_flash_attention_backward_bf16, for per-kernel timing and profiling
  * (no reference counterpart). phase 1: dq, and delta = rowsum(dout * out) of the same rows;
- * 2: dk, dv (reads delta). Running phases 1, 2 in order equals the full backward. phase 0
- * computes delta alone in a separate pass (equal to phase 1's up to fp32 summation order). */
+ * 2: dk, dv (reads delta). Running phases 1, 2 in order gives the full backward up to rounding:
+ * that one may run both kinds of workgroups in one launch, or another number of waves per row
+ * group, and then sums in another order. phase 0 computes delta alone in a separate pass (equal
+ * to phase 1's up to fp32 summation order). */
 int dadgpt_flash_attention_backward_bf16_phase(int phase, uint16_t* dq, uint16_t* dk,
                                                uint16_t* dv, float* delta,
                                                const uint16_t* dout, const uint16_t* out,
