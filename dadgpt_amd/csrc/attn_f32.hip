@@ -552,7 +552,6 @@ struct F32BwdArgs {
   int S;
   float scale;
   DropParams dr;
-  int first;  // what the workgroups of grid z = 0 compute: 0 dK/dV, 1 dQ
 };
 // LDS of a workgroup: the tiles, and per query row of a dK/dV tile lse and delta * scale.
 template <int D, int KS>
@@ -854,18 +853,31 @@ __device__ __forceinline__ void dq_f32_workgroup(const F32BwdArgs& a, int bh, in
 // us): 158 -> 143, 140 -> 86, 68 -> 55; where the CUs are full anyway (B16 H12 S1024) 532 -> 527.
 // OWN_DELTA: both kinds compute delta themselves, which saves the small grids a launch (4 x 64:
 // 10.0 -> 8.3 us); past kOwnDeltaMaxS rows, where dK/dV would read O and dO once per key block
-// more, a pass before does it (96 x 1024: 268 against 263.5 us). A backward in place (dq = q or
-// dout, or any gradient = out) runs as the delta pass, dK/dV and dQ, one after the other.
+// more, a pass before does it (96 x 1024: 268 against 263.5 us).
 constexpr int kOwnDeltaMaxS = 512;
 template <int D, bool DROP, int KS, bool OWN_DELTA>
 __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void bwd_f32_kernel(
     const F32BwdArgs a) {
   __shared__ F32BwdShared<D, KS> sm;
   __shared__ float own_delta[OWN_DELTA ? kOwnDeltaMaxS : 1];
-  if (a.first + blockIdx.z == 0)
+  if (blockIdx.z == 0)
     dkdv_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, blockIdx.y, sm, own_delta);
   else
     dq_f32_workgroup<D, DROP, KS, OWN_DELTA>(a, blockIdx.x, gridDim.y - 1 - blockIdx.y, sm);
+}
+
+// A backward in place (dq = q or dout, or any gradient = out) runs as the delta pass, dK/dV and
+// dQ, one after the other.
+template <int D, bool DROP>
+__global__ __launch_bounds__(64 * kGroups, wgs_per_cu(1)) void dkdv_f32_kernel(
+    const F32BwdArgs a) {
+  __shared__ F32BwdShared<D, 1> sm;
+  dkdv_f32_workgroup<D, DROP, 1, false>(a, blockIdx.x, blockIdx.y, sm, nullptr);
+}
+template <int D, bool DROP>
+__global__ __launch_bounds__(64 * kGroups, wgs_per_cu(1)) void dq_f32_kernel(const F32BwdArgs a) {
+  __shared__ F32BwdShared<D, 1> sm;
+  dq_f32_workgroup<D, DROP, 1, false>(a, blockIdx.x, gridDim.y - 1 - blockIdx.y, sm);
 }
 
 // Waves per row group. With one, a workgroup walks its chunks four waves wide, two workgroups
@@ -922,7 +934,7 @@ hipError_t bwd_f32_t(float* dq, float* dk, float* dv, float* delta, const float*
                      const float* out, const float* lse, const float* q, const float* k,
                      const float* v, int BH, int S, float scale, hipStream_t stream,
                      const Dropout* drop) {
-  F32BwdArgs args{dq, dk, dv, delta, q, k, v, dout, out, lse, S, scale, drop_params(drop), 0};
+  const F32BwdArgs args{dq, dk, dv, delta, q, k, v, dout, out, lse, S, scale, drop_params(drop)};
   auto span = [&](const float* p) { return Span{p, (size_t)BH * S * D * sizeof(float)}; };
   const bool separate = in_place({span(dq), span(dk), span(dv)},
                                  {span(q), span(k), span(v), span(dout), span(out)});
@@ -934,17 +946,18 @@ hipError_t bwd_f32_t(float* dq, float* dk, float* dv, float* delta, const float*
         delta, dout, out, rows);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  const dim3 grid(BH, (S + kRows - 1) / kRows, separate ? 1 : 2);
+  const dim3 blocks(BH, (S + kRows - 1) / kRows), grid(blocks.x, blocks.y, 2);
   with_f32_shape(bwd_waves_per_group(BH, S), drop != nullptr, [&](auto drop_c, auto ks) {
     constexpr int threads = 64 * kGroups * ks();
-    if (own)
+    if (separate) {
+      dkdv_f32_kernel<D, drop_c()><<<blocks, 64 * kGroups, 0, stream>>>(args);
+      if ((e = hipGetLastError()) != hipSuccess) return;
+      dq_f32_kernel<D, drop_c()><<<blocks, 64 * kGroups, 0, stream>>>(args);
+    } else if (own) {
       bwd_f32_kernel<D, drop_c(), ks(), true><<<grid, threads, 0, stream>>>(args);
-    else
+    } else {
       bwd_f32_kernel<D, drop_c(), ks(), false><<<grid, threads, 0, stream>>>(args);
-    e = hipGetLastError();
-    if (!separate || e != hipSuccess) return;
-    args.first = 1;
-    bwd_f32_kernel<D, drop_c(), ks(), false><<<grid, threads, 0, stream>>>(args);
+    }
     e = hipGetLastError();
   });
   return e;
