@@ -684,8 +684,8 @@ struct BwdPlan {
 //    more workgroups, at 8 (640 x 256 26.6 -> 24.4, 960 x 256 token-major 62.5 -> 64.9), with
 //    dropout none;
 //  - then at 4.5, one more per head counted (160 x 900 82.5 -> 81.1, dropout 96 x 1024 86.9 ->
-//    85.6, 128 x 600 56.6 -> 52.0; 192 x 1024 115 -> 122, dropout 256 x 400 58.7 -> 62.9), and at
-//    3 where delta takes a pass of its own (64 x 1500 79.3 -> 77.4; 72 x 1500 86.5 -> 90.1);
+//    85.6, 128 x 600 56.6 -> 52.0; 192 x 1024 115 -> 122, dropout 256 x 400 58.7 -> 62.9); with the
+//    delta pass, too (37 x 2886 163.7 -> 153.1, 48 x 2886 193.7 -> 188.4; 72 x 1500 86.5 -> 90.1);
 //  - with dropout at D = 32 over 512 rows, where two waves per group gain more apart, at 1.5 (64 x
 //    1024 44.7 -> 46.6, 48 x 1200 49.1 -> 53.3).
 // Apart, too, where the heads fill seven eighths of the CUs or more in one round: each CU then has
@@ -706,7 +706,6 @@ bool bwd_in_one_launch(int BH, int S, int D, bool drop) {
     return wgs <= (S <= 128 && !drop ? 13 : 5) * cus;
   }
   if (drop && D == 32 && S > 512) return 2 * (wgs + BH) <= 3 * cus;
-  if (!drop && S > kOwnDeltaMaxS) return wgs <= 3 * cus;
   return 2 * (wgs + BH) <= 9 * cus;
 }
 BwdPlan bwd_plan(int BH, int S, int D, bool drop) {
