@@ -348,7 +348,8 @@ __device__ __forceinline__ void store_rows_t(float* dst, int row0, int S,
 
 // ------------------------------------------------------------------------------ forward
 
-template <int D, bool DROP, int KS>
+// ONCE: the conversions of Q's and the weights' splits forced to happen once (pack_once).
+template <int D, bool DROP, int KS, bool ONCE>
 __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_kernel(
     float* __restrict__ out, float* __restrict__ lse, const float* __restrict__ q,
     const float* __restrict__ k, const float* __restrict__ v, int S, float scale,
@@ -374,12 +375,8 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
   const int last = min(S, (blk + 1) * kRows) - 1;  // the workgroup's last query
   const int n_tiles = last / TR + 1;
 
-  // Conversions of the weights once only with two waves per group: with one, the last workgroups
-  // run a wave per SIMD (192 x 400 48.6 -> 54.4 us, 256 x 384 42.8 -> 47.0 with it, for 161.5 ->
-  // 160.3 at 192 x 1024; with two, 48 x 1024 48.5 -> 47.8).
-  constexpr bool kOnce = KS == 2;
   X3 qb[D / 16];  // the lane's query row, split
-  load_split_row<D, kOnce>(qb, q + base + (size_t)min(qi, S - 1) * D, h);
+  load_split_row<D, ONCE>(qb, q + base + (size_t)min(qi, S - 1) * D, h);
   f32x16 o[D / 32];
 #pragma unroll
   for (int db = 0; db < D / 32; ++db) o[db] = zero16();
@@ -451,7 +448,7 @@ __global__ __launch_bounds__(64 * kGroups * KS, wgs_per_cu(KS)) void fwd_f32_ker
       if constexpr (DROP) keep = keep_words16(dr, (uint64_t)bh * S + qi, key0, h);
 #pragma unroll
       for (int u = 0; u < 16; ++u) s[u] = DROP ? w[u] * keep_factor(keep, u, dr) : w[u];
-      accumulate_t_p<D, TR, kOnce>(o, svp, 32 * c, s, lane);
+      accumulate_t_p<D, TR, ONCE>(o, svp, 32 * c, s, lane);
     }
   };
   if constexpr (KS == 1) {
@@ -923,8 +920,19 @@ hipError_t fwd_f32_t(float* out, float* lse, const float* q, const float* k, con
   const dim3 grid(BH, (S + kRows - 1) / kRows);
   const DropParams dr = drop_params(drop);
   with_f32_shape(fwd_waves_per_group(BH, S), drop != nullptr, [&](auto drop_c, auto ks) {
-    fwd_f32_kernel<D, drop_c(), ks()><<<grid, 64 * kGroups * ks(), 0, stream>>>(out, lse, q, k, v,
-                                                                             S, scale, dr);
+    auto launch = [&](auto once) {
+      fwd_f32_kernel<D, drop_c(), ks(), once()>
+          <<<grid, 64 * kGroups * ks(), 0, stream>>>(out, lse, q, k, v, S, scale, dr);
+    };
+    // At d_head 64 with one wave per group, up to two rounds of workgroups (two per CU), the last
+    // of which run a wave per SIMD: a lone wave is faster if the conversions need not wait for
+    // each other (once -> not: 192 x 400 54.7 -> 48.3 us, 256 x 384 47.1 -> 43.1, 128 x 777 90.8 ->
+    // 85.8; 400 x 483 103 -> 107, 192 x 1024 158.4 -> 161.6). With dropout or at d_head 32 once is
+    // faster everywhere.
+    constexpr bool kEither = D == 64 && !drop_c() && ks() == 1;
+    if constexpr (kEither)
+      if ((long long)grid.x * grid.y <= 4LL * device_cus()) return launch(std::false_type{});
+    launch(std::true_type{});
   });
   return hipGetLastError();
 }
