@@ -231,7 +231,8 @@ __device__ __forceinline__ void fwd_softmax_pv(f32x16 (&s)[NQB], f32x16 (&oacc)[
       for (int i = 0; i < NQB; ++i) oacc[i][db] = mfma32(va[db][j], pb[i][j], oacc[i][db]);
 }
 
-template <int D, bool STRIDED, bool DROP, int KS>
+// FRESH: V's tile-edge correction computed at each issue (DmaTile::load_any).
+template <int D, bool STRIDED, bool DROP, int KS, bool FRESH = false>
 __global__ __launch_bounds__(64 * kWaves, kMinBlocks)
 __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_kernel(
     bf16* __restrict__ out, float* __restrict__ lse, const bf16* __restrict__ q,
@@ -328,7 +329,7 @@ __attribute__((amdgpu_num_vgpr(512 / (kMinBlocks * kWaves / 4)))) void fwd_bf16_
     const bool prefetch = t + 1 < n_tiles;
     if (prefetch) {
       Dma::load_any(nk, kg, k0 + kTileRows, S, koff, wave, lane, kp);
-      Dma::load_any(nv, vg, k0 + kTileRows, S, voff, wave, lane, vp);
+      Dma::template load_any<FRESH>(nv, vg, k0 + kTileRows, S, voff, wave, lane, vp);
     }
     if (q0 < S && k0 <= q0 + kQW - 1) {  // some key of the tile at or before a query
       // One 32-key chunk at a time (holding both chunks' scores at once measured no faster
@@ -421,8 +422,19 @@ hipError_t launch_fwd_bf16_t(bf16* out, float* lse, const bf16* q, const bf16* k
     // workgroups, 3 per CU) and 6% slower at B16 (1,536).
     const int snake =
         cus > 0 && (long long)grid.x * grid.y <= (long long)cus * kMinBlocks ? cus : 0;
-    fwd_bf16_kernel<D, strided(), dropped(), ks()><<<grid, 64 * kWaves, 0, stream>>>(
-        out, lse, q, k, v, S, c, scale < 0.f, snake, L, dr);
+    auto run = [&](auto fresh) {
+      fwd_bf16_kernel<D, strided(), dropped(), ks(), fresh()><<<grid, 64 * kWaves, 0, stream>>>(
+          out, lse, q, k, v, S, c, scale < 0.f, snake, L, dr);
+    };
+    // With K's and V's edge corrections held, the two-wave strided kernel takes 129 registers,
+    // three workgroups per CU; where the grid has more, V's is computed at each issue (125, four):
+    // 96 x 600 token-major 13.2 -> 11.4 us, 120 x 467 12.3 -> 10.5, 64 x 900 16.2 -> 13.8, 48 x
+    // 1200 17.2 -> 16.9, 60 x 777 11.5 -> 11.7; not on smaller grids (12 x 916 11.2 -> 11.8) or
+    // longer rows, which last as long as one chain (36 x 1500 17.9 -> 19.1). (K's as well: 119
+    // registers, 24 x 1024 12.5 -> 13.9.)
+    if constexpr (D == 64 && strided() && ks() == 2)
+      if (S <= 1200 && (long long)grid.x * grid.y > 3LL * cus) return run(std::true_type{});
+    run(std::false_type{});
   };
   // dropout: contiguous layout only (checked by the caller)
   with_shape(waves_per_group(BH, S, D, drop != nullptr), drop != nullptr,
