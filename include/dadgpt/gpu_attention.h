@@ -20,8 +20,9 @@
  *    those rows reads: bf16 dk = k, dv = v, and one of dq, dk, dv = out; fp32 dq = q or dq =
  *    dout, and one of dq, dk, dv = out. Its kernels then run one after the other.
  *  - A call repeats bit for bit, and the strided and token-major calls give the contiguous
- *    ones' bits (unless gradients and inputs interleave in one buffer). The order of the sums follows from the shape and the number of compute units,
- *    though: the same (b, h) slice may differ in its last bits between calls of another BH or S.
+ *    ones' bits (unless gradients and inputs interleave in one buffer). The order of the sums
+ *    follows from the shape and the number of compute units, though: the same (b, h) slice may
+ *    differ in its last bits between calls of another BH or S.
  *  - Arguments are validated on the host before any HIP call; a failing call returns a
  *    nonzero dadgpt_status and dadgpt_last_error() describes it (thread-local). Launch errors
  *    (hipGetLastError) map to DADGPT_ERR_HIP; asynchronous faults surface at the caller's
