@@ -55,7 +55,7 @@ F32_SHAPES = [(3, 96, 64), (3, 97, 64), (2, 129, 64), (5, 160, 32), (1, 500, 64)
               (65, 1000, 64), (128, 385, 32), (129, 390, 32), (512, 100, 64), (513, 100, 32),
               (64, 40, 64), (65, 33, 64), (32, 1000, 64), (33, 1000, 32), (3, 512, 64),
               (3, 513, 64), (86, 300, 64), (85, 300, 64), (76, 600, 32), (77, 600, 64),
-              (24, 600, 32)]
+              (24, 600, 32), (160, 1000, 64)]
 
 
 @pytest.mark.parametrize("BH,S,D", F32_SHAPES)
@@ -201,16 +201,18 @@ def test_f32_backward_in_place(gpu, BH, S, D, p):
     gradients agree to the fp32 bound."""
     print(f"[case] fp32 backward in place BH={BH} S={S} D={D} p={p}", flush=True)
     q, k, v, dout = _inputs(BH, S, D, torch.float32, S)
-    shape = (BH, S, D, A.default_scale(D), p, 11)
+    shape = (BH, S, D, A.default_scale(D)) + ((p, 11) if p else ())
     out, lse = torch.empty_like(q), torch.empty((BH, S), device="cuda")
-    A.flash_attention_forward_dropout(out, lse, q, k, v, *shape)
+    forward, backward = ((A.flash_attention_forward_dropout, A.flash_attention_backward_dropout)
+                         if p else (A.flash_attention_forward, A.flash_attention_backward))
+    forward(out, lse, q, k, v, *shape)
     delta = torch.empty_like(lse)
     want = [torch.empty_like(q) for _ in range(3)]
-    A.flash_attention_backward_dropout(*want, delta, dout, out, lse, q, k, v, *shape)
+    backward(*want, delta, dout, out, lse, q, k, v, *shape)
     for places in (("q", "out", "v2"), ("dout", "k2", "out"), ("out", "k2", "v2")):
         t = {"q": q.clone(), "dout": dout.clone(), "out": out.clone(),
              "k2": torch.empty_like(q), "v2": torch.empty_like(q)}
-        A.flash_attention_backward_dropout(t[places[0]], t[places[1]], t[places[2]], delta,
-                                           t["dout"], t["out"], lse, t["q"], k, v, *shape)
+        backward(t[places[0]], t[places[1]], t[places[2]], delta, t["dout"], t["out"], lse, t["q"],
+                 k, v, *shape)
         for x, y in zip(places, want):
             assert (t[x] - y).abs().max().item() <= 1e-5, places

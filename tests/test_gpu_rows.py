@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 # counts that give one, two and four rows per wave with a last wave that is not full.
 SHAPES = [(1, 5), (3, 4099), (4, 9), (5, 16387), (66, 8193), (255, 16389), (256, 16384),
           (257, 8195), (511, 8193), (512, 4097), (513, 33), (1021, 7), (1024, 5), (1025, 6),
-          (2047, 3), (2048, 3), (2, 8193), (31, 4097), (63, 16387), (64, 33), (65, 16385)]
+          (2047, 3), (2048, 3), (2, 8193), (31, 4097), (63, 16387), (64, 33), (65, 16385),
+          (100, 9), (100, 8193), (511, 33), (512, 8193)]
 
 
 def _normal(shape, seed, scale=1.0):
@@ -44,7 +45,8 @@ def test_plain_rows(gpu, cols, rows):
 
 @pytest.mark.parametrize("S,BH", [(1, 3), (3, 5), (4, 2), (63, 70), (64, 260), (130, 127),
                                   (256, 65), (257, 32), (509, 17), (512, 9), (515, 2), (1023, 1),
-                                  (1030, 1), (31, 260), (65, 127), (1032, 1)])
+                                  (1030, 1), (31, 260), (65, 127), (1032, 1), (50, 170), (128, 70),
+                                  (130, 20), (257, 10), (512, 17), (1024, 1)])
 def test_causal_rows(gpu, S, BH):
     """attention_probs and attention_probs_backward, without and with dropout (p = 0, whose
     factors are exactly 1, must give the plain result's values). What lies past the diagonal of
@@ -113,11 +115,14 @@ def test_rows_of_special_values(gpu, cols):
     assert out[16384, cols // 2].item() == 0.0
 
 
-@pytest.mark.parametrize("L", [1022, 3, 33, 64, 65, 1300, 1301])
-def test_length_rows(gpu, L):
+@pytest.mark.parametrize("L,H", [(1022, 700), (3, 700), (33, 700), (64, 1400), (65, 700),
+                                 (1300, 700), (1301, 700), (64, 2800), (100, 700), (100, 1400),
+                                 (101, 1400), (100, 2800), (101, 2800), (300, 700), (301, 700),
+                                 (300, 1400), (301, 1400), (1000, 700)])
+def test_length_rows(gpu, L, H):
     """decode_probs over rows of `L` columns: only the first lens keys, zero past them, a zero
     row for an empty cache."""
-    n, H = 6, 700
+    n = 6
     s = _normal((n * H, L), 30, 4.0)
     lens = torch.tensor([1, 0, L // 2 + 1, L, min(4, L), L // 4 + 1], dtype=torch.int32,
                         device="cuda")
